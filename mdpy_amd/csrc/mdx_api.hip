@@ -821,6 +821,7 @@ extern "C" int mdx_ctx_destroy(mdx_ctx* c) {
   c->d_stencil.release(); c->qfix.release(); c->cgrid.release(); c->conv.release(); c->bc.release();
   c->twiddle.release(); c->excl_pairs.release(); c->xa.release(); c->xb.release(); c->va.release();
   c->vb.release(); c->acc_prev.release(); c->acc_cur.release(); c->ehist.release(); c->tmp64.release();
+  c->pc_part.release();
   c->pos_sorted.release(); c->fpart.release(); c->pme_grec.release(); c->pme_grec_n.release();
   c->ex_win.release(); c->s4_win.release(); c->win_bad.release(); c->ctab.release(); c->gsave.release();
   if (c->owns_stream) hipStreamDestroy(c->stream);
@@ -1607,7 +1608,7 @@ static int ensure_graphs(mdx_ctx* c, unsigned terms) {
   // the reciprocal forces that evaluation leaves, whatever the context evaluated last (a fresh
   // context has evaluated nothing yet)
   c->fpart_live = evaluation_leaves_fpart(c, terms);
-  int rc = 0;
+  int rc = (terms & MDX_TERM_COUL_PLAIN) ? mdx_coulomb_plain_prepare(c) : 0;
   for (int k = 0; k < MDX_NGRAPH_SIZES && !rc; ++k) rc = capture_steps(c, terms, kGraphSizes[k], false, &c->graph_f[k]);
   if (!rc) rc = capture_steps(c, terms, 1, true, &c->graph_e);
   if (!rc && fused_steps(c, terms)) rc = capture_head(c, terms, &c->graph_head);

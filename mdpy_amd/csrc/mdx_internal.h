@@ -330,6 +330,7 @@ struct mdx_ctx {
   unsigned forces_terms = 0;
   // scratch
   DevBuf<long long> tmp64;
+  DevBuf<double> pc_part;        // plain Coulomb: 4 sums per atom and partner slice
   // learned surrogate (optional)
   mdx_mlp* mlp = nullptr;
 };
@@ -499,6 +500,8 @@ int mdx_batch_launch_nb(const BatchKind& k, int lanes, bool s14, bool energy, hi
 // Rebuild the nonbonded kernel's Ewald-correction table when beta or the cutoff changed.
 #define MDX_CTAB_N 256
 int mdx_coulomb_table_update(mdx_ctx* c);
+// plain Coulomb: its scratch (sized before a capture), and the launches
+int mdx_coulomb_plain_prepare(mdx_ctx* c);
 int mdx_enqueue_coulomb_plain(mdx_ctx* c);
 int mdx_pme_enqueue(mdx_ctx* c, bool energy);
 int mdx_pme_enqueue_part(mdx_ctx* c, int part);  // one plane-path launch alone (timing)
