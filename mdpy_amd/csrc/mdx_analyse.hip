@@ -7,19 +7,50 @@
 // [0, rc] dropped, r == rc in the last bin). Counts are int64 per (i, bin), summed over frames,
 // so the result is an integer array that matches the reference bit for bit.
 #include "mdx_internal.h"
+#include <algorithm>
 
 #define HIST_BLOCK 256
-#define HIST_TILE 1024  // set-2 positions staged in LDS per pass
+#define HIST_TILE 256            // set-2 positions staged in LDS per pass
+#define HIST_WAVES_PER_SIMD 4
+
+#define HIST_EDGES 512           // bin edges staged in LDS (more bins read them from global memory)
+
+// VALU bound. A workgroup takes HIST_BLOCK atoms of set 1 (one lane each) of one frame against one
+// slice of set 2; the slices are as many as fill the chip (integer counts: any split gives the
+// same histogram). Most pairs lie outside [0, rc], so each is first tested on a cheap r^2: both
+// coordinates as 32-bit fractions of the box, whose wrapped integer difference is the minimum
+// image, then float32. Pairs that pass are queued per wave in LDS and evaluated 64 at a time with
+// the reference's exact float64 sequence (its square root, edge comparisons and one atomic per pair
+// would otherwise run for a wave whenever any of its lanes passes).
+// 7,776 x 7,776 atoms, 6 frames, 9 A: 1,890 -> 360 us (before: 186 workgroups, the exact
+// sequence for every pair; with a cheap test but no queue: 834 us).
+//
+// The test's slack: a fraction is off by at most 2^-32 + |x/L| 2^-52, so for |x| < 1e4 L a component
+// is off by less than 2^-30 L and r^2 by less than 4e-9 (Lx^2 + Ly^2 + Lz^2); float32 adds less
+// than 1e-6 of r^2. Tiles with coordinates beyond that (or not finite) queue every pair.
+__device__ __forceinline__ unsigned box_fraction(double x, double iL) {
+  double u = x * iL;
+  u -= floor(u);
+  return u >= 0.0 && u < 1.0 ? (unsigned)(u * 4294967296.0) : 0u;
+}
 
 __global__ __launch_bounds__(HIST_BLOCK) void k_pair_hist(const double* __restrict__ pos, int n_atoms,
                                                           const int* __restrict__ sel1, int n1,
-                                                          const int* __restrict__ sel2, int n2, double Lx,
-                                                          double Ly, double Lz, const double* __restrict__ edges,
-                                                          int nbins, unsigned long long* __restrict__ counts) {
-  __shared__ double tx[HIST_TILE], ty[HIST_TILE], tz[HIST_TILE];
+                                                          const int* __restrict__ sel2, int n2, int per_slice,
+                                                          double Lx, double Ly, double Lz,
+                                                          const double* __restrict__ edges, int nbins,
+                                                          unsigned long long* __restrict__ counts) {
+  __shared__ uint4 tf[HIST_TILE];                                        // set-2 box fractions
+  __shared__ double tx[HIST_TILE], ty[HIST_TILE], tz[HIST_TILE];         // set-2 positions
+  __shared__ double hx[HIST_BLOCK], hy[HIST_BLOCK], hz[HIST_BLOCK];      // set-1 positions
+  __shared__ double le[HIST_EDGES];
+  __shared__ unsigned queue[HIST_BLOCK / 64][128];                       // lane << 16 | tile entry
   const double* x = pos + (long long)blockIdx.y * n_atoms * 3;  // frame
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int a = blockIdx.x * HIST_BLOCK + tid;
   const bool active = a < n1;
+  const double iLx = 1.0 / Lx, iLy = 1.0 / Ly, iLz = 1.0 / Lz;
+  const double lx = 1e4 * Lx, ly = 1e4 * Ly, lz = 1e4 * Lz;
   double xi = 0, yi = 0, zi = 0;
   if (active) {
     const int i = sel1[a];
@@ -27,42 +58,84 @@ __global__ __launch_bounds__(HIST_BLOCK) void k_pair_hist(const double* __restri
     yi = x[3 * i + 1];
     zi = x[3 * i + 2];
   }
+  hx[tid] = xi;
+  hy[tid] = yi;
+  hz[tid] = zi;
+  const unsigned ux = box_fraction(xi, iLx), uy = box_fraction(yi, iLy), uz = box_fraction(zi, iLz);
+  const int far_i = !(fabs(xi) < lx && fabs(yi) < ly && fabs(zi) < lz);
+  const bool in_lds = nbins < HIST_EDGES;
+  if (in_lds)
+    for (int k = tid; k <= nbins; k += HIST_BLOCK) le[k] = edges[k];
   const double first = edges[0], last = edges[nbins];
   const double norm = (double)nbins / (last - first);
-  const double iLx = 1.0 / Lx, iLy = 1.0 / Ly, iLz = 1.0 / Lz;
-  for (int t0 = 0; t0 < n2; t0 += HIST_TILE) {
-    const int tn = min(HIST_TILE, n2 - t0);
+  const double slack = 1e-6 * last * last + 1e-8 * (Lx * Lx + Ly * Ly + Lz * Lz);
+  const float bound = (float)(last * last + slack) * (1.f + 1e-6f);
+  const float sx = (float)(Lx * 0x1p-32), sy = (float)(Ly * 0x1p-32), sz = (float)(Lz * 0x1p-32);
+  unsigned* q = queue[tid >> 6];
+  const int wbase = tid & ~63;  // the wave's first lane
+  // the first m queued pairs, one per lane, with the reference's arithmetic
+  auto evaluate = [&](int m) {
+    if (lane >= m) return;
+    const unsigned e = q[lane];
+    const int h = wbase + (int)(e >> 16), k = (int)(e & 0xffffu);
+    // vec = x_i - x_j (rdf_analyser.py:48-52), minimum image
+    double dx = hx[h] - tx[k], dy = hy[h] - ty[k], dz = hz[h] - tz[k];
+    double s = dx * iLx;
+    s -= rint(s);
+    dx = s * Lx;
+    s = dy * iLy;
+    s -= rint(s);
+    dy = s * Ly;
+    s = dz * iLz;
+    s -= rint(s);
+    dz = s * Lz;
+    // rounded products and sums in numpy's order ((x^2 + y^2) + z^2), never contracted to FMAs
+    const double r = sqrt(__dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz)));
+    if (!(r >= first && r <= last)) return;
+    const double f = (r - first) * norm;
+    int b = f < (double)nbins ? (int)f : nbins;  // f >= 0 here
+    if (b == nbins) b = nbins - 1;
+    const double lo = in_lds ? le[b] : edges[b], hi = in_lds ? le[b + 1] : edges[b + 1];
+    if (r < lo) --b;
+    else if (b != nbins - 1 && r >= hi) ++b;
+    atomicAdd(&counts[(long long)(blockIdx.x * HIST_BLOCK + h) * nbins + b], 1ull);
+  };
+  const int j0 = blockIdx.z * per_slice, j1 = min(n2, j0 + per_slice);
+  for (int t0 = j0; t0 < j1; t0 += HIST_TILE) {
+    const int tn = min(HIST_TILE, j1 - t0);
     __syncthreads();
-    for (int k = threadIdx.x; k < tn; k += blockDim.x) {
-      const int j = sel2[t0 + k];
-      tx[k] = x[3 * j];
-      ty[k] = x[3 * j + 1];
-      tz[k] = x[3 * j + 2];
+    int far = far_i;
+    if (tid < tn) {
+      const int j = sel2[t0 + tid];
+      const double xj = x[3 * j], yj = x[3 * j + 1], zj = x[3 * j + 2];
+      tx[tid] = xj;
+      ty[tid] = yj;
+      tz[tid] = zj;
+      tf[tid] = make_uint4(box_fraction(xj, iLx), box_fraction(yj, iLy), box_fraction(zj, iLz), 0u);
+      far |= !(fabs(xj) < lx && fabs(yj) < ly && fabs(zj) < lz);
     }
-    __syncthreads();
-    if (!active) continue;
+    far = __syncthreads_or(far);
+    int nq = 0;  // queued pairs of this wave
+#pragma unroll 4
     for (int k = 0; k < tn; ++k) {
-      // vec = x_i - x_j (rdf_analyser.py:48-52), minimum image
-      double dx = xi - tx[k], dy = yi - ty[k], dz = zi - tz[k];
-      double s = dx * iLx;
-      s -= rint(s);
-      dx = s * Lx;
-      s = dy * iLy;
-      s -= rint(s);
-      dy = s * Ly;
-      s = dz * iLz;
-      s -= rint(s);
-      dz = s * Lz;
-      // rounded products and sums in numpy's order ((x^2 + y^2) + z^2), never contracted to FMAs
-      const double r = sqrt(__dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz)));
-      if (!(r >= first && r <= last)) continue;
-      const double f = (r - first) * norm;
-      int b = f < (double)nbins ? (int)f : nbins;  // f >= 0 here
-      if (b == nbins) b = nbins - 1;
-      if (r < edges[b]) --b;
-      else if (b != nbins - 1 && r >= edges[b + 1]) ++b;
-      atomicAdd(&counts[(long long)a * nbins + b], 1ull);
+      const uint4 u = tf[k];
+      const float dx = (float)(int)(ux - u.x) * sx, dy = (float)(int)(uy - u.y) * sy, dz = (float)(int)(uz - u.z) * sz;
+      const bool near = active && (far || dx * dx + dy * dy + dz * dz <= bound);
+      const unsigned long long m = __ballot(near);
+      if (m == 0) continue;  // wave-uniform
+      if (near) q[nq + __popcll(m & ((1ull << lane) - 1ull))] = (unsigned)lane << 16 | (unsigned)k;
+      nq += __popcll(m);
+      if (nq >= 64) {
+        wave_lds_sync();
+        evaluate(64);
+        nq -= 64;
+        const unsigned rest = q[64 + lane];
+        wave_lds_sync();
+        if (lane < nq) q[lane] = rest;
+      }
     }
+    wave_lds_sync();
+    evaluate(nq);  // the tile's positions are replaced next
   }
 }
 
@@ -75,9 +148,16 @@ extern "C" int mdx_pair_histogram(void* hip_stream, int n_frames, int n_atoms, c
   MDX_CHECK(n_frames <= 65535, MDX_ERR_INVALID, "mdx_pair_histogram: at most 65535 frames per call");
   for (int d = 0; d < 3; ++d) MDX_CHECK(h_box[d] > 0, MDX_ERR_INVALID, "box edges must be positive");
   hipStream_t s = (hipStream_t)hip_stream;
-  dim3 g(div_up(n1, HIST_BLOCK), n_frames), b(HIST_BLOCK);
-  k_pair_hist<<<g, b, 0, s>>>(d_pos, n_atoms, d_sel1, n1, d_sel2, n2, h_box[0], h_box[1], h_box[2], d_edges, nbins,
-                              (unsigned long long*)d_counts);
+  int dev = 0, ncu = 0;
+  MDX_HIP(hipGetDevice(&dev));
+  MDX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  // slices of set 2 (whole tiles): about HIST_WAVES_PER_SIMD workgroups of 4 waves per compute unit
+  const int blocks = div_up(n1, HIST_BLOCK), tiles = div_up(n2, HIST_TILE);
+  const int want = std::max(1, std::min(tiles, div_up((long long)HIST_WAVES_PER_SIMD * ncu, (long long)blocks * n_frames)));
+  const int per = div_up(tiles, want);
+  dim3 g(blocks, n_frames, div_up(tiles, per)), b(HIST_BLOCK);
+  k_pair_hist<<<g, b, 0, s>>>(d_pos, n_atoms, d_sel1, n1, d_sel2, n2, per * HIST_TILE, h_box[0], h_box[1], h_box[2],
+                              d_edges, nbins, (unsigned long long*)d_counts);
   MDX_LAUNCH_CHECK();
   return 0;
 }

@@ -1,5 +1,5 @@
 """GPU tests of the kernels that walk all pairs in slices: plain Coulomb against a float64 double
-loop, at atom counts around the tile and slice edges."""
+loop and pair histograms against numpy's, at atom counts around the tile and slice edges."""
 import numpy as np
 import pytest
 
@@ -53,3 +53,30 @@ def test_plain_coulomb_slices(n):
     assert np.all(np.abs(F - ref) <= 2.0 ** -41 + 8 * n * 2.0 ** -53 * size)
     blocks = (n + 255) // 256
     assert abs(en["coulomb_plain"] - 0.5 * w.sum()) <= blocks * 2.0 ** -41 + 8 * n * 2.0 ** -53 * np.abs(w).sum()
+
+
+@pytest.mark.parametrize("n1,n2,frames,unwrapped", [(1, 1, 1, False), (255, 257, 2, False), (256, 512, 1, True),
+                                                    (300, 1000, 3, True)])
+def test_pair_histogram_slices(n1, n2, frames, unwrapped):
+    """Counts equal numpy.histogram's, for wrapped and unwrapped (also very distant) coordinates."""
+    from mdpy_amd.analyser.pair_histogram import pair_histograms
+    from mdpy_amd.core import Particle, Topology, Trajectory
+    from oracle import analyse as A
+    print("case: pair histogram %d x %d, %d frames" % (n1, n2, frames), flush=True)
+    n = max(n1, n2)
+    x = np.stack([box_of(n, 7 + f)[0] for f in range(frames)])
+    box = box_of(n, 7)[1].astype(np.float32).astype(np.float64)
+    if unwrapped:
+        rng = np.random.default_rng(3)
+        x += box * rng.integers(-3, 4, x.shape)
+        x[:, :2] += box * 30000.0
+    t = Trajectory(Topology())
+    t.topology.add_particles([Particle(particle_id=i, particle_type="A", particle_name="A", mass=1.0, charge=0.0)
+                              for i in range(n)])
+    t = Trajectory(t.topology)
+    t.set_pbc_matrix(np.diag(box))
+    t.append(x.astype(np.float32))
+    ids1, ids2 = list(range(n - n1, n)), list(range(n2))
+    got, edges = pair_histograms(t, ids1, ids2, 9.0, 37)
+    ref, _ = A.pair_counts(np.asarray(t.positions, np.float64), box, ids1, ids2, 9.0, 37)
+    assert np.array_equal(got, ref)
