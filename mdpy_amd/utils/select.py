@@ -46,7 +46,8 @@ def select_all(target):
 
 
 def select_particle_type(target, particle_types):
-    return _where(target, lambda p: p.particle_type in particle_types)
+    # the particles' own attributes: two property calls a particle are most of a selection's time
+    return [p._matrix_id for p in _topology(target).particles if p._particle_type in particle_types]
 
 
 def select_particle_name(target, particle_names):
@@ -159,44 +160,61 @@ def parse_selection_condition(conditions):
     return " or ".join(out)
 
 
+def _mask(n, ids):
+    """Boolean mask of the matrix ids in [0, n)."""
+    ids = np.asarray(ids, dtype=np.int64)
+    m = np.zeros(n, dtype=bool)
+    m[ids[(ids >= 0) & (ids < n)]] = True
+    return m
+
+
 def _select_topological(target, conditions):
     n = _topology(target).num_particles
-    everyone = set(range(n))
-    chosen = set()
+    chosen = np.zeros(n, dtype=bool)
     for condition in conditions:
-        cur = set(everyone)
+        cur = np.ones(n, dtype=bool)
         for key, value in condition.items():
             inverse = "not" in key
             key = key.split("not")[-1].strip()
             if key not in SELECTION_SUPPORTED_TOPOLOGICAL_KEYWORDS:
                 raise SelectionConditionPoorDefinedError("%r is not a topological selection keyword" % key)
-            res = set(METHOD_DICT[key](target, *value))
-            cur &= (everyone ^ res) if inverse else res
+            res = _mask(n, METHOD_DICT[key](target, *value))
+            cur &= ~res if inverse else res
         chosen |= cur
-    return sorted(chosen)
+    return np.flatnonzero(chosen).tolist()
 
 
 def _select_frame(target, conditions, frame, cache):
     n = target.topology.num_particles
-    everyone = set(range(n))
-    chosen = set()
+    chosen = np.zeros(n, dtype=bool)
     for index, condition in enumerate(conditions):
-        cur = set(everyone)
+        cur = np.ones(n, dtype=bool)
         for key, value in condition.items():
             inverse = "not" in key
             key = key.split("not")[-1].strip()
             if key in SELECTION_SUPPORTED_TOPOLOGICAL_KEYWORDS:
                 tag = (index, key, repr(value))
                 if tag not in cache:
-                    cache[tag] = set(METHOD_DICT[key](target, *value))
+                    cache[tag] = _mask(n, METHOD_DICT[key](target, *value))
                 res = cache[tag]
             elif key in SELECTION_SUPPORTED_STERIC_KEYWORDS:
-                res = set(STERIC_METHODS[key](target, frame, *value))
+                res = _mask(n, STERIC_METHODS[key](target, frame, *value))
             else:
                 raise SelectionConditionPoorDefinedError("%r is not a selection keyword" % key)
-            cur &= (everyone ^ res) if inverse else res
+            cur &= ~res if inverse else res
         chosen |= cur
-    return sorted(chosen)
+    return np.flatnonzero(chosen).tolist()
+
+
+def select_first_frame(trajectory, conditions):
+    """select(trajectory, conditions)[0] without evaluating the later frames (what the analysers
+    use: their conditions are topological, the same for every frame)."""
+    from ..core.trajectory import Trajectory
+    if not isinstance(trajectory, Trajectory):
+        raise TypeError("frames belong to a Trajectory, not %s" % type(trajectory))
+    if trajectory.num_frames == 0:
+        raise IndexError("the trajectory has no frames")
+    return _select_frame(trajectory, conditions, 0, {})
 
 
 def select(target, conditions):
