@@ -278,6 +278,7 @@ struct StepPro {
   const int* orig_sorted;
   const float* qs;
   float4* xq;
+  int4* xf;
   double* pos_sorted;
   long long* efix;
   int ne;
@@ -325,7 +326,7 @@ __device__ void prologue_atom(const IntArgs& A, const StepPro& P, int i, const P
     dd -= A.L[d] * rint(dd * A.inv[d]);
     *d2 += dd * dd;
   }
-  pack_atom(xn[0], xn[1], xn[2], in.q, A.L[0], A.L[1], A.L[2], &P.xq[in.s], &P.pos_sorted[3 * in.s]);
+  pack_atom(xn[0], xn[1], xn[2], in.q, A.L, A.inv, &P.xq[in.s], &P.xf[in.s], &P.pos_sorted[3 * in.s]);
   if (P.bin) {  // the list-grid cell, as k_grid_bin computes it
     int c[3];
     for (int d = 0; d < 3; ++d) {
@@ -816,7 +817,7 @@ extern "C" int mdx_ctx_destroy(mdx_ctx* c) {
   c->ffix.release(); c->efix.release(); c->dstate.release();
   c->ref_cell_lin.release(); c->ref_counts.release(); c->ref_cursor.release();
   c->cell_count.release(); c->cell_start.release(); c->cell_cursor.release(); c->atom_cell.release();
-  c->sorted_orig.release(); c->orig_sorted.release(); c->xq.release(); c->ljs.release(); c->ljs14.release();
+  c->sorted_orig.release(); c->orig_sorted.release(); c->xq.release(); c->xf.release(); c->ljs.release(); c->ljs14.release();
   c->ref_cell_sorted.release(); c->pos_at_build.release(); c->nbr_count.release(); c->nbr_list.release();
   c->d_stencil.release(); c->qfix.release(); c->cgrid.release(); c->conv.release(); c->bc.release();
   c->twiddle.release(); c->excl_pairs.release(); c->xa.release(); c->xb.release(); c->va.release();
@@ -1298,6 +1299,7 @@ static StepPro step_pro(mdx_ctx* c) {
   P.orig_sorted = c->orig_sorted.p;
   P.qs = c->has_charges ? c->charge_s.p : nullptr;
   P.xq = c->xq.p;
+  P.xf = c->xf.p;
   P.pos_sorted = c->pos_sorted.p;
   P.efix = c->efix.p;
   P.ne = MDX_NTERMS + 1;
@@ -1620,7 +1622,7 @@ static int ensure_graphs(mdx_ctx* c, unsigned terms) {
   }
   c->graph_terms = terms;
   c->graph_kind = c->int_kind;
-  c->graph_lanes = c->nb_lanes;
+  c->graph_lanes = mdx_nb_lanes(c);
   c->forces_current = cur;
   c->forces_terms = cur_terms;
   return 0;
@@ -1713,10 +1715,10 @@ struct BatchFused {
   hipGraphExec_t gf[MDX_NGRAPH_SIZES] = {};
   hipGraphExec_t ge = nullptr;
   std::vector<unsigned long long> gens;  // the contexts' graph generations the tables were built at
+  std::vector<int> lanes;                // and their nonbonded lanes per atom
   unsigned terms = 0;
   bool ready = false;
   bool gjf = false, s14 = false;
-  int lanes = 0;
 };
 
 struct mdx_batch {
@@ -1819,9 +1821,10 @@ static const unsigned kFusedBonded = MDX_TERM_BOND | MDX_TERM_ANGLE | MDX_TERM_D
 static int fused_prepare(mdx_batch* b, unsigned terms) {
   BatchFused& f = b->fz;
   const int n = (int)b->ctx.size();
-  bool fresh = f.ready && f.terms == terms && f.gens.size() == (size_t)n && f.lanes == b->ctx[0]->nb_lanes &&
+  bool fresh = f.ready && f.terms == terms && f.gens.size() == (size_t)n && f.lanes.size() == (size_t)n &&
                f.gjf == (b->ctx[0]->int_kind == MDX_INT_LANGEVIN);
-  for (int r = 0; r < n && fresh; ++r) fresh = f.gens[r] == b->ctx[r]->graph_gen;
+  for (int r = 0; r < n && fresh; ++r)
+    fresh = f.gens[r] == b->ctx[r]->graph_gen && f.lanes[r] == mdx_nb_lanes(b->ctx[r]);
   if (fresh) return 0;
   fused_drop_graphs(b);
   // the tables are rewritten in place: no earlier batched launch may still be reading them
@@ -1858,11 +1861,14 @@ static int fused_prepare(mdx_batch* b, unsigned terms) {
       (rc = mdx_batch_prepare_nb(b->ctx.data(), n, terms & (kFusedBonded | MDX_TERM_COUL_RECIP), &f.nb)))
     return rc;
   f.gjf = c0->int_kind == MDX_INT_LANGEVIN;
-  f.lanes = c0->nb_lanes;
   f.s14 = c0->has_s14;
   f.terms = terms;
   f.gens.resize(n);
-  for (int r = 0; r < n; ++r) f.gens[r] = b->ctx[r]->graph_gen;
+  f.lanes.resize(n);
+  for (int r = 0; r < n; ++r) {
+    f.gens[r] = b->ctx[r]->graph_gen;
+    f.lanes[r] = mdx_nb_lanes(b->ctx[r]);
+  }
   f.ready = true;
   return 0;
 }
@@ -1887,7 +1893,7 @@ static int fused_step(mdx_batch* b, bool energy, bool fuse_prev) {
   MDX_HIP(hipStreamWaitEvent(f.side, f.ev_fork, 0));
   if ((rc = mdx_batch_launch_pme(f.pfwd, f.pfft, f.pgat, f.side))) return rc;
   MDX_HIP(hipEventRecord(f.ev_join, f.side));
-  if ((rc = mdx_batch_launch_list(f.lfast, f.lcell, s)) || (rc = mdx_batch_launch_nb(f.nb, f.lanes, f.s14, energy, s)))
+  if ((rc = mdx_batch_launch_list(f.lfast, f.lcell, s)) || (rc = mdx_batch_launch_nb(f.nb, f.s14, energy, s)))
     return rc;
   MDX_HIP(hipStreamWaitEvent(s, f.ev_join, 0));
   return 0;
@@ -2261,7 +2267,7 @@ __global__ void k_count_pairs(int n, int cap, const int* __restrict__ nbr_count,
     slots = cnt;
     float4 xi = xq[s];
     for (int k = 0; k < cnt; ++k) {
-      int t = (int)(nbr_list[(long long)s * cap + k] & 0x7fffffffu);
+      int t = nbr_slot(nbr_list[(long long)s * cap + k]);
       float dx = xq[t].x - xi.x, dy = xq[t].y - xi.y, dz = xq[t].z - xi.z;
       dx -= Lx * rintf(dx / Lx);
       dy -= Ly * rintf(dy / Ly);
@@ -2308,6 +2314,7 @@ extern "C" int mdx_nonbonded_tune(mdx_ctx* c, unsigned terms, int lanes, int rep
   if (lanes == 0) {
     double best_ms = 1e300;
     const int cand[3] = {16, 32, 64};
+    c->nb_lanes_set = true;
     for (int k = 0; k < 3; ++k) {
       c->nb_lanes = cand[k];
       double ms = 0;
@@ -2323,6 +2330,7 @@ extern "C" int mdx_nonbonded_tune(mdx_ctx* c, unsigned terms, int lanes, int rep
   // they were captured with, so they are dropped only when that differs from the choice
   if (best != c->graph_lanes) mdx_invalidate_graph(c);
   c->nb_lanes = best;
+  c->nb_lanes_set = true;
   if (h_lanes) *h_lanes = best;
   return 0;
 }
@@ -2361,7 +2369,7 @@ struct StatePart {
   void* p;
   size_t bytes;
 };
-static const int kProStateParts = 9;
+static const int kProStateParts = 10;
 static int prologue_state_parts(mdx_ctx* c, StatePart* parts) {
   MDX_CHECK(c->int_configured && c->acc_prev.p && c->gsave.p && c->xq.p && c->pos_sorted.p &&
                 (c->int_kind == MDX_INT_LANGEVIN || c->int_kind == MDX_INT_VELOCITY_VERLET),
@@ -2370,7 +2378,8 @@ static int prologue_state_parts(mdx_ctx* c, StatePart* parts) {
   const StatePart q[kProStateParts] = {
       {c->pos, n3 * 8},        {c->vel, n3 * 8},  {c->acc_prev.p, n3 * 8},
       {c->gsave.p, n3 * 8},    {c->ffix.p, n3 * 8}, {c->efix.p, (MDX_NTERMS + 1) * 8},
-      {c->dstate.p, sizeof(DevState)}, {c->xq.p, (size_t)c->n * sizeof(float4)}, {c->pos_sorted.p, n3 * 8}};
+      {c->dstate.p, sizeof(DevState)}, {c->xq.p, (size_t)c->n * sizeof(float4)},
+      {c->xf.p, (size_t)c->n * sizeof(int4)}, {c->pos_sorted.p, n3 * 8}};
   for (int k = 0; k < kProStateParts; ++k) parts[k] = q[k];
   return 0;
 }
@@ -2553,7 +2562,7 @@ extern "C" int mdx_batch_time_kernel(mdx_batch* b, int which, int reps, double* 
   if (which != 5) MDX_HIP(hipEventRecord(k.e0, s));
   for (int rep = 0; rep < reps && !rc; ++rep) {
     if (which == 0) {
-      rc = mdx_batch_launch_nb(f.nb, f.lanes, f.s14, false, s);
+      rc = mdx_batch_launch_nb(f.nb, f.s14, false, s);
     } else if (which == 4) {
       const ProCall* pc = (const ProCall*)k.pro.calls;
       if (f.gjf) k_step_pro_batch<true, true><<<k.pro.blocks, PRO_THREADS, 0, s>>>(k.pro.map, pc);

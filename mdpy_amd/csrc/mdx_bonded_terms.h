@@ -23,8 +23,16 @@ __device__ __forceinline__ void mi(const Box3& b, const double* v, double* out) 
     out[q] = s * b.L[q];
   }
 }
+// coordinate d of atom i in the primary image: exactly the value that the wrap at the end of an
+// integrate call stores (the product with 0 or +-1 is exact), so a term is the same to the last bit
+// whether its atoms have just been wrapped or have just crossed the box edge
+__device__ __forceinline__ double primary(const Box3& b, const double* __restrict__ pos, int i, int d) {
+  const double x = pos[3 * i + d];
+  return fma(-rint(x * b.inv[d]), b.L[d], x);
+}
 __device__ __forceinline__ void sub_mi(const Box3& b, const double* __restrict__ pos, int j, int i, double* out) {
-  double v[3] = {pos[3 * j] - pos[3 * i], pos[3 * j + 1] - pos[3 * i + 1], pos[3 * j + 2] - pos[3 * i + 2]};
+  double v[3];
+  for (int d = 0; d < 3; ++d) v[d] = primary(b, pos, j, d) - primary(b, pos, i, d);
   mi(b, v, out);
 }
 __device__ __forceinline__ double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }

@@ -110,6 +110,11 @@ struct DevState {
   unsigned long long ke_acc;  // kinetic-energy partial sums of the opening kernel (0 between calls)
 };
 
+// A neighbour-list entry is the partner's byte offset into the 16-byte sorted-order records (slot
+// * 16; atom indices stay below 2^28), with bit 0 set for a 1-4 pair.
+__device__ __forceinline__ unsigned nbr_entry(int slot, bool s14) { return (unsigned)slot << 4 | (s14 ? 1u : 0u); }
+__device__ __forceinline__ int nbr_slot(unsigned e) { return (int)(e >> 4); }
+
 // neighbour-list entries allocated past the last row (at least the longest read-ahead: one
 // chunk of 64 lanes x 4 entries)
 #define MDX_LIST_SLACK 512
@@ -176,17 +181,29 @@ __device__ __forceinline__ int clamped_floor_index(double u, int n) {
   return u >= 1.0 ? (u < (double)n ? (int)u : n - 1) : 0;
 }
 
-// float32 sorted-order copy of one atom: wrapped, centred position and q*sqrt(ke) (the layout
-// the pair kernels read), plus its float64 position
-__device__ __forceinline__ void pack_atom(double x, double y, double z, float q, double Lx, double Ly, double Lz,
-                                          float4* __restrict__ xq_s, double* __restrict__ ps_s) {
+// sorted-order copies of one atom: xq its wrapped, centred float32 position and q*sqrt(ke) (list
+// build), xf the position as 32-bit fractions of the box with the same charge (pair kernels: the
+// wrapped difference of two fractions is the minimum image, to 2^-32 of an edge where centred
+// float32 positions carry 2^-24), and its float64 position (PME). iL: inverse edges.
+__device__ __forceinline__ void pack_atom(double x, double y, double z, float q, const double* L, const double* iL,
+                                          float4* __restrict__ xq_s, int4* __restrict__ xf_s,
+                                          double* __restrict__ ps_s) {
   ps_s[0] = x;
   ps_s[1] = y;
   ps_s[2] = z;
-  x -= Lx * floor(x / Lx);
-  y -= Ly * floor(y / Ly);
-  z -= Lz * floor(z / Lz);
-  *xq_s = make_float4((float)(x - 0.5 * Lx), (float)(y - 0.5 * Ly), (float)(z - 0.5 * Lz), q);
+  const double p[3] = {x, y, z};
+  double u[3];
+  int f[3];
+  for (int d = 0; d < 3; ++d) {
+    // the primary image first (exact for a coordinate within one image): the same fraction for a
+    // coordinate before and after it is wrapped
+    u[d] = fma(-rint(p[d] * iL[d]), L[d], p[d]) * iL[d];
+    u[d] -= floor(u[d]);
+    // the range is decided before the conversion (NaN, or a tiny negative coordinate rounding to 1)
+    f[d] = (int)(u[d] >= 0.0 && u[d] < 1.0 ? (unsigned)(u[d] * 4294967296.0) : 0u);
+  }
+  *xq_s = make_float4((float)((u[0] - 0.5) * L[0]), (float)((u[1] - 0.5) * L[1]), (float)((u[2] - 0.5) * L[2]), q);
+  *xf_s = make_int4(f[0], f[1], f[2], __float_as_int(q));
 }
 
 struct mdx_ctx {
@@ -237,6 +254,7 @@ struct mdx_ctx {
   DevBuf<int> sorted_orig;       // sorted slot -> original atom
   DevBuf<int> orig_sorted;       // original atom -> sorted slot
   DevBuf<float4> xq;             // sorted: x, y, z (centred, float), q*sqrt(ke)
+  DevBuf<int4> xf;               // sorted: x, y, z (32-bit box fractions), q*sqrt(ke) as float bits
   DevBuf<float2> ljs, ljs14;     // sorted: sigma/2, sqrt(eps)
   DevBuf<float4> ctab;           // Ewald correction G(r^2) as cubic pieces (MDX_CTAB_N of them)
   double ctab_beta = 0, ctab_rc = 0;
@@ -245,9 +263,10 @@ struct mdx_ctx {
   DevBuf<double> pos_at_build;   // original order, 3N
   DevBuf<double> pos_sorted;     // sorted order, 3N, refreshed with xq every evaluation
   DevBuf<int> nbr_count;         // sorted
-  DevBuf<unsigned> nbr_list;     // column major: [k * stride + s]
+  DevBuf<unsigned> nbr_list;     // rows of nbr_cap entries: neighbour slot * 16 | 1-4 flag (nbr_slot)
   int nbr_cap = 0;               // capacity per atom
-  int nb_lanes = 32;             // lanes per atom in the nonbonded kernel (16, 32 or 64)
+  int nb_lanes = 32;             // lanes per atom in the nonbonded kernel (16, 32 or 64) chosen by the
+  bool nb_lanes_set = false;     // caller or the tuner; else mdx_nb_lanes chooses by system size
   // nonbonded workgroups per compute unit looping over the work (0: one per unit of work); 3 (12
   // waves of 123 VGPRs) leaves a quarter of every SIMD's registers to the PME kernels beside it
   int nb_persist = 3;
@@ -380,8 +399,9 @@ struct FillArgs {
   double thr2;
   const float* qs;
   float4* xq;
+  int4* xf;
   double* pos_sorted;
-  double L[3];
+  double L[3], iL[3];
   int ncell;
 };
 
@@ -392,7 +412,7 @@ struct FillArgs {
 __device__ inline void fill_slot(const FillArgs& f, int s, int o) {
   f.orig_sorted[o] = s;
   for (int d = 0; d < 3; ++d) f.pos_build[3 * o + d] = f.pos[3 * o + d];
-  pack_atom(f.pos[3 * o], f.pos[3 * o + 1], f.pos[3 * o + 2], f.qs ? f.qs[o] : 0.f, f.L[0], f.L[1], f.L[2], &f.xq[s],
+  pack_atom(f.pos[3 * o], f.pos[3 * o + 1], f.pos[3 * o + 2], f.qs ? f.qs[o] : 0.f, f.L, f.iL, &f.xq[s], &f.xf[s],
             &f.pos_sorted[3 * s]);
   if (f.lj64) {
     double e = f.lj64[4 * o + 0], sg = f.lj64[4 * o + 1], e14 = f.lj64[4 * o + 2], s14 = f.lj64[4 * o + 3];
@@ -407,7 +427,14 @@ __device__ inline void fill_slot(const FillArgs& f, int s, int o) {
   }
 }
 
-// per cell: sort members ascending (deterministic order), then fill the per-slot arrays
+// sort key of atom o within its cell: atoms with LJ parameters first, then ascending id (a wave of
+// the nonbonded kernel then mostly holds atoms of one kind and skips LJ where none has it)
+#define SORT_NO_LJ (1 << 29)  // above every atom id (below 2^28)
+__device__ __forceinline__ int sort_key(const FillArgs& f, int o) {
+  return o | (f.lj64 && f.lj64[4 * o] == 0.0 && f.lj64[4 * o + 2] == 0.0 ? SORT_NO_LJ : 0);
+}
+
+// per cell: sort the members by sort_key (deterministic order), then fill the per-slot arrays
 __device__ inline void grid_sort_fill_block(const FillArgs& f, int cell) {
   __shared__ int buf[SORT_MAX];
   int* sorted_orig = f.sorted_orig;
@@ -422,7 +449,7 @@ __device__ inline void grid_sort_fill_block(const FillArgs& f, int cell) {
     return;
   }
   while (P < cnt) P <<= 1;
-  for (int t = threadIdx.x; t < P; t += blockDim.x) buf[t] = t < cnt ? sorted_orig[start + t] : 0x7fffffff;
+  for (int t = threadIdx.x; t < P; t += blockDim.x) buf[t] = t < cnt ? sort_key(f, sorted_orig[start + t]) : 0x7fffffff;
   __syncthreads();
   for (int k = 2; k <= P; k <<= 1) {
     for (int j = k >> 1; j > 0; j >>= 1) {
@@ -441,7 +468,7 @@ __device__ inline void grid_sort_fill_block(const FillArgs& f, int cell) {
     }
   }
   for (int t = threadIdx.x; t < cnt; t += blockDim.x) {
-    int o = buf[t];
+    int o = buf[t] & ~SORT_NO_LJ;
     int s = start + t;
     sorted_orig[s] = o;
     fill_slot(f, s, o);
@@ -485,6 +512,7 @@ int mdx_nlist_enqueue_pack(mdx_ctx* c);
 int mdx_nlist_enqueue_clear(mdx_ctx* c);
 int mdx_enqueue_request_rebuild(mdx_ctx* c);
 // forces
+int mdx_nb_lanes(const mdx_ctx* c);  // lanes per atom of the nonbonded kernel
 // nonbonded launch; the bonded terms in `bonded_terms` (bond/angle/dihedral/improper bits, and the
 // PME exclusion correction with MDX_TERM_COUL_RECIP) ride along as extra workgroups
 int mdx_enqueue_nonbonded(mdx_ctx* c, bool lj, bool coul, bool energy, unsigned bonded_terms = 0u);
@@ -496,7 +524,7 @@ int mdx_batch_prepare_pme(mdx_ctx* const* cs, int n, BatchKind* fwd, BatchKind* 
 int mdx_batch_launch_pme(const BatchKind& fwd, const BatchKind& fft, const BatchKind& gat, hipStream_t s,
                          unsigned parts = 7u);  // bits: forward, x-axis pass, inverse + gather
 int mdx_batch_prepare_nb(mdx_ctx* const* cs, int n, unsigned bonded_terms, BatchKind* out);
-int mdx_batch_launch_nb(const BatchKind& k, int lanes, bool s14, bool energy, hipStream_t s);
+int mdx_batch_launch_nb(const BatchKind& k, bool s14, bool energy, hipStream_t s);
 // Rebuild the nonbonded kernel's Ewald-correction table when beta or the cutoff changed.
 #define MDX_CTAB_N 256
 int mdx_coulomb_table_update(mdx_ctx* c);

@@ -127,7 +127,7 @@ __device__ __forceinline__ void stage_neighbours(const MlAtoms& a, const MlConst
   float ux = 0.f, uy = 0.f, uz = 0.f, r = 1e30f;
   int e = 0, t = 0;
   if (kk < cnt) {
-    t = (int)(row[kk] & 0x3fffffffu);
+    t = nbr_slot(row[kk]);
     const float4 xj = xq[t];
     float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
     dx -= a.Lx * rintf(dx * a.ix);
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(64) void k_ml_desc(MlAtoms a, MlConst k, const floa
     float ux = 0.f, uy = 0.f, uz = 0.f, r = 1e30f;
     int e = 0;
     if (kk < cnt) {
-      const int t = (int)(lrow[kk] & 0x3fffffffu);
+      const int t = nbr_slot(lrow[kk]);
       const float4 xj = xq[t];
       float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
       dx -= a.Lx * rintf(dx * a.ix);
@@ -387,7 +387,7 @@ __global__ __launch_bounds__(64) void k_ml_force(MlAtoms a, MlConst k, const flo
       float4 u = make_float4(0.f, 0.f, 0.f, 0.f);
       int te = 0;
       if (kk < cnt) {
-        const int t = (int)(lrow[kk] & 0x3fffffffu);
+        const int t = nbr_slot(lrow[kk]);
         const float4 xj = xq[t];
         float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
         dx -= a.Lx * rintf(dx * a.ix);

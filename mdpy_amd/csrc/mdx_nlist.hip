@@ -347,23 +347,23 @@ FillArgs fill_args(mdx_ctx* c, double thr2) {
   f.thr2 = thr2;
   f.qs = c->has_charges ? c->charge_s.p : nullptr;
   f.xq = c->xq.p;
+  f.xf = c->xf.p;
   f.pos_sorted = c->pos_sorted.p;
-  f.L[0] = c->box[0];
-  f.L[1] = c->box[1];
-  f.L[2] = c->box[2];
+  for (int d = 0; d < 3; ++d) {
+    f.L[d] = c->box[d];
+    f.iL[d] = 1.0 / c->box[d];
+  }
   f.ncell = c->ncell;
   return f;
 }
 
-// every evaluation: float32 positions (wrapped, centred) and scaled charges in sorted order,
-// plus the float64 positions as they are (sorted order, read by the PME plane kernels)
-__global__ void k_pack(const double* __restrict__ pos, const int* __restrict__ sorted_orig,
-                       const float* __restrict__ qs, int n, double Lx, double Ly, double Lz,
-                       float4* __restrict__ xq, double* __restrict__ pos_sorted) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
+// every evaluation: the sorted-order copies of pack_atom
+__global__ void k_pack(FillArgs f, int n) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
-  int o = sorted_orig[s];
-  pack_atom(pos[3 * o + 0], pos[3 * o + 1], pos[3 * o + 2], qs ? qs[o] : 0.f, Lx, Ly, Lz, &xq[s], &pos_sorted[3 * s]);
+  const int o = f.sorted_orig[s];
+  pack_atom(f.pos[3 * o], f.pos[3 * o + 1], f.pos[3 * o + 2], f.qs ? f.qs[o] : 0.f, f.L, f.iL, &f.xq[s], &f.xf[s],
+            &f.pos_sorted[3 * s]);
 }
 
 struct ListArgs {
@@ -693,7 +693,7 @@ __device__ __forceinline__ void build_list_cell_body(const ListCall& L, const in
           }
           const unsigned long long m = __ballot(acc) & gmask;
           const int slot = cnt + __popcll(m & below);
-          if (acc && slot < a.cap) row[slot] = (unsigned)tj[u].x | (s14 ? 0x80000000u : 0u);
+          if (acc && slot < a.cap) row[slot] = nbr_entry(tj[u].x, s14);
           cnt += __popcll(m);
         }
       }
@@ -895,7 +895,7 @@ __device__ __forceinline__ void build_list_fast_body(const ListCall& L, const in
             const unsigned long long m = mn & __ballot(kept);  // two compares, no re-materialised mask
             const int slot = cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-            if (acc && slot < a.cap) row[slot] = (unsigned)tj[u].x | ((unsigned)((s4m >> dw) & 1ull) << 31);
+            if (acc && slot < a.cap) row[slot] = nbr_entry(tj[u].x, (s4m >> dw) & 1ull);
             cnt += __popcll(m);
           }
         }
@@ -918,7 +918,7 @@ __device__ __forceinline__ void build_list_fast_body(const ListCall& L, const in
           const unsigned long long m = __ballot(acc);
           const int slot = cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-          if (acc && slot < a.cap) row[slot] = (unsigned)tj.x | (s14 ? 0x80000000u : 0u);
+          if (acc && slot < a.cap) row[slot] = nbr_entry(tj.x, s14);
           cnt += __popcll(m);
         }
         wave_lds_sync();  // the wave's next home atom overwrites my_ex / my_s4
@@ -1028,7 +1028,7 @@ int mdx_nlist_prepare(mdx_ctx* c) {
   MDX_HIP(hipMemcpy(c->d_stencil.p, c->stencil.data(), c->stencil.size() * sizeof(int), hipMemcpyHostToDevice));
   if ((rc = c->cell_count.ensure(c->ncell)) || (rc = c->cell_start.ensure(c->ncell)) ||
       (rc = c->cell_cursor.ensure(c->ncell)) || (rc = c->atom_cell.ensure(c->n)) ||
-      (rc = c->sorted_orig.ensure(c->n)) || (rc = c->orig_sorted.ensure(c->n)) || (rc = c->xq.ensure(c->n)) ||
+      (rc = c->sorted_orig.ensure(c->n)) || (rc = c->orig_sorted.ensure(c->n)) || (rc = c->xq.ensure(c->n)) || (rc = c->xf.ensure(c->n)) ||
       (rc = c->ljs.ensure(c->n)) || (rc = c->ljs14.ensure(c->n)) || (rc = c->ref_cell_sorted.ensure(c->n)) ||
       (rc = c->pos_at_build.ensure(3 * (size_t)c->n)) || (rc = c->nbr_count.ensure(c->n)) ||
       (rc = c->pos_sorted.ensure(3 * (size_t)c->n)))
@@ -1052,10 +1052,7 @@ int mdx_nlist_prepare(mdx_ctx* c) {
 }
 
 int mdx_nlist_enqueue_pack(mdx_ctx* c) {
-  k_pack<<<div_up(c->n, NL_BLOCK), NL_BLOCK, 0, c->stream>>>(c->pos, c->sorted_orig.p,
-                                                            c->has_charges ? c->charge_s.p : nullptr, c->n,
-                                                            c->box[0], c->box[1], c->box[2], c->xq.p,
-                                                            c->pos_sorted.p);
+  k_pack<<<div_up(c->n, NL_BLOCK), NL_BLOCK, 0, c->stream>>>(fill_args(c, 0.0), c->n);
   MDX_LAUNCH_CHECK();
   return 0;
 }
@@ -1252,7 +1249,7 @@ __global__ void k_emit_pairs(int n, int cap, const int* __restrict__ nbr_count, 
   double L[3] = {Lx, Ly, Lz};
   for (int k = 0; k < cnt; ++k) {
     unsigned e = nbr_list[(long long)s * cap + k];
-    int t = (int)(e & 0x7fffffffu);
+    int t = nbr_slot(e);
     int jo = sorted_orig[t];
     if (jo <= o) continue;  // unique pairs, i < j (original ids)
     double d[3];

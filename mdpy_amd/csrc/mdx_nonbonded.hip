@@ -82,19 +82,30 @@ __global__ __launch_bounds__(NB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
   for (int vb = blockIdx.x; vb < nb_blocks; vb += nres) nb_block<LJ, COUL, ENERGY, G, NB_BLOCK, S14>(a, P, vb);
 }
 
+// Lanes per atom. Fewer lanes leave less of a row's last chunk empty and share the reduction and
+// the row set-up among more atoms of a wave; more lanes give small systems enough waves. Measured
+// alone with 16 / 32 / 64 lanes (us): 648 atoms r_c 9 A 7.3 / 5.3 / 4.5, 2,592 r_c 12 12.4 / 9.4 / 8.4,
+// 3,000 r_c 9 8.0 / 6.5 / 5.9, 9,000 r_c 9 11.8 / 12.1 / 13.6, r_c 12 21.0 / 21.2 / 22.6,
+// 23,328 r_c 12 40.8 / 43.2 / 50.9, 98,304 r_c 12 188 / 207 / 259.
+int mdx_nb_lanes(const mdx_ctx* c) {
+  if (c->nb_lanes_set) return c->nb_lanes;
+  return c->n >= 8192 ? 16 : (c->n >= 3072 ? 32 : 64);
+}
+
 NbArgs nb_args(const mdx_ctx* c) {
   NbArgs a;
   a.n = c->n;
   a.cap = c->nbr_cap;
-  a.Lx = (float)c->box[0];
-  a.Ly = (float)c->box[1];
-  a.Lz = (float)c->box[2];
-  a.ix = 1.0f / a.Lx;
-  a.iy = 1.0f / a.Ly;
-  a.iz = 1.0f / a.Lz;
+  const double s[3] = {c->box[0] * 0x1p-32, c->box[1] * 0x1p-32, c->box[2] * 0x1p-32};
+  a.sx = (float)s[0];
+  a.sy = (float)s[1];
+  a.sz = (float)s[2];
+  a.sx2 = (float)(s[0] * s[0]);
+  a.sy2 = (float)(s[1] * s[1]);
+  a.sz2 = (float)(s[2] * s[2]);
   a.rc2 = (float)(c->rc * c->rc);
-  // float32 r^2 carries ~2 * r * 4e-6 A^2 of error from the float positions: re-decide within
-  // ~20x that band in float64
+  // float32 r^2 carries ~5e-7 of itself in error (the box fractions hold 32 bits): re-decide within
+  // a band of more than 20x that in float64
   a.guard2 = (float)(c->rc * 2e-4);
   a.beta = (float)c->beta;
   a.twob_sqrtpi = (float)(2.0 * c->beta / sqrt(M_PI));
@@ -109,7 +120,7 @@ NbArgs nb_args(const mdx_ctx* c) {
 
 NbPtrs nb_ptrs(const mdx_ctx* c) {
   NbPtrs P;
-  P.xq = c->xq.p;
+  P.xf = c->xf.p;
   P.ljs = c->ljs.p;
   P.ljs14 = c->ljs14.p;
   P.nbr_count = c->nbr_count.p;
@@ -127,7 +138,7 @@ int mdx_enqueue_nonbonded(mdx_ctx* c, bool lj, bool coul, bool energy, unsigned 
   const NbPtrs P = nb_ptrs(c);
   MDX_CHECK(!coul || (a.ctab && c->ctab_beta == c->beta && c->ctab_rc == c->rc), MDX_ERR_INVALID,
             "Ewald-correction table not built for the current beta and cutoff");
-  const int lanes = c->nb_lanes;
+  const int lanes = mdx_nb_lanes(c);
   static_assert(NB_BLOCK == BD_BLOCK, "bonded workgroups share the nonbonded launch");
   BondedArgs ba{};
   const int nbb = (int)div_up((long long)c->n * lanes, NB_BLOCK);
@@ -339,9 +350,10 @@ struct NbCall {
   NbPtrs P;
   BondedArgs ba;
   int nb_blocks;  // the replica's nonbonded workgroups; the rest of its workgroups are bonded
+  int lanes;      // the replica's lanes per atom
 };
 
-template <bool LJ, bool COUL, bool ENERGY, int G, bool S14>
+template <bool LJ, bool COUL, bool ENERGY, bool S14>
 __global__ __launch_bounds__(NB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_nonbonded_batch(
     BatchMap map, const NbCall* __restrict__ calls) {
   int b;
@@ -350,23 +362,31 @@ __global__ __launch_bounds__(NB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
     bonded_block(k.ba, b - k.nb_blocks);
     return;
   }
-  nb_block<LJ, COUL, ENERGY, G, NB_BLOCK, S14>(k.a, k.P, b);
+  if (k.lanes == 16) nb_block<LJ, COUL, ENERGY, 16, NB_BLOCK, S14>(k.a, k.P, b);
+  else if (k.lanes == 64) nb_block<LJ, COUL, ENERGY, 64, NB_BLOCK, S14>(k.a, k.P, b);
+  else nb_block<LJ, COUL, ENERGY, 32, NB_BLOCK, S14>(k.a, k.P, b);
 }
 
 int mdx_batch_prepare_nb(mdx_ctx* const* cs, int n, unsigned bonded_terms, BatchKind* out) {
   std::vector<NbCall> calls;
   std::vector<int> blocks;
+  bool any_set = false;
+  for (int r = 0; r < n; ++r) any_set |= cs[r]->nb_lanes_set;
+  const int want = cs[0]->nb_lanes_set ? cs[0]->nb_lanes : 32;
   for (int r = 0; r < n; ++r) {
     mdx_ctx* c = cs[r];
     NbCall k;
+    k.lanes = mdx_nb_lanes(c);
     k.a = nb_args(c);
     k.P = nb_ptrs(c);
     MDX_CHECK(k.a.ctab && c->ctab_beta == c->beta && c->ctab_rc == c->rc, MDX_ERR_INVALID,
               "replica %d: Ewald-correction table not built for the current beta and cutoff", r);
-    MDX_CHECK(c->nb_lanes == cs[0]->nb_lanes && c->has_s14 == cs[0]->has_s14, MDX_ERR_INVALID,
-              "replica %d: batched replicas need the same lanes per atom and 1-4 pair mode", r);
+    // lanes chosen by the caller have to agree (32 where another replica's were chosen and this
+    // one's not); the ones each system gets by itself may differ
+    MDX_CHECK((!any_set || (c->nb_lanes_set ? c->nb_lanes : 32) == want) && c->has_s14 == cs[0]->has_s14,
+              MDX_ERR_INVALID, "replica %d: batched replicas need the same lanes per atom and 1-4 pair mode", r);
     k.ba = BondedArgs{};
-    k.nb_blocks = (int)div_up((long long)c->n * c->nb_lanes, NB_BLOCK);
+    k.nb_blocks = (int)div_up((long long)c->n * k.lanes, NB_BLOCK);
     const int nbo = bonded_terms ? mdx_bonded_args(c, bonded_terms, &k.ba) : 0;
     calls.push_back(k);
     blocks.push_back(k.nb_blocks + nbo);
@@ -375,21 +395,14 @@ int mdx_batch_prepare_nb(mdx_ctx* const* cs, int n, unsigned bonded_terms, Batch
 }
 
 // LJ + direct-space Coulomb, the batched step's pair terms
-int mdx_batch_launch_nb(const BatchKind& k, int lanes, bool s14, bool energy, hipStream_t s) {
+int mdx_batch_launch_nb(const BatchKind& k, bool s14, bool energy, hipStream_t s) {
   const NbCall* calls = (const NbCall*)k.calls;
-#define NBB(E_, G_, S_) k_nonbonded_batch<true, true, E_, G_, S_><<<k.blocks, NB_BLOCK, 0, s>>>(k.map, calls)
-#define NBB_G(E_, S_)                 \
-  do {                                \
-    if (lanes == 16) NBB(E_, 16, S_); \
-    else if (lanes == 64) NBB(E_, 64, S_); \
-    else NBB(E_, 32, S_);             \
-  } while (0)
+#define NBB(E_, S_) k_nonbonded_batch<true, true, E_, S_><<<k.blocks, NB_BLOCK, 0, s>>>(k.map, calls)
   if (energy) {
-    if (s14) NBB_G(true, true); else NBB_G(true, false);
+    if (s14) NBB(true, true); else NBB(true, false);
   } else {
-    if (s14) NBB_G(false, true); else NBB_G(false, false);
+    if (s14) NBB(false, true); else NBB(false, false);
   }
-#undef NBB_G
 #undef NBB
   MDX_LAUNCH_CHECK();
   return 0;

@@ -10,8 +10,9 @@
 //
 // Layout: a group of G lanes per atom (16, 32 or 64, chosen by mdx_nonbonded_tune) in
 // cell-sorted order walks the atom's contiguous
-// neighbour list (coalesced index loads), gathers each neighbour's float4 (x, y, z, q*sqrt(ke))
-// and float2 (sigma/2, sqrt(24 eps)), and keeps partial forces in registers. Every pair is
+// neighbour list (coalesced index loads), gathers each neighbour's int4 (x, y, z as 32-bit
+// fractions of the box, q*sqrt(ke) as float bits) and float2 (sigma/2, sqrt(24 eps)), and keeps
+// partial forces in registers. Every pair is
 // evaluated from both ends (full list), so there are no atomics in the pair loop; the group
 // reduces with xor shuffles and adds each atom's force once to the int64 fixed-point
 // accumulator (deterministic).
@@ -24,7 +25,7 @@
 
 struct NbArgs {
   int n, cap;
-  float Lx, Ly, Lz, ix, iy, iz;
+  float sx, sy, sz, sx2, sy2, sz2;  // A per unit of a 32-bit box fraction, and squared
   float rc2, guard2;
   float beta, twob_sqrtpi;
   float ct_scale;  // Ewald-correction table pieces per A^2
@@ -74,6 +75,13 @@ static __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// v_cvt_u32_f32 as the instruction: it saturates, where a C++ conversion out of range is undefined
+static __device__ __forceinline__ unsigned cvt_u32(float x) {
+  unsigned r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+
 template <bool B>
 struct NbTail {
   static constexpr bool value = B;
@@ -84,7 +92,7 @@ struct NbTail {
 // index loads and its neighbours' position loads are contiguous; the group reduces its partial
 // forces with xor shuffles at the end.
 struct NbPtrs {
-  const float4* xq;
+  const int4* xf;
   const float2* ljs;
   const float2* ljs14;
   const int* nbr_count;
@@ -96,11 +104,16 @@ struct NbPtrs {
   DevState* st;
 };
 
-// S14: the list may hold 1-4 pairs (bit 31), which take the (sigma14, eps14) columns; without
+// VALU bound: about 34 instructions a slot for a wave without LJ and 44 with (54 before, with centred
+// float32 positions and an explicit minimum image, LJ for every slot, a cutoff branch per slot and a
+// shift per gathered array). 23,328 atoms, r_c 12 A, 1.5 A skin: 49.2 us (32 lanes) -> 40.8 us (16).
+// The box fractions also take the error of the forces against 64 bits from 2.2e-6 to 0.8e-6.
+//
+// S14: the list may hold 1-4 pairs (bit 0), which take the (sigma14, eps14) columns; without
 // any, the per-slot column choice is compiled out.
 template <bool LJ, bool COUL, bool ENERGY, int G, int BS, bool S14>
 __device__ __forceinline__ void nb_block(const NbArgs& a, const NbPtrs& P, int vb) {
-  const float4* __restrict__ xq = P.xq;
+  const int4* __restrict__ xf = P.xf;
   const float2* __restrict__ ljs = P.ljs;
   const float2* __restrict__ ljs14 = P.ljs14;
   const int* __restrict__ nbr_count = P.nbr_count;
@@ -111,15 +124,11 @@ __device__ __forceinline__ void nb_block(const NbArgs& a, const NbPtrs& P, int v
   long long* __restrict__ efix = P.efix;
   DevState* st = P.st;
   constexpr bool TAB = COUL && !ENERGY;
-#if NB_TAB_GLOBAL
-  const float4* __restrict__ ctab = a.ctab;
-#else
   __shared__ float4 ctab[TAB ? MDX_CTAB_N : 1];
   if (TAB) {
     for (int k = threadIdx.x; k < MDX_CTAB_N; k += blockDim.x) ctab[k] = a.ctab[k];
     __syncthreads();
   }
-#endif
   const int gt = vb * BS + threadIdx.x;
   const int s = gt / G;
   const int g = gt & (G - 1);
@@ -130,7 +139,8 @@ __device__ __forceinline__ void nb_block(const NbArgs& a, const NbPtrs& P, int v
   float fx = 0.f, fy = 0.f, fz = 0.f;
   double elj = 0.0, ec = 0.0;
   if (s < a.n) {
-    const float4 xi = xq[s];
+    const int4 xi = xf[s];
+    const float qi = __int_as_float(xi.w);
     float2 pi = make_float2(0.f, 0.f), pi14 = pi;
     if (LJ) {
       pi = ljs[s];
@@ -138,65 +148,74 @@ __device__ __forceinline__ void nb_block(const NbArgs& a, const NbPtrs& P, int v
     }
     const int cnt = nbr_count[s];
     const unsigned* lp = nbr_list + (long long)s * a.cap + g;
-    // neighbours are addressed by 32-bit byte offsets from the array bases (atom indices stay
-    // below 2^28), and the shifts that form them also drop the 1-4 flag in bit 31
-    const char* xqb = reinterpret_cast<const char*>(xq);
+    // list entries are 32-bit byte offsets into xf (slot * 16, atom indices stay below 2^28); bit 0
+    // marks a 1-4 pair. The pair's LJ columns are half as far into theirs.
+    const char* xfb = reinterpret_cast<const char*>(xf);
     const char* ljb = reinterpret_cast<const char*>(ljs);
     const char* lj14b = reinterpret_cast<const char*>(ljs14);
-    int oi = -1;
     // one pass over NB_U list entries per lane: all neighbour loads are issued before any is
     // consumed, so each pass waits for memory once, not 2*NB_U times. In the tail pass (tail =
     // NbTail<true>) bit u of `valid` marks the slots inside the row; the others hold the atom
-    // itself (zero separation: finite, and zeroed below)
-    auto pass = [&](const unsigned* e, unsigned valid, auto tail) {
-      constexpr bool TAIL = decltype(tail)::value;
-      float4 xj[NB_U];
+    // itself (zero separation: finite or zeroed below). lj = NbTail<false>: no lane of the wave
+    // has LJ parameters (its q_i is then applied to the sums once, at the end).
+    auto pass = [&](const unsigned* e, unsigned valid, auto tail, auto lj) {
+      constexpr bool TAIL = decltype(tail)::value, LJP = decltype(lj)::value;
+      int4 xj[NB_U];
       float2 pj[NB_U];
 #pragma unroll
       for (int u = 0; u < NB_U; ++u) {
-        xj[u] = *reinterpret_cast<const float4*>(xqb + (e[u] << 4));
-        if (LJ) pj[u] = *reinterpret_cast<const float2*>(((S14 && (e[u] >> 31)) ? lj14b : ljb) + (e[u] << 3));
+        const unsigned o = S14 ? e[u] & ~15u : e[u];
+        xj[u] = *reinterpret_cast<const int4*>(xfb + o);
+        if (LJP) pj[u] = *reinterpret_cast<const float2*>(((S14 && (e[u] & 1u)) ? lj14b : ljb) + (o >> 1));
+      }
+      // the wrapped difference of two 32-bit box fractions is the minimum image
+      float dx[NB_U], dy[NB_U], dz[NB_U], r2[NB_U];
+      bool in[NB_U];
+      float edge = 1e30f;
+#pragma unroll
+      for (int u = 0; u < NB_U; ++u) {
+        dx[u] = (float)(int)((unsigned)xj[u].x - (unsigned)xi.x);
+        dy[u] = (float)(int)((unsigned)xj[u].y - (unsigned)xi.y);
+        dz[u] = (float)(int)((unsigned)xj[u].z - (unsigned)xi.z);
+        r2[u] = dx[u] * dx[u] * a.sx2 + (dy[u] * dy[u] * a.sy2 + dz[u] * dz[u] * a.sz2);
+        const float past = r2[u] - a.rc2;
+        in[u] = past <= 0.f && (!TAIL || ((valid >> u) & 1u));
+        edge = fminf(edge, fabsf(past));
+      }
+      if (edge < a.guard2) {  // near the cutoff: decide in float64 like the reference (rare)
+        const int oi = sorted_orig[s];
+        for (int u = 0; u < NB_U; ++u)
+          if (fabsf(r2[u] - a.rc2) < a.guard2)
+            in[u] = within_cutoff64(pos, oi, sorted_orig[e[u] >> 4], a.Lxd, a.Lyd, a.Lzd, a.rcd);
       }
 #pragma unroll
       for (int u = 0; u < NB_U; ++u) {
-        float dx = xj[u].x - xi.x, dy = xj[u].y - xi.y, dz = xj[u].z - xi.z;
-        dx -= a.Lx * rintf(dx * a.ix);
-        dy -= a.Ly * rintf(dy * a.iy);
-        dz -= a.Lz * rintf(dz * a.iz);
-        const float r2 = dx * dx + dy * dy + dz * dz;
-        bool in = r2 <= a.rc2 && (!TAIL || ((valid >> u) & 1u));
-        if (fabsf(r2 - a.rc2) < a.guard2) {
-          // near the cutoff: decide in float64 like the reference (rare)
-          if (oi < 0) oi = sorted_orig[s];
-          in = within_cutoff64(pos, oi, sorted_orig[e[u] & 0x7fffffffu], a.Lxd, a.Lyd, a.Lzd, a.rcd);
-        }
         // out-of-cutoff and padding slots compute with their own r2 (> rc^2, or 0) and are
         // zeroed below; in-cutoff pairs have r2 >= ~0.5 A^2, never denormal for v_rsq_f32
-        const float rinv = __builtin_amdgcn_rsqf(r2);
+        const float rinv = __builtin_amdgcn_rsqf(r2[u]);
         const float r2inv = rinv * rinv;
+        const float qj = __int_as_float(xj[u].w);
         float fr = 0.f;
-        if (LJ) {
-          const float2 pp = (S14 && (e[u] >> 31)) ? pi14 : pi;
+        if (LJP) {
+          const float2 pp = (S14 && (e[u] & 1u)) ? pi14 : pi;
           const float sig = pp.x + pj[u].x;
-          const float eps = pp.y * pj[u].y;
+          const float eps = pp.y * pj[u].y;  // 24 eps_ij
           const float s2 = sig * sig * r2inv;
           const float s6 = s2 * s2 * s2;
-          const float s12 = s6 * s6;
-          fr -= eps * (2.f * s12 - s6) * r2inv;  // eps holds 24 eps_ij
-          if (ENERGY) elj += in ? (double)(eps * (1.f / 6.f) * (s12 - s6)) : 0.0;
+          fr -= eps * s6 * fmaf(2.f, s6, -1.f) * r2inv;
+          if (ENERGY) elj += in[u] ? (double)(eps * (1.f / 6.f) * (s6 * s6 - s6)) : 0.0;
         }
+        const float qq = LJP ? qi * qj : qj;
         if (TAB) {
-          const float zt = r2 * a.ct_scale;
-          const float fl = floorf(zt);
-          const float t = zt - fl;
-          // clamp in float before the conversion: beyond the cutoff the index stays inside
-          // the table
-          const float4 cf = ctab[(int)fminf(fl, (float)(MDX_CTAB_N - 1))];
+          const float zt = r2[u] * a.ct_scale;
+          // piece index as a byte offset, masked (beyond the cutoff it stays inside the table)
+          const unsigned at = cvt_u32(zt) << 4 & (MDX_CTAB_N - 1) << 4;
+          const float t = __builtin_amdgcn_fractf(zt);
+          const float4 cf = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(ctab) + at);
           const float gz = fmaf(t, fmaf(t, fmaf(t, cf.w, cf.z), cf.y), cf.x);
-          fr -= xi.w * xj[u].w * (rinv * r2inv - gz);
+          fr -= qq * fmaf(rinv, r2inv, -gz);
         } else if (COUL) {
-          const float qq = xi.w * xj[u].w;
-          const float x = a.beta * (r2 * rinv);
+          const float x = a.beta * (r2[u] * rinv);
           const float ex = __expf(-x * x);
           // 1/(1 + p x): v_rcp_f32 plus one Newton step (the raw 1-ulp reciprocal is biased, and the
           // direct-space energy sum cancels strongly enough to show it)
@@ -207,41 +226,55 @@ __device__ __forceinline__ void nb_block(const NbArgs& a, const NbPtrs& P, int v
               ERFC_C1 + tt * (ERFC_C2 + tt * (ERFC_C3 + tt * (ERFC_C4 + tt * (ERFC_C5 + tt * (ERFC_C6 + tt * ERFC_C7)))));
           const float erfcx = tt * poly * ex;
           fr -= qq * (erfcx * rinv + a.twob_sqrtpi * ex) * r2inv;
-          if (ENERGY) ec += in ? (double)(qq * erfcx * rinv) : 0.0;
+          if (ENERGY) ec += in[u] ? (double)(qq * erfcx * rinv) : 0.0;
         }
-        fr = in ? fr : 0.f;
-        fx += fr * dx;
-        fy += fr * dy;
-        fz += fr * dz;
+        fr = in[u] ? fr : 0.f;
+        fx += fr * dx[u];
+        fy += fr * dy[u];
+        fz += fr * dz[u];
       }
     };
     // whole chunks of G * NB_U entries: unpredicated index loads, the next chunk's issued before
     // this chunk is evaluated (the rows are followed by slack, so a load past a row's end reads
     // the next row or the slack and is never used)
-    int cb = 0;
-    if (G * NB_U <= cnt) {
-      unsigned e[NB_U];
+    auto row = [&](auto lj) {
+      int cb = 0;
+      if (G * NB_U <= cnt) {
+        unsigned e[NB_U];
 #pragma unroll
-      for (int u = 0; u < NB_U; ++u) e[u] = lp[u * G];
-      for (; cb + G * NB_U <= cnt; cb += G * NB_U) {
-        unsigned en[NB_U];
+        for (int u = 0; u < NB_U; ++u) e[u] = lp[u * G];
+        for (; cb + G * NB_U <= cnt; cb += G * NB_U) {
+          unsigned en[NB_U];
 #pragma unroll
-        for (int u = 0; u < NB_U; ++u) en[u] = lp[cb + G * NB_U + u * G];
-        pass(e, 0u, NbTail<false>());
+          for (int u = 0; u < NB_U; ++u) en[u] = lp[cb + G * NB_U + u * G];
+          pass(e, 0u, NbTail<false>(), lj);
 #pragma unroll
-        for (int u = 0; u < NB_U; ++u) e[u] = en[u];
+          for (int u = 0; u < NB_U; ++u) e[u] = en[u];
+        }
       }
-    }
-    if (cb < cnt) {  // the row's last, partial chunk: slots past the end take the atom itself
-      unsigned e[NB_U], valid = 0;
+      if (cb < cnt) {  // the row's last, partial chunk: slots past the end take the atom itself
+        unsigned e[NB_U], valid = 0;
 #pragma unroll
-      for (int u = 0; u < NB_U; ++u) {
-        const bool v = cb + g + u * G < cnt;
-        e[u] = v ? lp[cb + u * G] : (unsigned)s;
-        valid |= (v ? 1u : 0u) << u;
+        for (int u = 0; u < NB_U; ++u) {
+          const bool v = cb + g + u * G < cnt;
+          e[u] = v ? lp[cb + u * G] : (unsigned)s << 4;
+          valid |= (v ? 1u : 0u) << u;
+        }
+        pass(e, valid, NbTail<true>(), lj);
       }
-      pass(e, valid, NbTail<true>());
-    }
+    };
+    // Atoms without LJ parameters (eps = 0 in both columns) add no LJ to any pair. Within a cell they
+    // are sorted after the others (grid_sort_fill_block), so most waves hold only one kind and
+    // the waves of the other kind leave out the LJ loads and arithmetic (about 13 of 47 VALU
+    // instructions a slot).
+    const bool any_lj = LJ && __ballot(pi.y != 0.f || (S14 && pi14.y != 0.f)) != 0;
+    if (any_lj) row(NbTail<true>());
+    else if (COUL) row(NbTail<false>());
+    const float c = any_lj ? 1.f : qi;
+    fx *= c * a.sx;
+    fy *= c * a.sy;
+    fz *= c * a.sz;
+    if (ENERGY && !any_lj) ec *= (double)qi;
   }
   for (int off = G / 2; off > 0; off >>= 1) {
     fx += __shfl_xor(fx, off, 64);

@@ -1167,8 +1167,7 @@ int mdx_pme_enqueue_part(mdx_ctx* c, int part) {
 
 bool mdx_force_phases_ok(const mdx_ctx* c) {
   return c->phases_on && c->pme_configured && c->pme_planes && c->pme_wf_phase > 0 && c->pme_fused_B > 0 &&
-         c->nb_configured && c->has_lj && c->has_charges &&
-         (c->nb_lanes == 16 || c->nb_lanes == 32 || c->nb_lanes == 64);
+         c->nb_configured && c->has_lj && c->has_charges;
 }
 
 int mdx_force_phases_enqueue(mdx_ctx* c, bool energy, unsigned bonded_terms) {
@@ -1225,7 +1224,7 @@ int mdx_force_phases_enqueue(mdx_ctx* c, bool energy, unsigned bonded_terms) {
             "Ewald-correction table not built for the current beta and cutoff");
   BondedArgs ba{};
   const int nbo = bonded_terms ? mdx_bonded_args(c, bonded_terms, &ba, PLANE_THREADS) : 0;
-  const int G = c->nb_lanes;
+  const int G = mdx_nb_lanes(c);
   const int nbt = (int)div_up((long long)c->n * G, PLANE_THREADS);
   const int n0 = std::min(nbt, (int)(c->phase_frac[0] * nbt + 0.5));
   const int n1 = std::min(nbt - n0, (int)(c->phase_frac[1] * nbt + 0.5));
