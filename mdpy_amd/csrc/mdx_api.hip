@@ -819,7 +819,7 @@ extern "C" int mdx_ctx_destroy(mdx_ctx* c) {
   c->cell_count.release(); c->cell_start.release(); c->cell_cursor.release(); c->atom_cell.release();
   c->sorted_orig.release(); c->orig_sorted.release(); c->xq.release(); c->xf.release(); c->ljs.release(); c->ljs14.release();
   c->ref_cell_sorted.release(); c->pos_at_build.release(); c->nbr_count.release(); c->nbr_list.release();
-  c->d_stencil.release(); c->qfix.release(); c->cgrid.release(); c->conv.release(); c->bc.release();
+  c->d_stencil.release(); c->qfix.release(); c->cgrid.release(); c->conv.release(); c->bc.release(); c->bch.release();
   c->twiddle.release(); c->excl_pairs.release(); c->xa.release(); c->xb.release(); c->va.release();
   c->vb.release(); c->acc_prev.release(); c->acc_cur.release(); c->ehist.release(); c->tmp64.release();
   c->pc_part.release();

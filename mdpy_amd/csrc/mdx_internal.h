@@ -16,7 +16,18 @@ static constexpr double kFixScale = 1099511627776.0;          // 2^40
 static constexpr double kFixInv = 1.0 / 1099511627776.0;
 
 __device__ __forceinline__ long long to_fix(double v) { return __double2ll_rn(v * kFixScale); }
-__device__ __forceinline__ long long to_fix_f(float v) { return __double2ll_rn((double)v * kFixScale); }
+// v * 2^40 rounded to nearest even, in float32: the scaling and both words' split are exact. The
+// conversions are the instructions themselves, which saturate (and give 0 for NaN).
+__device__ __forceinline__ long long to_fix_f(float v) {
+  const float f = rintf(v * 1099511627776.f);
+  const float h = floorf(f * 0x1p-32f);
+  const float l = fmaf(-h, 4294967296.f, f);  // 0 <= l < 2^32
+  int hi;
+  unsigned lo;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(hi) : "v"(h));
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(lo) : "v"(l));
+  return (long long)(((unsigned long long)(unsigned)hi << 32) | lo);
+}
 
 // Orders one wave's LDS writes before its later LDS reads (and the reads before later writes):
 // a wave's LDS operations complete in program order, so only compiler motion must be stopped.
@@ -100,8 +111,7 @@ struct DevState {
   int maxpc;                // largest cell population (reference binning)
   int pad;
   long long hist_base;      // step counter value at the start of the current integrate call
-  int pme_slots;            // reciprocal force slots written in the current evaluation
-  unsigned pme_ticket;      // finished blocks of the PME gather kernel
+  unsigned long long pme_count;  // PME gather: slots written (40 bits) and finished plane workgroups
   unsigned step_ticket;     // finished blocks of the fused step prologue
   unsigned bar_count;       // grid barrier of the fused PME kernel: blocks arrived
   unsigned bar_gen;         // and its generation (advanced by the last arrival)
@@ -295,6 +305,7 @@ struct mdx_ctx {
   DevBuf<float2> cgrid;          // complex work grid
   DevBuf<float> conv;            // real convolved grid
   DevBuf<float> bc;              // influence function B*C (float)
+  DevBuf<float> bch;             // the same over the plane path's half spectrum (kz <= Kz/2)
   DevBuf<float2> twiddle;        // per axis, K entries each (3 * maxK)
   DevBuf<int> excl_pairs;        // unique excluded pairs (i<j), 2 x n_excl_pairs
   int n_excl_pairs = 0;

@@ -4,8 +4,9 @@
 //
 //   spread   order-4 cardinal B-splines, q_i * sqrt(ke) added to an int64 fixed-point grid
 //            (deterministic), one lane per atom
-//   FFT      hand-written mixed-radix (2,3,4,5) Stockham passes in LDS, one kernel per axis;
-//            the x-axis kernel also applies the influence function B*C, sums the reciprocal
+//   FFT      hand-written mixed-radix (2 ... 16) Stockham passes in LDS. The charge grid is real, so
+//            two rows along z share one complex transform and Kz/2 + 1 columns go on along y and
+//            x; the x-axis kernel also applies the influence function B*C, sums the reciprocal
 //            energy and runs the inverse x transform on the same LDS tile
 //   gather   one lane per atom, 64 grid values, force = -q grad(theta) . conv
 //   corrections  float64 excluded-pair erf correction, self energy and neutralising background,
@@ -17,9 +18,9 @@
 
 #define PME_BLOCK 256
 #define FFT_THREADS 256
-#define MAX_RADICES 16
+#define MAX_RADICES 8
 
-// radix of pass p in bits [4p, 4p+4) of `code` (a register-friendly stand-in for an array that
+// radix of pass p in bits [8p, 8p+8) of `code` (a register-friendly stand-in for an array that
 // a dynamically indexed kernel argument would otherwise put in scratch memory)
 struct FftPlan {
   int K;
@@ -79,112 +80,123 @@ __device__ __forceinline__ void dft5(float2* u, float s) {
   u[3] = csub(p2, q2);
 }
 
+// W_R^j = cos(2 pi j / R) + i sin(2 pi j / R) of the composite radices
+template <int R> struct Roots;
+template <> struct Roots<6> { static constexpr float w[6][2] = {{1.0f, 0.0f}, {0.5f, 0.866025404f}, {-0.5f, 0.866025404f}, {-1.0f, 1.2246468e-16f}, {-0.5f, -0.866025404f}, {0.5f, -0.866025404f}}; };
+template <> struct Roots<8> { static constexpr float w[8][2] = {{1.0f, 0.0f}, {0.707106781f, 0.707106781f}, {6.123234e-17f, 1.0f}, {-0.707106781f, 0.707106781f}, {-1.0f, 1.2246468e-16f}, {-0.707106781f, -0.707106781f}, {-1.8369702e-16f, -1.0f}, {0.707106781f, -0.707106781f}}; };
+template <> struct Roots<9> { static constexpr float w[9][2] = {{1.0f, 0.0f}, {0.766044443f, 0.64278761f}, {0.173648178f, 0.984807753f}, {-0.5f, 0.866025404f}, {-0.939692621f, 0.342020143f}, {-0.939692621f, -0.342020143f}, {-0.5f, -0.866025404f}, {0.173648178f, -0.984807753f}, {0.766044443f, -0.64278761f}}; };
+template <> struct Roots<10> { static constexpr float w[10][2] = {{1.0f, 0.0f}, {0.809016994f, 0.587785252f}, {0.309016994f, 0.951056516f}, {-0.309016994f, 0.951056516f}, {-0.809016994f, 0.587785252f}, {-1.0f, 1.2246468e-16f}, {-0.809016994f, -0.587785252f}, {-0.309016994f, -0.951056516f}, {0.309016994f, -0.951056516f}, {0.809016994f, -0.587785252f}}; };
+template <> struct Roots<12> { static constexpr float w[12][2] = {{1.0f, 0.0f}, {0.866025404f, 0.5f}, {0.5f, 0.866025404f}, {6.123234e-17f, 1.0f}, {-0.5f, 0.866025404f}, {-0.866025404f, 0.5f}, {-1.0f, 1.2246468e-16f}, {-0.866025404f, -0.5f}, {-0.5f, -0.866025404f}, {-1.8369702e-16f, -1.0f}, {0.5f, -0.866025404f}, {0.866025404f, -0.5f}}; };
+template <> struct Roots<16> { static constexpr float w[16][2] = {{1.0f, 0.0f}, {0.923879533f, 0.382683432f}, {0.707106781f, 0.707106781f}, {0.382683432f, 0.923879533f}, {6.123234e-17f, 1.0f}, {-0.382683432f, 0.923879533f}, {-0.707106781f, 0.707106781f}, {-0.923879533f, 0.382683432f}, {-1.0f, 1.2246468e-16f}, {-0.923879533f, -0.382683432f}, {-0.707106781f, -0.707106781f}, {-0.382683432f, -0.923879533f}, {-1.8369702e-16f, -1.0f}, {0.382683432f, -0.923879533f}, {0.707106781f, -0.707106781f}, {0.923879533f, -0.382683432f}}; };
+
+template <int R>
+__device__ __forceinline__ void dft(float2* u, float s);
+// R = R1 R2: R2 transforms of R1 points (stride R2), the roots between, R1 transforms of R2 points
+template <int R1, int R2>
+__device__ __forceinline__ void dft_split(float2* u, float s) {
+  constexpr int R = R1 * R2;
+  float2 v[R];
+#pragma unroll
+  for (int b = 0; b < R2; ++b) {
+    float2 x[R1];
+#pragma unroll
+    for (int a = 0; a < R1; ++a) x[a] = u[a * R2 + b];
+    dft<R1>(x, s);
+#pragma unroll
+    for (int k = 0; k < R1; ++k) {
+      const int j = b * k % R;
+      v[k * R2 + b] = j == 0 ? x[k] : cmul(x[k], make_float2(Roots<R>::w[j][0], s * Roots<R>::w[j][1]));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < R1; ++k) {
+    dft<R2>(v + k * R2, s);
+#pragma unroll
+    for (int m = 0; m < R2; ++m) u[k + R1 * m] = v[k * R2 + m];
+  }
+}
+template <int R>
+__device__ __forceinline__ void dft(float2* u, float s) {
+  if constexpr (R == 2) dft2(u);
+  else if constexpr (R == 3) dft3(u, s);
+  else if constexpr (R == 4) dft4(u, s);
+  else if constexpr (R == 5) dft5(u, s);
+  else if constexpr (R == 6) dft_split<2, 3>(u, s);
+  else if constexpr (R == 8) dft_split<2, 4>(u, s);
+  else if constexpr (R == 9) dft_split<3, 3>(u, s);
+  else if constexpr (R == 10) dft_split<2, 5>(u, s);
+  else if constexpr (R == 12) dft_split<3, 4>(u, s);
+  else dft_split<4, 4>(u, s);
+}
+
 // one Stockham pass of radix R over B lines (element e of line l at l*ls + e*es); p is the
-// product of the radices of the passes already done
-template <int DIR, int R>
-__device__ __forceinline__ void stockham_pass(const float2* src, float2* dst, int K, int p, int B,
-                                              const float2* __restrict__ tw, int ls, int es) {
-  const int T = K / R;
-  const int tstep = K / (p * R);
-  const float s = (float)DIR;
+// product of the radices of the passes already done, rest = K/p, iB and ip the reciprocals of B and
+// p. Consecutive lanes take consecutive lines:
+// with ls odd or 1 (in 8-byte elements) every LDS access falls on distinct banks. The quotients by
+// B and p are exact in float32 (operands below 2^20).
+template <int R>
+__device__ __forceinline__ void stockham_pass(const float2* src, float2* dst, int K, int p, int rest, int B, float iB,
+                                              float ip, const float2* __restrict__ tw, int ls, int es, float s) {
+  const int T = K / R;         // uniform: scalar multiplications
+  const int tstep = rest / R;  // K / (p R)
   for (int b = threadIdx.x; b < B * T; b += blockDim.x) {
-    int l, i;
-    if (es == 1) { l = b / T; i = b - l * T; }
-    else { i = b / B; l = b - i * B; }
-    const int k = i % p;
+    const int i = (int)(((float)b + 0.5f) * iB), l = b - i * B;
+    const int k = i - (int)(((float)i + 0.5f) * ip) * p;  // i mod p
     const float2* X = src + l * ls;
     float2* Y = dst + l * ls;
     float2 u[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) u[r] = X[(i + r * T) * es];
+    if (p > 1) {
 #pragma unroll
-    for (int r = 1; r < R; ++r) {
-      float2 w = tw[(r * k * tstep) % K];
-      if (DIR > 0) w.y = -w.y;
-      u[r] = cmul(u[r], w);
+      for (int r = 1; r < R; ++r) {
+        float2 w = tw[r * k * tstep];  // r k T/p < K; exp(-2 pi i j/K), conjugated for the inverse
+        w.y *= -s;
+        u[r] = cmul(u[r], w);
+      }
     }
-    if constexpr (R == 2) dft2(u);
-    else if constexpr (R == 3) dft3(u, s);
-    else if constexpr (R == 4) dft4(u, s);
-    else dft5(u, s);
+    dft<R>(u, s);
     const int j = (i - k) * R + k;
 #pragma unroll
     for (int r = 0; r < R; ++r) Y[(j + r * p) * es] = u[r];
   }
 }
 
-// B lines of length K held in LDS (src); element e of line l sits at l*ls + e*es. Stockham
-// passes ping-pong with dst; returns the buffer holding the result. Consecutive threads take
-// consecutive elements of a line when es == 1 and consecutive lines otherwise, so LDS accesses
-// stay on distinct banks for both contiguous and strided lines.
-template <int DIR>
-__device__ float2* lds_fft(float2* src, float2* dst, const FftPlan& pl, int B, const float2* __restrict__ tw,
-                           int ls = -1, int es = 1) {
+// B lines of length K held in LDS (src); element e of line l sits at l*ls + e*es; s = -1 forward,
+// +1 inverse. Stockham passes ping-pong with dst; returns the buffer holding the result. The
+// kernels run every transform of a workgroup through one call in a loop: a pass is a few hundred
+// instructions that a latency-bound workgroup executes once, so a second copy of the code
+// (another direction or axis) costs its instruction fetches again.
+__device__ __forceinline__ float2* lds_fft(float2* src, float2* dst, const FftPlan& pl, int B,
+                                           const float2* __restrict__ tw, int ls, int es, float s) {
   const int K = pl.K;
-  if (ls < 0) ls = K;
-  int p = 1;
+  const float iB = __builtin_amdgcn_rcpf((float)B);
+  float ip = 1.f;
+  int p = 1, rest = K;
+#pragma unroll 1
   for (int pass = 0; pass < pl.nrad; ++pass) {
-    const int R = (int)((pl.code >> (4 * pass)) & 15ull);
+    const int R = (int)((pl.code >> (8 * pass)) & 255ull);
     switch (R) {
-      case 2: stockham_pass<DIR, 2>(src, dst, K, p, B, tw, ls, es); break;
-      case 3: stockham_pass<DIR, 3>(src, dst, K, p, B, tw, ls, es); break;
-      case 4: stockham_pass<DIR, 4>(src, dst, K, p, B, tw, ls, es); break;
-      default: stockham_pass<DIR, 5>(src, dst, K, p, B, tw, ls, es); break;
+      case 2: stockham_pass<2>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 3: stockham_pass<3>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 4: stockham_pass<4>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 5: stockham_pass<5>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 6: stockham_pass<6>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 8: stockham_pass<8>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 9: stockham_pass<9>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 10: stockham_pass<10>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      case 12: stockham_pass<12>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
+      default: stockham_pass<16>(src, dst, K, p, rest, B, iB, ip, tw, ls, es, s); break;
     }
     __syncthreads();
     float2* t = src;
     src = dst;
     dst = t;
     p *= R;
+    rest = K / p;
+    ip = __builtin_amdgcn_rcpf((float)p);
   }
   return src;
-}
-
-// ---- 64 x 64 planes: each wave transforms 4 whole lines, so the three radix-4 Stockham passes
-// of a 64-point line need only wave-level ordering (no workgroup barrier between passes), and
-// every index is a compile-time shift or mask. Planes are held with row stride 65 (PLANE64_LS)
-// so that both rows and columns are read across lanes without LDS bank conflicts.
-#define PLANE64_LS 65
-
-// one radix-4 pass (p = 4^S) of the 64-point line at X/Y + off, elements es apart; lane i of
-// the line's 16 computes butterfly i
-template <int DIR, int S>
-__device__ __forceinline__ void fft64_pass(const float2* X, float2* Y, int off, int es, int i,
-                                           const float2* __restrict__ tw) {
-  constexpr int p = 1 << (2 * S);
-  constexpr int tstep = 16 >> (2 * S);
-  const int k = i & (p - 1);
-  float2 u[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) u[r] = X[off + (i + 16 * r) * es];
-  if (S > 0) {
-#pragma unroll
-    for (int r = 1; r < 4; ++r) {
-      float2 w = tw[(r * k * tstep) & 63];
-      if (DIR > 0) w.y = -w.y;
-      u[r] = cmul(u[r], w);
-    }
-  }
-  dft4(u, (float)DIR);
-  const int j = ((i - k) << 2) + k;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) Y[off + (j + r * p) * es] = u[r];
-}
-
-// 64-point transforms of the 4 nw rows (rows = true: elements contiguous) or columns of a
-// padded plane in a (nw = waves of the block), with b as the ping-pong buffer; the result ends in
-// b. Wave w takes lines w, w + nw, w + 2 nw, w + 3 nw.
-template <int DIR>
-__device__ __forceinline__ void plane64_lines(float2* a, float2* b, bool rows, const float2* __restrict__ tw) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int line = w + nw * (lane >> 4), i = lane & 15;
-  const int off = rows ? line * PLANE64_LS : line;
-  const int es = rows ? 1 : PLANE64_LS;
-  fft64_pass<DIR, 0>(a, b, off, es, i, tw);
-  wave_lds_sync();
-  fft64_pass<DIR, 1>(b, a, off, es, i, tw);
-  wave_lds_sync();
-  fft64_pass<DIR, 2>(a, b, off, es, i, tw);
 }
 
 __device__ __forceinline__ void load_twiddles(float2* dst, const float2* __restrict__ src, int K) {
@@ -195,20 +207,19 @@ __device__ __forceinline__ long long line_base(const FftLines& ln, int l) {
   return (long long)(l / ln.inner) * ln.outer_stride + (long long)(l % ln.inner) * ln.inner_stride;
 }
 
+// The axis passes of the path without plane kernels (a full complex grid).
 // MODE 0: complex in/out.  MODE 1: load int64 fixed grid (real), clear it.  MODE 2: store real
 // part to a float grid.  MODE 3: forward, multiply by B*C (+ energy), inverse, in place.
 // lines [l0, l0 + B) of one axis pass, by one workgroup, in the LDS region lds
 template <int DIR, int MODE>
-__device__ void fft_axis_body(const FftPlan& pl, const FftLines& ln, const float2* __restrict__ tw,
+__device__ __forceinline__ void fft_axis_body(const FftPlan& pl, const FftLines& ln, const float2* __restrict__ tw,
                               float2* __restrict__ cg, long long* __restrict__ qfix, float* __restrict__ rout,
                               const float* __restrict__ bc, long long* __restrict__ eslot, int l0, float2* lds) {
   const int K = pl.K;
   const int B = ln.B;
   const int nb = min(B, ln.nlines - l0);
   const bool contiguous = ln.estride == 1;
-  // lines of strided axes are loaded line-across-lanes: pad the LDS line stride to K + 1 so
-  // consecutive lanes fall on different banks
-  const int ls = contiguous ? K : K + 1;
+  const int ls = K | 1;  // odd: lanes on consecutive lines use distinct banks
   float2* A = lds;
   float2* Bf = lds + B * ls;
   float2* stw = Bf + B * ls;
@@ -230,36 +241,27 @@ __device__ void fft_axis_body(const FftPlan& pl, const FftLines& ln, const float
     A[l * ls + e] = v;
   }
   __syncthreads();
-  // 64-point strided lines, four per wave: wave-level passes (padded stride 65)
-  const bool w64 = K == 64 && !contiguous && nb == B && B == 4 * (int)(blockDim.x >> 6);
-  float2* res;
-  if (w64) {
-    plane64_lines<DIR>(A, Bf, true, stw);
-    res = Bf;
-    __syncthreads();
-  } else {
-    res = lds_fft<DIR>(A, Bf, pl, nb, stw, ls);
-  }
-  if (MODE == 3) {
-    float2* other = (res == A) ? Bf : A;
-    double en = 0.0;
-    for (int idx = threadIdx.x; idx < nb * K; idx += blockDim.x) {
-      int l = idx / K, e = idx - l * K;
-      long long g = line_base(ln, l0 + l) + (long long)e * ln.estride;
-      float f = bc[g];
-      float2 v = res[l * ls + e];
-      en += 0.5 * (double)f * ((double)v.x * v.x + (double)v.y * v.y);
-      res[l * ls + e] = cscale(v, f);
-    }
-    __syncthreads();
-    if (w64) {
-      plane64_lines<-DIR>(res, other, true, stw);
-      res = other;
+  float2* res = A;
+  float2* other = Bf;
+  double en = 0.0;
+#pragma unroll 1
+  for (int q = 0; q < (MODE == 3 ? 2 : 1); ++q) {
+    float2* r = lds_fft(res, other, pl, nb, stw, ls, 1, MODE == 3 && q == 1 ? (float)-DIR : (float)DIR);
+    other = r == res ? other : res;
+    res = r;
+    if (MODE == 3 && q == 0) {
+      for (int idx = threadIdx.x; idx < nb * K; idx += blockDim.x) {
+        int l = idx / K, e = idx - l * K;
+        long long g = line_base(ln, l0 + l) + (long long)e * ln.estride;
+        float f = bc[g];
+        float2 v = res[l * ls + e];
+        en += 0.5 * (double)f * ((double)v.x * v.x + (double)v.y * v.y);
+        res[l * ls + e] = cscale(v, f);
+      }
       __syncthreads();
-    } else {
-      res = lds_fft<-DIR>(res, other, pl, nb, stw, ls);
     }
-    // block energy
+  }
+  if (MODE == 3) {  // block energy
     __shared__ double sm[16];
     for (int off = 32; off > 0; off >>= 1) en += __shfl_xor(en, off, 64);
     if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = en;
@@ -289,6 +291,90 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftPlan pl, FftLines l
                                                         long long* __restrict__ eslot) {
   extern __shared__ float2 lds[];
   fft_axis_body<DIR, MODE>(pl, ln, tw, cg, qfix, rout, bc, eslot, blockIdx.x * ln.B, lds);
+}
+
+// The x-axis pass of the plane path: lines [l0, l0 + B) of the nl = Ky nz columns (y, kz) of the
+// half spectrum, element x of line l at x nl + l. Forward transform, multiply by B C (`bc`, same
+// layout), reciprocal energy (a column stands for its mirror image too, except kz = 0 and, for
+// even Kz, kz = Kz/2), inverse transform, in place.
+#define XBC 6  // elements per lane whose influence function is loaded ahead
+struct XPass {
+  FftPlan pl;
+  int nl, nz, kz_even, B;
+};
+__device__ __forceinline__ void fft_x_body(const XPass& xp, const float2* __restrict__ tw, float2* __restrict__ cg,
+                           const float* __restrict__ bc, long long* __restrict__ eslot, int l0, float2* lds) {
+  __shared__ double sm[16];
+  const int K = xp.pl.K, nb = min(xp.B, xp.nl - l0);
+  const int es = xp.B | 1;  // odd: the lanes' strided stores of a pass spread over the banks
+  float2* A = lds;
+  float2* Bf = lds + es * K;
+  float2* stw = Bf + es * K;
+  load_twiddles(stw, tw, K);
+  const float inb = 1.f / (float)nb;
+  float fc[XBC];  // influence function of this lane's first elements, loaded with the grid
+#pragma unroll
+  for (int q = 0; q < XBC; ++q) {
+    const int idx = threadIdx.x + q * blockDim.x;
+    fc[q] = 0.f;
+    if (idx < nb * K) {
+      const int e = (int)(((float)idx + 0.5f) * inb), l = idx - e * nb;
+      const long long g = (long long)e * xp.nl + l0 + l;
+      fc[q] = bc[g];
+      A[e * es + l] = cg[g];
+    }
+  }
+  for (int idx = threadIdx.x + XBC * blockDim.x; idx < nb * K; idx += blockDim.x) {
+    const int e = (int)(((float)idx + 0.5f) * inb), l = idx - e * nb;
+    A[e * es + l] = cg[(long long)e * xp.nl + l0 + l];
+  }
+  __syncthreads();
+  float2* res = A;
+  float2* other = Bf;
+  double en = 0.0;
+#pragma unroll 1
+  for (int q = 0; q < 2; ++q) {
+    float2* r = lds_fft(res, other, xp.pl, nb, stw, 1, es, q == 0 ? -1.f : 1.f);
+    other = r == res ? other : res;
+    res = r;
+    if (q == 1) break;
+    auto times = [&](int idx, bool held, float fh) {
+      const int e = (int)(((float)idx + 0.5f) * inb), l = idx - e * nb;
+      const float f = held ? fh : bc[(long long)e * xp.nl + l0 + l];
+      const float2 v = res[e * es + l];
+      const int kz = (l0 + l) % xp.nz;
+      const double w = kz == 0 || (xp.kz_even && kz == xp.nz - 1) ? 0.5 : 1.0;
+      en += w * (double)f * ((double)v.x * v.x + (double)v.y * v.y);
+      res[e * es + l] = cscale(v, f);
+    };
+#pragma unroll
+    for (int k = 0; k < XBC; ++k)
+      if ((int)(threadIdx.x + k * blockDim.x) < nb * K) times(threadIdx.x + k * blockDim.x, true, fc[k]);
+    for (int idx = threadIdx.x + XBC * blockDim.x; idx < nb * K; idx += blockDim.x) times(idx, false, 0.f);
+    __syncthreads();
+  }
+  for (int idx = threadIdx.x; idx < nb * K; idx += blockDim.x) {
+    const int e = (int)(((float)idx + 0.5f) * inb), l = idx - e * nb;
+    cg[(long long)e * xp.nl + l0 + l] = res[e * es + l];
+  }
+  for (int off = 32; off > 0; off >>= 1) en += __shfl_xor(en, off, 64);
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = en;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double sacc = 0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) sacc += sm[w];
+    atomicAdd((unsigned long long*)eslot, (unsigned long long)to_fix(sacc));
+  }
+}
+
+// Latency bound: one 128-byte segment per x and workgroup, two register-level passes each way.
+#define FFTX_THREADS 128
+#define FFTX_B 8
+__global__ __launch_bounds__(FFTX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fft_x(XPass xp, const float2* __restrict__ tw,
+                                                        float2* __restrict__ cg, const float* __restrict__ bc,
+                                                        long long* __restrict__ eslot) {
+  extern __shared__ float2 lds[];
+  fft_x_body(xp, tw, cg, bc, eslot, blockIdx.x * xp.B, lds);
 }
 
 // ---------------------------------------------------------------- spread / gather
@@ -406,26 +492,31 @@ __global__ __launch_bounds__(PME_BLOCK) void k_gather(PmeArgs a, const double* _
 // x0 for some kx in 0..3) are found in the cell-sorted atom order of the neighbour-list grid:
 // cells are x-major, so the x-slices of cells that can hold such atoms form at most two
 // contiguous ranges of sorted slots, and no atom is more than skin/2 away from its slice.
-// Phase 1 (one lane per candidate) compacts the touching atoms into LDS records; phase 2 gives
-// each record 16 lanes, one per (ky, kz) point of its 4x4 stencil in the plane.
-#define PLANE_THREADS 1024  // the 64 x 64 wave-level transforms need all 16 waves (4 lines each)
+// Phase 1 (one lane per candidate) lists the touching atoms' slots in LDS; phase 2 (one lane per
+// touching atom) computes its splines, adds its 4x4 points and writes the record that the gather
+// reads. A plane occupies one compute unit and its VALU and LDS atomics bound it, so both kernels
+// are written for few instructions: the second phase runs on touching atoms only (a quarter of the
+// candidates), the gather uses one lane per record (the splines once, not once per ky), and the
+// set-up of a transform pass runs on scalars (16 waves repeat it). Forward / x pass / gather alone:
+// 23,328 atoms, 64^3 20.7 / 8.8 / 16.2 -> 17.1 / 11.1 / 10.3 us; 30,021 atoms, 72^3 28.9 / 16.3 / 27.0
+// -> 17.7 / 12.7 / 11.4; 98,304 atoms, 100^3 31.5 / 19.1 / 18.2, against 292 on the global grid, which
+// complex planes in LDS left to grids beyond 81 x 81 (half spectra reach 128 x 128).
+#define PLANE_THREADS 1024
+#define PLANE_REG 8  // row pairs' values held per lane between the two layouts of a plane
 
 struct PlaneArgs {
   int n;
   int Kx, Ky, Kz;
   double Lx, Ly, Lz;
   double iLx, iLy, iLz;
+  double gx, gy, gz;  // grid points per A
   int gnx, gny, gnz;  // neighbour-list grid
   double wx;          // its cell width along x
   double margin;      // list skin/2 plus rounding slack
-  int W;              // candidates examined per round (bounded by the LDS record space)
+  int W;              // candidates examined per round (bounded by the LDS list of touching ones)
   int rec_cap;        // gather records per plane in global memory
 };
 
-struct SpreadRec {  // 16 B
-  int yz;           // by | bz << 12
-  float wy, wz, qx; // fractional offsets, q sqrt(ke) theta_kx(wx)
-};
 struct GatherRec {  // 24 B (stored in an int buffer, 6 words per record)
   int atom;
   int yzk;          // by | bz << 12 | kx << 24
@@ -486,40 +577,48 @@ __device__ __forceinline__ int reserve_slot(bool keep, int* counter) {
   return base + __popcll(m & ((1ull << lane) - 1ull));
 }
 
-// candidates examined per lane per round of phase 1 (independent loads in flight)
+// candidates examined per lane per round of phase 1 (independent loads in flight), and gather
+// records held ahead per lane
 #define PLANE_U 4
+#define GATHER_U 2
+
+// complex elements of one of the two transform buffers of a plane: (Ky + 1)/2 packed lines of
+// stride Kz | 1, or Ky rows of the Kz/2 + 1 half spectrum
+__host__ __device__ __forceinline__ int plane_buf(int Ky, int Kz) {
+  const int packed = ((Ky + 1) / 2) * (Kz | 1), half = Ky * (Kz / 2 + 1);
+  return packed > half ? packed : half;
+}
 
 // spread q*sqrt(ke) of every atom touching plane x0 into an LDS int64 plane (integer sums, so the
-// result is independent of the order of the atomics), then forward FFT along z and y; the
-// plane goes to cg[x0][y][z].  LDS: twiddles (Kz + Ky), two complex planes; the records
-// overlay the second plane and what follows it.
-__device__ void plane_fwd_body(const PlaneArgs& a, const FftPlan& plz, const FftPlan& ply,
+// result is independent of the order of the atomics), then forward FFT along z (two real rows per
+// complex line) and y; the half spectrum goes to cg[x0][y][kz], kz <= Kz/2.  LDS: twiddles
+// (Kz + Ky), then the int64 plane and the list of touching atoms, which two transform buffers overlay.
+__device__ __forceinline__ void plane_fwd_body(const PlaneArgs& a, const FftPlan& plz, const FftPlan& ply,
                                const float2* __restrict__ twz_g, const float2* __restrict__ twy_g,
                                const int* __restrict__ sorted_orig, const int* __restrict__ cell_start,
                                const double* __restrict__ pos_sorted, const float4* __restrict__ xq,
                                float2* __restrict__ cg, GatherRec* __restrict__ grec, int* __restrict__ grec_n,
-                               DevState* st, int x0, float2* lds, bool wave64 = true) {
-  __shared__ int nrec;
-  __shared__ int ngrec;
-  const int P = a.Ky * a.Kz;
-  // wave-level transforms on a padded plane (they need PLANE_THREADS lanes)
-  const bool p64 = wave64 && a.Ky == 64 && a.Kz == 64;
+                               DevState* st, int x0, float2* lds) {
+  __shared__ int ntouch;
+  const int S = plane_buf(a.Ky, a.Kz);
   float2* twz = lds;
   float2* twy = lds + a.Kz;
   float2* A = twy + a.Ky;
-  float2* Bf = A + (p64 ? 64 * PLANE64_LS : P);
+  float2* Bf = A + S;
+  const int ls = a.Kz | 1;  // row stride of the fixed-point plane and of the packed lines (odd: the
+                            // four rows of a stencil fall on distinct banks)
   long long* plane = (long long*)A;
-  SpreadRec* rec = (SpreadRec*)Bf;
+  int* list = (int*)(plane + a.Ky * ls);
   load_twiddles(twz, twz_g, a.Kz);
   load_twiddles(twy, twy_g, a.Ky);
-  for (int i = threadIdx.x; i < P; i += blockDim.x) plane[i] = 0;
-  if (threadIdx.x == 0) ngrec = 0;
+  for (int i = threadIdx.x; i < a.Ky * ls; i += blockDim.x) plane[i] = 0;
   GatherRec* gout = grec + (long long)x0 * a.rec_cap;
   int b0, e0, b1, e1;
   plane_ranges(a, cell_start, x0, &b0, &e0, &b1, &e1);
   const int len0 = e0 - b0, total = len0 + (e1 - b1);
+  int done = 0;  // records written by earlier rounds
   for (int w0 = 0; w0 < total; w0 += a.W) {
-    if (threadIdx.x == 0) nrec = 0;
+    if (threadIdx.x == 0) ntouch = 0;
     __syncthreads();
     const int wend = min(total, w0 + a.W);
     // uniform trip count so every lane reaches the ballots
@@ -530,93 +629,114 @@ __device__ void plane_fwd_body(const PlaneArgs& a, const FftPlan& plz, const Fft
       for (int u = 0; u < PLANE_U; ++u) {
         const int ci = c0 + u * blockDim.x + threadIdx.x;
         sl[u] = ci < wend ? (ci < len0 ? b0 + ci : b1 + (ci - len0)) : -1;
-        px[u] = sl[u] >= 0 ? pos_sorted[3 * sl[u]] : 0.0;
+        px[u] = pos_sorted[3 * max(sl[u], 0)];
       }
 #pragma unroll
       for (int u = 0; u < PLANE_U; ++u) {
-        bool keep = false, touch = false;
-        SpreadRec r;
-        GatherRec g;
-        if (sl[u] >= 0) {
-          int bx;
-          float wx;
-          frac_coord(px[u], a.iLx, a.Kx, &bx, &wx);
-          int kx = bx - x0;
-          kx += kx < 0 ? a.Kx : 0;
-          if (kx <= 3) {
-            const int s = sl[u];
-            const float q = xq[s].w;
-            int by, bz;
-            frac_coord(pos_sorted[3 * s + 1], a.iLy, a.Ky, &by, &r.wy);
-            frac_coord(pos_sorted[3 * s + 2], a.iLz, a.Kz, &bz, &r.wz);
-            r.yz = by | (bz << 12);
-            r.qx = q * bsp4(wx, kx);
-            keep = q != 0.f;
-            // the same atom's record for the gather of this plane (zero charges included: the
-            // gather writes their slot, so every atom owns exactly four)
-            g.atom = sorted_orig[s];
-            g.yzk = by | (bz << 12) | (kx << 24);
-            g.wx = wx;
-            g.wy = r.wy;
-            g.wz = r.wz;
-            g.q = q;
-            touch = true;
-          }
-        }
-        const int slot = reserve_slot(keep, &nrec);
-        if (keep) rec[slot] = r;
-        const int gslot = reserve_slot(touch, &ngrec);
-        if (touch && gslot < a.rec_cap) gout[gslot] = g;
+        int bx;
+        float wx;
+        frac_coord(px[u], a.iLx, a.Kx, &bx, &wx);
+        int kx = bx - x0;
+        kx += kx < 0 ? a.Kx : 0;
+        const bool touch = sl[u] >= 0 && kx <= 3;
+        const int slot = reserve_slot(touch, &ntouch);
+        if (touch) list[slot] = sl[u];
       }
     }
     __syncthreads();
-    // four lanes per record, one per ky, each adding its 4 z points
-    const int nr = nrec;
-    for (int e = threadIdx.x; e < nr * 4; e += blockDim.x) {
-      const SpreadRec r = rec[e >> 2];
-      const int ky = e & 3;
-      int gy = (r.yz & 4095) - ky;
-      gy += gy < 0 ? a.Ky : 0;
-      const float qxy = r.qx * bsp4(r.wy, ky);
-      const float w = r.wz, w2 = w * w, w3 = w2 * w, om = 1.f - w;
-      const float tz[4] = {w3 * (1.f / 6.f), (-3.f * w3 + 3.f * w2 + 3.f * w + 1.f) * (1.f / 6.f),
-                           (3.f * w3 - 6.f * w2 + 4.f) * (1.f / 6.f), om * om * om * (1.f / 6.f)};
-      const int bz = r.yz >> 12;
-      long long* row = plane + gy * a.Kz;
+    const int nt = ntouch;
+    for (int e = threadIdx.x; e < nt; e += blockDim.x) {
+      const int s = list[e];
+      const double x = pos_sorted[3 * s], y = pos_sorted[3 * s + 1], z = pos_sorted[3 * s + 2];
+      const float q = xq[s].w;
+      GatherRec g;
+      g.atom = sorted_orig[s];
+      int bx, by, bz;
+      frac_coord(x, a.iLx, a.Kx, &bx, &g.wx);
+      frac_coord(y, a.iLy, a.Ky, &by, &g.wy);
+      frac_coord(z, a.iLz, a.Kz, &bz, &g.wz);
+      int kx = bx - x0;
+      kx += kx < 0 ? a.Kx : 0;
+      g.yzk = by | (bz << 12) | (kx << 24);
+      g.q = q;
+      // the gather's record (zero charges included: the gather writes their slot, so every atom
+      // owns exactly four)
+      if (done + e < a.rec_cap) gout[done + e] = g;
+      if (q == 0.f) continue;
+      float ty[4], tz[4];
+      bspline4(g.wy, ty, nullptr);
+      bspline4(g.wz, tz, nullptr);
+      const float qx = q * bsp4(g.wx, kx);
+      int gz[4];
 #pragma unroll
-      for (int kz = 0; kz < 4; ++kz) {
-        int gz = bz - kz;
-        gz += gz < 0 ? a.Kz : 0;
-        atomicAdd((unsigned long long*)&row[gz], (unsigned long long)to_fix_f(qxy * tz[kz]));
+      for (int k = 0; k < 4; ++k) gz[k] = bz - k + (bz < k ? a.Kz : 0);
+#pragma unroll
+      for (int ky = 0; ky < 4; ++ky) {
+        long long* row = plane + (by - ky + (by < ky ? a.Ky : 0)) * ls;
+        const float qxy = qx * ty[ky];
+#pragma unroll
+        for (int kz = 0; kz < 4; ++kz)
+          atomicAdd((unsigned long long*)&row[gz[kz]], (unsigned long long)to_fix_f(qxy * tz[kz]));
       }
     }
+    done += nt;
     __syncthreads();
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    grec_n[x0] = min(ngrec, a.rec_cap);
-    if (ngrec > a.rec_cap) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
+    grec_n[x0] = min(done, a.rec_cap);
+    if (done > a.rec_cap) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
   }
-  if (p64) {
-    float2* out = cg + (long long)x0 * P;
-    for (int i = threadIdx.x; i < P; i += blockDim.x)
-      Bf[(i >> 6) * PLANE64_LS + (i & 63)] = make_float2((float)((double)plane[i] * kFixInv), 0.f);
+  // Rows 2m and 2m + 1 become the real and imaginary part of packed line m (stride Kz | 1). The
+  // packed lines overlay the fixed-point plane: every value is in registers before the first
+  // store (pairs * Kz <= PLANE_REG * lanes, plane_lanes_ok).
+  const int pairs = (a.Ky + 1) >> 1, nz = a.Kz / 2 + 1;
+  {
+    float2 v[PLANE_REG];
+    const float iKz = 1.f / (float)a.Kz;
+#pragma unroll
+    for (int q = 0; q < PLANE_REG; ++q) {
+      const int idx = threadIdx.x + q * blockDim.x;
+      if (idx < pairs * a.Kz) {
+        const int m = (int)(((float)idx + 0.5f) * iKz), k = idx - m * a.Kz;
+        const long long lo = plane[2 * m * ls + k], hi = 2 * m + 1 < a.Ky ? plane[(2 * m + 1) * ls + k] : 0;
+        v[q] = make_float2((float)((double)lo * kFixInv), (float)((double)hi * kFixInv));
+      }
+    }
     __syncthreads();
-    plane64_lines<-1>(Bf, A, true, twz);   // z lines (rows) -> A
-    __syncthreads();
-    plane64_lines<-1>(A, Bf, false, twy);  // y lines (columns) -> Bf
-    __syncthreads();
-    for (int i = threadIdx.x; i < P; i += blockDim.x) out[i] = Bf[(i >> 6) * PLANE64_LS + (i & 63)];
-    return;
+#pragma unroll
+    for (int q = 0; q < PLANE_REG; ++q) {
+      const int idx = threadIdx.x + q * blockDim.x;
+      if (idx < pairs * a.Kz) {
+        const int m = (int)(((float)idx + 0.5f) * iKz);
+        A[m * ls + idx - m * a.Kz] = v[q];
+      }
+    }
   }
-  // in place: lane i reads int64 element i and writes complex element i (same 8 bytes)
-  for (int i = threadIdx.x; i < P; i += blockDim.x) A[i] = make_float2((float)((double)plane[i] * kFixInv), 0.f);
   __syncthreads();
-  float2* r1 = lds_fft<-1>(A, Bf, plz, a.Ky, twz);                // z lines: contiguous
-  float2* o1 = (r1 == A) ? Bf : A;
-  float2* r2 = lds_fft<-1>(r1, o1, ply, a.Kz, twy, 1, a.Kz);      // y lines: stride Kz
-  float2* out = cg + (long long)x0 * P;
-  for (int i = threadIdx.x; i < P; i += blockDim.x) out[i] = r2[i];
+  float2* r = A;
+  float2* o = Bf;
+  const float inz = 1.f / (float)nz;
+#pragma unroll 1
+  for (int axis = 0; axis < 2; ++axis) {
+    float2* f = lds_fft(r, o, axis ? ply : plz, axis ? nz : pairs, axis ? twy : twz, axis ? 1 : ls, axis ? nz : 1, -1.f);
+    o = f == r ? o : r;
+    r = f;
+    if (axis) break;
+    // separate the two rows' spectra: X_2m = (Z_k + conj Z_-k)/2, X_2m+1 = (Z_k - conj Z_-k)/2i
+    for (int idx = threadIdx.x; idx < pairs * nz; idx += blockDim.x) {
+      const int m = (int)(((float)idx + 0.5f) * inz), k = idx - m * nz;
+      const float2 p = r[m * ls + k], q = r[m * ls + (k ? a.Kz - k : 0)];
+      o[2 * m * nz + k] = make_float2(0.5f * (p.x + q.x), 0.5f * (p.y - q.y));
+      if (2 * m + 1 < a.Ky) o[(2 * m + 1) * nz + k] = make_float2(0.5f * (p.y + q.y), 0.5f * (q.x - p.x));
+    }
+    __syncthreads();
+    float2* h = o;
+    o = r;
+    r = h;
+  }
+  float2* out = cg + (long long)x0 * (a.Ky * nz);
+  for (int i = threadIdx.x; i < a.Ky * nz; i += blockDim.x) out[i] = r[i];
 }
 
 __global__ __launch_bounds__(PLANE_THREADS) void k_pme_plane_fwd(
@@ -632,107 +752,111 @@ __global__ __launch_bounds__(PLANE_THREADS) void k_pme_plane_fwd(
 // inverse FFT along y and z of plane x0, then for every atom touching the plane its share of
 // the reciprocal force, -q (dtheta_x theta_y theta_z, ...) . conv over this plane's 4x4 (y,z)
 // stencil, written to fpart[kx][3*atom + d] (each slot once per evaluation).
-// LDS: twiddles, real part of the convolved plane (floats), two complex planes that the
-// records overlay after the transforms.
-__device__ void plane_gather_body(const PlaneArgs& a, const FftPlan& plz, const FftPlan& ply,
+// LDS: twiddles and two transform buffers (plane_buf); the convolved plane is left in packed lines.
+__device__ __forceinline__ void plane_gather_body(const PlaneArgs& a, const FftPlan& plz, const FftPlan& ply,
                                   const float2* __restrict__ twz_g, const float2* __restrict__ twy_g,
                                   const int* __restrict__ sorted_orig, const int* __restrict__ cell_start,
                                   const double* __restrict__ pos_sorted, const float4* __restrict__ xq,
                                   const float2* __restrict__ cg, const GatherRec* __restrict__ grec,
                                   const int* __restrict__ grec_n, double* __restrict__ fpart, DevState* st, int x0,
-                                  float2* lds, bool wave64 = true) {
-  __shared__ int bcount;
-  const int P = a.Ky * a.Kz;
-  // wave-level transforms on a padded plane (they need PLANE_THREADS lanes)
-  const bool p64 = wave64 && a.Ky == 64 && a.Kz == 64;
+                                  float2* lds) {
+  const int S = plane_buf(a.Ky, a.Kz);
+  const int pairs = (a.Ky + 1) >> 1, ls = a.Kz | 1, nz = a.Kz / 2 + 1;
   float2* twz = lds;
   float2* twy = lds + a.Kz;
-  float* convr = (float*)(twy + a.Ky);
-  float2* A = (float2*)(convr + P + (P & 1));
-  float2* Bf = A + (p64 ? 64 * PLANE64_LS : P);
+  float2* A = twy + a.Ky;
+  float2* Bf = A + S;
   load_twiddles(twz, twz_g, a.Kz);
   load_twiddles(twy, twy_g, a.Ky);
-  const float2* in = cg + (long long)x0 * P;
-  if (p64) {
-    for (int i = threadIdx.x; i < P; i += blockDim.x) A[(i >> 6) * PLANE64_LS + (i & 63)] = in[i];
-    __syncthreads();
-    plane64_lines<1>(A, Bf, false, twy);  // y lines (columns) -> Bf
-    __syncthreads();
-    plane64_lines<1>(Bf, A, true, twz);   // z lines (rows) -> A
-    __syncthreads();
-    for (int i = threadIdx.x; i < P; i += blockDim.x) convr[i] = A[(i >> 6) * PLANE64_LS + (i & 63)].x;
-  } else {
-    for (int i = threadIdx.x; i < P; i += blockDim.x) A[i] = in[i];
-    __syncthreads();
-    float2* r1 = lds_fft<1>(A, Bf, ply, a.Kz, twy, 1, a.Kz);        // y lines first (reverse order)
-    float2* o1 = (r1 == A) ? Bf : A;
-    float2* r2 = lds_fft<1>(r1, o1, plz, a.Ky, twz);                // z lines
-    for (int i = threadIdx.x; i < P; i += blockDim.x) convr[i] = r2[i].x;
-  }
-  const long long n3 = 3LL * a.n;
-  // the records of the atoms touching this plane, written by the forward kernel
+  // the records of the atoms touching this plane, written by the forward kernel; each lane's first
+  // ones are loaded with the grid, the others GATHER_U at a time ahead of their use
   const int nr = grec_n[x0];
   const GatherRec* gin = grec + (long long)x0 * a.rec_cap;
-  __syncthreads();  // convr complete
-  // four lanes per record (one per ky, 4 z points each); nr * 4 and blockDim.x are multiples
-  // of 4, so the four lanes of a record stay together through the reduction. Zero charges give
-  // zero forces through the same arithmetic (their slot is still written).
-  for (int e = threadIdx.x; e < nr * 4; e += blockDim.x) {
-    const GatherRec r = gin[e >> 2];
-    const int ky = e & 3;
-    int gy = (r.yzk & 4095) - ky;
-    gy += gy < 0 ? a.Ky : 0;
-    const float ty = bsp4(r.wy, ky), dy = dbsp4(r.wy, ky);
-    const float w = r.wz, w2 = w * w, w3 = w2 * w, om = 1.f - w;
-    const float tz[4] = {w3 * (1.f / 6.f), (-3.f * w3 + 3.f * w2 + 3.f * w + 1.f) * (1.f / 6.f),
-                         (3.f * w3 - 6.f * w2 + 4.f) * (1.f / 6.f), om * om * om * (1.f / 6.f)};
-    const float dz[4] = {0.5f * w2, 0.5f * (-3.f * w2 + 2.f * w + 1.f), 0.5f * (3.f * w2 - 4.f * w),
-                         -0.5f * om * om};
-    const int bz = (r.yzk >> 12) & 4095;
-    const float* row = convr + gy * a.Kz;
-    float c = 0.f, cz = 0.f;
+  GatherRec rec[GATHER_U];
+  auto fetch = [&](int e0) {
 #pragma unroll
-    for (int kz = 0; kz < 4; ++kz) {
-      int gz = bz - kz;
-      gz += gz < 0 ? a.Kz : 0;
-      const float cv = row[gz];
-      c += tz[kz] * cv;
-      cz += dz[kz] * cv;
+    for (int u = 0; u < GATHER_U; ++u) {
+      const int e = e0 + u * (int)blockDim.x;
+      if (e < nr) rec[u] = gin[e];
     }
-    float sx = ty * c, sy = dy * c, sz = ty * cz;
-#pragma unroll
-    for (int off = 2; off > 0; off >>= 1) {
-      sx += __shfl_xor(sx, off, 64);
-      sy += __shfl_xor(sy, off, 64);
-      sz += __shfl_xor(sz, off, 64);
-    }
-    if (ky == 0) {
-      const int kx = r.yzk >> 24;
-      const float tx = bsp4(r.wx, kx), dx = dbsp4(r.wx, kx);
-      double* dst = fpart + kx * n3 + 3LL * r.atom;
-      if (r.q == 0.f) {
-        dst[0] = dst[1] = dst[2] = 0.0;
-      } else {
-        dst[0] = -(double)r.q * (double)(dx * sx) * (a.Kx / a.Lx);
-        dst[1] = -(double)r.q * (double)(tx * sy) * (a.Ky / a.Ly);
-        dst[2] = -(double)r.q * (double)(tx * sz) * (a.Kz / a.Lz);
-      }
-    }
-  }
-  if (threadIdx.x == 0) bcount = nr;
-  // every atom owns exactly one slot per kx: the grid-wide count must be 4 n. The last block
-  // to finish checks it and re-arms the counters for the next evaluation.
+  };
+  fetch(threadIdx.x);
+  const float2* in = cg + (long long)x0 * (a.Ky * nz);
+  for (int i = threadIdx.x; i < a.Ky * nz; i += blockDim.x) A[i] = in[i];
   __syncthreads();
+  float2* r = A;
+  float2* o = Bf;
+  const float inz = 1.f / (float)nz;
+#pragma unroll 1
+  for (int axis = 0; axis < 2; ++axis) {
+    float2* f = lds_fft(r, o, axis ? plz : ply, axis ? pairs : nz, axis ? twz : twy, axis ? ls : 1, axis ? 1 : nz, 1.f);
+    o = f == r ? o : r;
+    r = f;
+    if (axis) break;
+    // rows 2m and 2m + 1 again as one packed line, Z = X_2m + i X_2m+1 over the whole period
+    for (int idx = threadIdx.x; idx < pairs * nz; idx += blockDim.x) {
+      const int m = (int)(((float)idx + 0.5f) * inz), k = idx - m * nz;
+      const float2 p = r[2 * m * nz + k], q = 2 * m + 1 < a.Ky ? r[(2 * m + 1) * nz + k] : make_float2(0.f, 0.f);
+      o[m * ls + k] = make_float2(p.x - q.y, p.y + q.x);
+      if (k > 0 && 2 * k != a.Kz) o[m * ls + a.Kz - k] = make_float2(p.x + q.y, q.x - p.y);
+    }
+    __syncthreads();
+    float2* h = o;
+    o = r;
+    r = h;
+  }
+  const float* convr = (const float*)r;  // real parts: row 2m, imaginary parts: row 2m + 1
+  const long long n3 = 3LL * a.n;
+  // one lane per record; zero charges give zero forces (their slot is still written)
+  auto share = [&](const GatherRec& r) {
+    const int by = r.yzk & 4095, bz = (r.yzk >> 12) & 4095, kx = r.yzk >> 24;
+    float ty[4], dy[4], tz[4], dz[4];
+    bspline4(r.wy, ty, dy);
+    bspline4(r.wz, tz, dz);
+    int gz[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) gz[k] = 2 * (bz - k + (bz < k ? a.Kz : 0));
+    float sx = 0.f, sy = 0.f, sz = 0.f;
+#pragma unroll
+    for (int ky = 0; ky < 4; ++ky) {
+      const int gy = by - ky + (by < ky ? a.Ky : 0);
+      const float* row = convr + 2 * (gy >> 1) * ls + (gy & 1);
+      float c = 0.f, cz = 0.f;
+#pragma unroll
+      for (int kz = 0; kz < 4; ++kz) {
+        const float cv = row[gz[kz]];
+        c += tz[kz] * cv;
+        cz += dz[kz] * cv;
+      }
+      sx += ty[ky] * c;
+      sy += dy[ky] * c;
+      sz += ty[ky] * cz;
+    }
+    const float tx = bsp4(r.wx, kx), dx = dbsp4(r.wx, kx);
+    double* dst = fpart + kx * n3 + 3LL * r.atom;
+    const double q = -(double)r.q;
+    dst[0] = r.q == 0.f ? 0.0 : q * (double)(dx * sx) * a.gx;
+    dst[1] = r.q == 0.f ? 0.0 : q * (double)(tx * sy) * a.gy;
+    dst[2] = r.q == 0.f ? 0.0 : q * (double)(tx * sz) * a.gz;
+  };
+  for (int e0 = threadIdx.x; e0 < nr; e0 += GATHER_U * blockDim.x) {
+    GatherRec now[GATHER_U];
+#pragma unroll
+    for (int u = 0; u < GATHER_U; ++u) now[u] = rec[u];
+    fetch(e0 + GATHER_U * blockDim.x);
+#pragma unroll
+    for (int u = 0; u < GATHER_U; ++u)
+      if (e0 + u * (int)blockDim.x < nr) share(now[u]);
+  }
+  // every atom owns exactly one slot per kx: the grid-wide count must be 4 n. One 64-bit add per
+  // workgroup carries its slots (40 bits) and its arrival (above); the last of the Kx plane
+  // workgroups (launches may hold others) checks the total and re-arms the counter.
   if (threadIdx.x == 0) {
-    atomicAdd(&st->pme_slots, bcount);
-    __threadfence();
-    const unsigned t = atomicAdd(&st->pme_ticket, 1u);
-    if (t == (unsigned)a.Kx - 1) {  // the last of the Kx plane workgroups (launches may hold others)
-      __threadfence();
-      const int tot = atomicAdd(&st->pme_slots, 0);
-      if (tot != 4 * a.n) atomicOr(&st->flags, MDX_FLAG_PME_COVERAGE);
-      atomicExch(&st->pme_slots, 0);
-      atomicExch(&st->pme_ticket, 0u);
+    const unsigned long long mine = (1ull << 40) + (unsigned)nr;
+    const unsigned long long all = atomicAdd(&st->pme_count, mine) + mine;
+    if (all >> 40 == (unsigned)a.Kx) {
+      if ((all & ((1ull << 40) - 1ull)) != 4ull * (unsigned)a.n) atomicOr(&st->flags, MDX_FLAG_PME_COVERAGE);
+      atomicExch(&st->pme_count, 0ull);
     }
   }
 }
@@ -783,7 +907,7 @@ __device__ void grid_barrier(DevState* st) {
 // x0 back and gathers its forces. The blocks keep their compute units for the whole
 // evaluation, so kernels running concurrently on other streams cannot delay the later phases.
 __global__ __launch_bounds__(PLANE_THREADS) void k_pme_fused(
-    PlaneArgs a, FftPlan plz, FftPlan ply, FftPlan plx, FftLines lnx, const float2* __restrict__ twz_g,
+    PlaneArgs a, FftPlan plz, FftPlan ply, XPass xp, const float2* __restrict__ twz_g,
     const float2* __restrict__ twy_g, const float2* __restrict__ twx_g, const int* __restrict__ sorted_orig,
     const int* __restrict__ cell_start, const double* __restrict__ pos_sorted, const float4* __restrict__ xq,
     float2* __restrict__ cg, const float* __restrict__ bc, long long* __restrict__ eslot,
@@ -792,9 +916,9 @@ __global__ __launch_bounds__(PLANE_THREADS) void k_pme_fused(
   plane_fwd_body(a, plz, ply, twz_g, twy_g, sorted_orig, cell_start, pos_sorted, xq, cg, grec, grec_n, st,
                  blockIdx.x, lds);
   grid_barrier(st);
-  const int nchunks = (lnx.nlines + lnx.B - 1) / lnx.B;
+  const int nchunks = (xp.nl + xp.B - 1) / xp.B;
   for (int ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-    fft_axis_body<-1, 3>(plx, lnx, twx_g, cg, nullptr, nullptr, bc, eslot, ch * lnx.B, lds);
+    fft_x_body(xp, twx_g, cg, bc, eslot, ch * xp.B, lds);
     __syncthreads();
   }
   grid_barrier(st);
@@ -811,8 +935,8 @@ __global__ __launch_bounds__(PLANE_THREADS) void k_pme_fused(
 // path and its fork and join.
 struct PhaseArgs {
   PlaneArgs a;
-  FftPlan plz, ply, plx;
-  FftLines lnx;
+  FftPlan plz, ply;
+  XPass xp;
   const float2 *twz, *twy, *twx;
   const int* sorted_orig;
   const int* cell_start;
@@ -837,7 +961,7 @@ __global__ __launch_bounds__(PLANE_THREADS) void k_force_phase(int phase, int np
       plane_fwd_body(p.a, p.plz, p.ply, p.twz, p.twy, p.sorted_orig, p.cell_start, p.pos_sorted, p.xq, p.cg, p.grec,
                      p.grec_n, p.st, b, lds);
     else if (phase == 1)
-      fft_axis_body<-1, 3>(p.plx, p.lnx, p.twx, p.cg, nullptr, nullptr, p.bc, p.eslot, b * p.lnx.B, lds);
+      fft_x_body(p.xp, p.twx, p.cg, p.bc, p.eslot, b * p.xp.B, lds);
     else
       plane_gather_body(p.a, p.plz, p.ply, p.twz, p.twy, p.sorted_orig, p.cell_start, p.pos_sorted, p.xq, p.cg,
                         p.grec, p.grec_n, p.fpart, p.st, b, lds);
@@ -858,34 +982,50 @@ static PhaseKernel phase_kernel(bool energy, int G) {
   return energy ? k_force_phase<true, 32> : k_force_phase<false, 32>;
 }
 
-// LDS bytes of the two plane kernels (the forward one for a record window of W candidates)
-// (64 x 64 planes are held padded to 64 x PLANE64_LS complex values)
+// LDS bytes of the two plane kernels (the forward one for a window of W candidates)
 static inline size_t plane_fwd_lds(int Ky, int Kz, int W) {
-  const size_t P = (size_t)Ky * Kz;
-  const size_t Pp = (Ky == 64 && Kz == 64) ? 64 * PLANE64_LS : P;
-  return (size_t)(Ky + Kz) * 8 + std::max(2 * Pp * 8, Pp * 8 + (size_t)W * sizeof(SpreadRec));
+  return (size_t)(Ky + Kz) * 8 +
+         std::max(2 * (size_t)plane_buf(Ky, Kz) * 8, (size_t)Ky * (Kz | 1) * 8 + (size_t)W * sizeof(int));
 }
 static inline size_t plane_gather_lds(int Ky, int Kz) {
-  const size_t P = (size_t)Ky * Kz;
-  const size_t Pp = (Ky == 64 && Kz == 64) ? 64 * PLANE64_LS : P;
-  return (size_t)(Ky + Kz) * 8 + (P + (P & 1)) * 4 + 2 * Pp * 8;
+  return (size_t)(Ky + Kz) * 8 + 2 * (size_t)plane_buf(Ky, Kz) * 8;
 }
+// the forward kernel holds a plane's packed values in PLANE_REG registers a lane
+static inline bool plane_lanes_ok(int Ky, int Kz, int threads) {
+  return (long long)((Ky + 1) / 2) * Kz <= (long long)PLANE_REG * threads;
+}
+static inline size_t x_pass_lds(int K, int B) { return (2 * (size_t)(B | 1) * K + K) * sizeof(float2); }
 
 // ---------------------------------------------------------------- host
+// K as a product of the fewest radices (every pass is a round trip through LDS and a barrier), the
+// largest one as small as possible among those (fewer registers, more butterflies)
+static bool split_radices(int k, int passes, int largest, int* out, int* n) {
+  static const int radices[] = {2, 3, 4, 5, 6, 8, 9, 10, 12, 16};
+  if (passes == 0) return k == 1;
+  for (int q = 9; q >= 0; --q) {
+    const int r = radices[q];
+    if (r > largest || k % r) continue;
+    const int m = *n;
+    out[(*n)++] = r;
+    if (split_radices(k / r, passes - 1, r, out, n)) return true;
+    *n = m;
+  }
+  return false;
+}
 static int factorize(int K, FftPlan* pl) {
+  static const int radices[] = {2, 3, 4, 5, 6, 8, 9, 10, 12, 16};
   pl->K = K;
   pl->nrad = 0;
   pl->code = 0;
-  int k = K;
-  auto push = [&](unsigned long long r) {
-    if (pl->nrad < MAX_RADICES) pl->code |= r << (4 * pl->nrad);
-    pl->nrad++;
-  };
-  while (k % 4 == 0) { push(4); k /= 4; }
-  while (k % 2 == 0) { push(2); k /= 2; }
-  while (k % 3 == 0) { push(3); k /= 3; }
-  while (k % 5 == 0) { push(5); k /= 5; }
-  return (k == 1 && pl->nrad <= MAX_RADICES) ? 0 : -1;
+  for (int passes = 1; passes <= MAX_RADICES; ++passes)
+    for (int largest : radices) {
+      int r[MAX_RADICES], n = 0;
+      if (!split_radices(K, passes, largest, r, &n)) continue;
+      for (int q = 0; q < n; ++q) pl->code |= (unsigned long long)r[q] << (8 * q);
+      pl->nrad = n;
+      return 0;
+    }
+  return -1;
 }
 
 // |b(m)|^-2 of Essmann eq. 4.4 for order 4: M4(1)=1/6, M4(2)=2/3, M4(3)=1/6
@@ -923,7 +1063,7 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
   size_t G = (size_t)c->K[0] * c->K[1] * c->K[2];
   int rc;
   if ((rc = c->qfix.ensure(G)) || (rc = c->cgrid.ensure(G)) || (rc = c->conv.ensure(G)) || (rc = c->bc.ensure(G)) ||
-      (rc = c->fpart.ensure(12 * (size_t)c->n)))
+      (rc = c->bch.ensure((size_t)c->K[0] * c->K[1] * (c->K[2] / 2 + 1))) || (rc = c->fpart.ensure(12 * (size_t)c->n)))
     return rc;
   MDX_HIP(hipMemset(c->qfix.p, 0, G * sizeof(long long)));
   // influence function B(m) C(m), C(0) = 0
@@ -949,6 +1089,11 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
     }
   }
   MDX_HIP(hipMemcpy(c->bc.p, h_bc.data(), G * sizeof(float), hipMemcpyHostToDevice));
+  const int nz = c->K[2] / 2 + 1;  // the plane path's half spectrum
+  std::vector<float> h_bch((size_t)c->K[0] * c->K[1] * nz);
+  for (size_t row = 0; row < (size_t)c->K[0] * c->K[1]; ++row)
+    std::memcpy(&h_bch[row * nz], &h_bc[row * c->K[2]], nz * sizeof(float));
+  MDX_HIP(hipMemcpy(c->bch.p, h_bch.data(), h_bch.size() * sizeof(float), hipMemcpyHostToDevice));
   int Kmax = std::max(c->K[0], std::max(c->K[1], c->K[2]));
   if ((rc = c->twiddle.ensure(3 * (size_t)Kmax))) return rc;
   std::vector<float2> tw(3 * (size_t)Kmax);
@@ -958,16 +1103,17 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
       tw[(size_t)d * Kmax + k] = make_float2((float)cos(a), (float)sin(a));
     }
   MDX_HIP(hipMemcpy(c->twiddle.p, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice));
-  // the plane kernels hold twiddles, two complex Ky x Kz planes and a window of atom records
-  // in LDS; the window is as large as the device allows (at most 8192 candidates)
+  // the plane kernels hold twiddles, the fixed-point plane and a window of touching atoms (forward),
+  // or two half-spectrum planes (gather) in LDS: up to 128 x 128 points on 160 KB. The window is
+  // as large as the device allows (at most 8192 candidates)
   int lds_max = 0;
   MDX_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
   const size_t budget = lds_max > 1024 ? (size_t)lds_max - 1024 : 0;  // static LDS of the kernels
   c->pme_wf = 0;
   for (int W = 8192; W >= PLANE_THREADS; W -= PLANE_THREADS)
     if (!c->pme_wf && plane_fwd_lds(c->K[1], c->K[2], W) <= budget) c->pme_wf = W;
-  c->pme_planes = c->pme_wf > 0 && plane_gather_lds(c->K[1], c->K[2]) <= budget && c->K[1] < 4096 &&
-                  c->K[2] < 4096;
+  c->pme_planes = c->pme_wf > 0 && plane_gather_lds(c->K[1], c->K[2]) <= budget &&
+                  plane_lanes_ok(c->K[1], c->K[2], PLANE_THREADS) && c->K[1] < 4096 && c->K[2] < 4096;
   // gather records: each atom touches 4 of the Kx planes; room for twice the mean plus slack
   c->pme_rec_cap = (int)std::min<long long>(c->n, 8LL * c->n / c->K[0] + 4096);
   if ((rc = c->pme_grec.ensure((size_t)c->K[0] * c->pme_rec_cap * 6)) || (rc = c->pme_grec_n.ensure(c->K[0])))
@@ -977,6 +1123,7 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
     MDX_HIP(hipFuncSetAttribute((const void*)k_pme_plane_inv_gather, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)budget));
     MDX_HIP(hipFuncSetAttribute((const void*)k_pme_fused, hipFuncAttributeMaxDynamicSharedMemorySize, (int)budget));
+    MDX_HIP(hipFuncSetAttribute((const void*)k_fft_x, hipFuncAttributeMaxDynamicSharedMemorySize, (int)budget));
   }
   // one-launch kernel: Kx blocks that must all be resident together (one per compute unit);
   // the x-axis pass takes ceil(Ky Kz / Kx) pencils per block if the LDS allows
@@ -984,11 +1131,10 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
   MDX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
   c->pme_fused_B = 0;
   if (c->pme_planes && c->K[0] <= ncu) {
-    const int nl = c->K[1] * c->K[2];
+    const int nl = c->K[1] * nz;
     int B = (nl + c->K[0] - 1) / c->K[0];
-    const size_t ls = c->K[0] + 1;  // strided lines: padded LDS line stride
-    while (B > 1 && (2 * (size_t)B * ls + c->K[0]) * sizeof(float2) > budget) B = (B + 1) / 2;
-    const size_t lds_x = (2 * (size_t)B * ls + c->K[0]) * sizeof(float2);
+    while (B > 1 && x_pass_lds(c->K[0], B) > budget) B = (B + 1) / 2;
+    const size_t lds_x = x_pass_lds(c->K[0], B);
     c->pme_fused_B = lds_x <= budget ? B : 0;
     c->pme_fused_lds = std::max(lds_x, std::max(plane_fwd_lds(c->K[1], c->K[2], c->pme_wf),
                                                 plane_gather_lds(c->K[1], c->K[2])));
@@ -1006,7 +1152,7 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
     const size_t pb = (size_t)lds_max > st_max + 256 ? (size_t)lds_max - st_max - 256 : 0;
     for (int W = 8192; W >= PLANE_THREADS; W -= PLANE_THREADS)
       if (!c->pme_wf_phase && plane_fwd_lds(c->K[1], c->K[2], W) <= pb) c->pme_wf_phase = W;
-    const size_t lx = (2 * (size_t)c->pme_fused_B * (c->K[0] + 1) + c->K[0]) * sizeof(float2);
+    const size_t lx = x_pass_lds(c->K[0], c->pme_fused_B);
     if (plane_gather_lds(c->K[1], c->K[2]) > pb || lx > pb) c->pme_wf_phase = 0;
     if (c->pme_wf_phase)
       for (int e = 0; e < 2; ++e)
@@ -1058,8 +1204,18 @@ static void fft_axis_of(const mdx_ctx* c, int axis, FftPlan* plo, FftLines* lno,
     ln.B = std::min(16, Kz);
   }
   *two = c->twiddle.p + (size_t)axis * Kmax;
-  const size_t ls = ln.estride == 1 ? pl.K : pl.K + 1;
-  *ldso = (2 * (size_t)ln.B * ls + pl.K) * sizeof(float2);
+  *ldso = (2 * (size_t)ln.B * (pl.K | 1) + pl.K) * sizeof(float2);
+}
+
+// the plane path's x-axis pass, B lines per workgroup
+static XPass x_pass_of(const mdx_ctx* c, int B) {
+  XPass xp;
+  factorize(c->K[0], &xp.pl);
+  xp.nz = c->K[2] / 2 + 1;
+  xp.nl = c->K[1] * xp.nz;
+  xp.kz_even = c->K[2] % 2 == 0;
+  xp.B = B;
+  return xp;
 }
 
 static int fft_pass(mdx_ctx* c, int axis, int dir, int mode) {
@@ -1101,6 +1257,9 @@ static void plane_args_of(const mdx_ctx* c, PlaneArgs* out) {
   a.iLx = 1.0 / c->box[0];
   a.iLy = 1.0 / c->box[1];
   a.iLz = 1.0 / c->box[2];
+  a.gx = Kx / c->box[0];
+  a.gy = Ky / c->box[1];
+  a.gz = Kz / c->box[2];
   a.gnx = c->gn[0];
   a.gny = c->gn[1];
   a.gnz = c->gn[2];
@@ -1123,19 +1282,10 @@ static int pme_enqueue_planes(mdx_ctx* c, unsigned parts = 7u) {
   const float2* twy = c->twiddle.p + (size_t)Kmax;
   const float2* twz = c->twiddle.p + 2 * (size_t)Kmax;
   if (parts == 7u && c->pme_fused_B > 0 && c->pme_fused_on && !c->in_batch) {
-    FftPlan plx;
-    factorize(Kx, &plx);
-    FftLines ln;
-    ln.nlines = Ky * Kz;
-    ln.inner = ln.nlines;
-    ln.inner_stride = 1;
-    ln.outer_stride = 0;
-    ln.estride = Ky * Kz;
-    ln.B = c->pme_fused_B;
     a.W = c->pme_wf;
     k_pme_fused<<<Kx, PLANE_THREADS, c->pme_fused_lds, c->stream>>>(
-        a, plz, ply, plx, ln, twz, twy, c->twiddle.p, c->sorted_orig.p, c->cell_start.p, c->pos_sorted.p, c->xq.p,
-        c->cgrid.p, c->bc.p, c->efix.p + 2, grec, c->pme_grec_n.p, c->fpart.p, c->dstate.p);
+        a, plz, ply, x_pass_of(c, c->pme_fused_B), twz, twy, c->twiddle.p, c->sorted_orig.p, c->cell_start.p,
+        c->pos_sorted.p, c->xq.p, c->cgrid.p, c->bch.p, c->efix.p + 2, grec, c->pme_grec_n.p, c->fpart.p, c->dstate.p);
     MDX_LAUNCH_CHECK();
     return 0;
   }
@@ -1146,8 +1296,12 @@ static int pme_enqueue_planes(mdx_ctx* c, unsigned parts = 7u) {
         c->pme_grec_n.p, c->dstate.p);
     MDX_LAUNCH_CHECK();
   }
-  int rc;
-  if ((parts & 2u) && (rc = fft_pass(c, 0, -1, 3))) return rc;  // x forward, * B C, energy, x inverse
+  if (parts & 2u) {  // x forward, * B C, energy, x inverse
+    const XPass xp = x_pass_of(c, FFTX_B);
+    k_fft_x<<<div_up(xp.nl, xp.B), FFTX_THREADS, x_pass_lds(Kx, xp.B), c->stream>>>(xp, c->twiddle.p, c->cgrid.p,
+                                                                                   c->bch.p, c->efix.p + 2);
+    MDX_LAUNCH_CHECK();
+  }
   if (parts & 4u) {
     k_pme_plane_inv_gather<<<Kx, PLANE_THREADS, plane_gather_lds(Ky, Kz), c->stream>>>(
         a, plz, ply, twz, twy, c->sorted_orig.p, c->cell_start.p, c->pos_sorted.p, c->xq.p, c->cgrid.p, grec,
@@ -1176,33 +1330,12 @@ int mdx_force_phases_enqueue(mdx_ctx* c, bool energy, unsigned bonded_terms) {
   const int Kx = c->K[0], Ky = c->K[1], Kz = c->K[2];
   PhaseArgs p;
   PlaneArgs& a = p.a;
-  a.n = c->n;
-  a.Kx = Kx;
-  a.Ky = Ky;
-  a.Kz = Kz;
-  a.Lx = c->box[0];
-  a.Ly = c->box[1];
-  a.Lz = c->box[2];
-  a.iLx = 1.0 / c->box[0];
-  a.iLy = 1.0 / c->box[1];
-  a.iLz = 1.0 / c->box[2];
-  a.gnx = c->gn[0];
-  a.gny = c->gn[1];
-  a.gnz = c->gn[2];
-  a.wx = c->box[0] / c->gn[0];
-  a.margin = 0.5 * c->skin + 1e-6 * c->box[0] + 1e-9;
-  a.rec_cap = c->pme_rec_cap;
+  plane_args_of(c, &a);
   a.W = c->pme_wf_phase;
   MDX_CHECK(c->pme_grec.n >= (size_t)Kx * a.rec_cap * 6, MDX_ERR_INVALID, "PME configured for another system size");
   factorize(Kz, &p.plz);
   factorize(Ky, &p.ply);
-  factorize(Kx, &p.plx);
-  p.lnx.nlines = Ky * Kz;
-  p.lnx.inner = p.lnx.nlines;
-  p.lnx.inner_stride = 1;
-  p.lnx.outer_stride = 0;
-  p.lnx.estride = Ky * Kz;
-  p.lnx.B = c->pme_fused_B;
+  p.xp = x_pass_of(c, c->pme_fused_B);
   const int Kmax = std::max(Kx, std::max(Ky, Kz));
   p.twx = c->twiddle.p;
   p.twy = c->twiddle.p + (size_t)Kmax;
@@ -1212,7 +1345,7 @@ int mdx_force_phases_enqueue(mdx_ctx* c, bool energy, unsigned bonded_terms) {
   p.pos_sorted = c->pos_sorted.p;
   p.xq = c->xq.p;
   p.cg = c->cgrid.p;
-  p.bc = c->bc.p;
+  p.bc = c->bch.p;
   p.eslot = c->efix.p + 2;
   p.grec = (GatherRec*)c->pme_grec.p;
   p.grec_n = c->pme_grec_n.p;
@@ -1229,8 +1362,8 @@ int mdx_force_phases_enqueue(mdx_ctx* c, bool energy, unsigned bonded_terms) {
   const int n0 = std::min(nbt, (int)(c->phase_frac[0] * nbt + 0.5));
   const int n1 = std::min(nbt - n0, (int)(c->phase_frac[1] * nbt + 0.5));
   const int n2 = nbt - n0 - n1;
-  const int nx = (p.lnx.nlines + p.lnx.B - 1) / p.lnx.B;  // x-pass workgroups
-  const size_t lx = (2 * (size_t)p.lnx.B * (Kx + 1) + Kx) * sizeof(float2);
+  const int nx = div_up(p.xp.nl, p.xp.B);  // x-pass workgroups
+  const size_t lx = x_pass_lds(Kx, p.xp.B);
   PhaseKernel k = phase_kernel(energy, G);
   k<<<Kx + n0, PLANE_THREADS, plane_fwd_lds(Ky, Kz, a.W), c->stream>>>(0, Kx, 0, n0, p, na, P, ba);
   MDX_LAUNCH_CHECK();
@@ -1308,31 +1441,27 @@ struct PlaneCall {
   DevState* st;
 };
 struct FftCall {
-  FftPlan pl;
-  FftLines ln;
+  XPass xp;
   const float2* tw;
   float2* cg;
-  long long* qfix;
-  float* rout;
   const float* bc;
   long long* eslot;
 };
 
-// Batched plane kernels of BS lanes: PLANE_THREADS, or fewer when no replica has 64 x 64 planes
-// (which need all PLANE_THREADS lanes for their wave-level transforms).
+// Batched plane kernels of BS lanes: PLANE_THREADS, or fewer when every replica's planes are small.
 template <int BS>
 __global__ __launch_bounds__(BS) void k_pme_plane_fwd_batch(BatchMap map, const PlaneCall* __restrict__ calls) {
   extern __shared__ float2 lds[];
   int x0;
   const PlaneCall& p = calls[batch_replica(map, &x0)];
   plane_fwd_body(p.a, p.plz, p.ply, p.twz, p.twy, p.sorted_orig, p.cell_start, p.pos_sorted, p.xq, p.cg, p.grec,
-                 p.grec_n, p.st, x0, lds, BS == PLANE_THREADS);
+                 p.grec_n, p.st, x0, lds);
 }
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis_batch(BatchMap map, const FftCall* __restrict__ calls) {
+__global__ __launch_bounds__(FFTX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_fft_x_batch(BatchMap map, const FftCall* __restrict__ calls) {
   extern __shared__ float2 lds[];
   int ch;
   const FftCall& f = calls[batch_replica(map, &ch)];
-  fft_axis_body<-1, 3>(f.pl, f.ln, f.tw, f.cg, f.qfix, f.rout, f.bc, f.eslot, ch * f.ln.B, lds);
+  fft_x_body(f.xp, f.tw, f.cg, f.bc, f.eslot, ch * f.xp.B, lds);
 }
 template <int BS>
 __global__ __launch_bounds__(BS) void k_pme_plane_inv_gather_batch(BatchMap map, const PlaneCall* __restrict__ calls) {
@@ -1340,7 +1469,7 @@ __global__ __launch_bounds__(BS) void k_pme_plane_inv_gather_batch(BatchMap map,
   int x0;
   const PlaneCall& p = calls[batch_replica(map, &x0)];
   plane_gather_body(p.a, p.plz, p.ply, p.twz, p.twy, p.sorted_orig, p.cell_start, p.pos_sorted, p.xq, p.cg, p.grec,
-                    p.grec_n, p.fpart, p.st, x0, lds, BS == PLANE_THREADS);
+                    p.grec_n, p.fpart, p.st, x0, lds);
 }
 // Without 64 x 64 planes the batched forward kernel runs 256-lane workgroups with a window of
 // 1,024 candidates (more planes in flight: 109 vs 133 us over the 64 water replicas); the gather
@@ -1353,16 +1482,16 @@ int mdx_batch_prepare_pme(mdx_ctx* const* cs, int n, BatchKind* fwd, BatchKind* 
   std::vector<FftCall> fc;
   std::vector<int> bp, bf;
   size_t lf = 0, lx = 0, lg = 0;
-  bool any64 = false;
-  for (int r = 0; r < n; ++r) any64 |= cs[r]->K[1] == 64 && cs[r]->K[2] == 64;
-  const int fthreads = any64 ? PLANE_THREADS : PLANE_BATCH_SMALL;
+  bool small = true;
+  for (int r = 0; r < n; ++r) small &= plane_lanes_ok(cs[r]->K[1], cs[r]->K[2], PLANE_BATCH_SMALL);
+  const int fthreads = small ? PLANE_BATCH_SMALL : PLANE_THREADS;
   for (int r = 0; r < n; ++r) {
     mdx_ctx* c = cs[r];
     MDX_CHECK(c->pme_configured && c->pme_planes && c->nb_configured && c->has_charges, MDX_ERR_INVALID,
               "replica %d: batched steps need the PME plane path", r);
     PlaneCall p;
     plane_args_of(c, &p.a);
-    if (!any64) p.a.W = std::min(p.a.W, PLANE_BATCH_W);
+    if (small) p.a.W = std::min(p.a.W, PLANE_BATCH_W);
     MDX_CHECK(c->pme_grec.n >= (size_t)c->K[0] * p.a.rec_cap * 6 && c->fpart.p && c->fpart.n >= 12 * (size_t)c->n,
               MDX_ERR_INVALID, "replica %d: PME configured for another system size", r);
     factorize(c->K[2], &p.plz);
@@ -1384,21 +1513,19 @@ int mdx_batch_prepare_pme(mdx_ctx* const* cs, int n, BatchKind* fwd, BatchKind* 
     lf = std::max(lf, plane_fwd_lds(c->K[1], c->K[2], p.a.W));
     lg = std::max(lg, plane_gather_lds(c->K[1], c->K[2]));
     FftCall f;
-    size_t l;
-    fft_axis_of(c, 0, &f.pl, &f.ln, &f.tw, &l);
+    f.xp = x_pass_of(c, FFTX_B);
+    f.tw = c->twiddle.p;
     f.cg = c->cgrid.p;
-    f.qfix = c->qfix.p;
-    f.rout = c->conv.p;
-    f.bc = c->bc.p;
+    f.bc = c->bch.p;
     f.eslot = c->efix.p + 2;
     fc.push_back(f);
-    bf.push_back(div_up(f.ln.nlines, f.ln.B));
-    lx = std::max(lx, l);
+    bf.push_back(div_up(f.xp.nl, f.xp.B));
+    lx = std::max(lx, x_pass_lds(c->K[0], FFTX_B));
   }
   const void* kf = fthreads == PLANE_THREADS ? (const void*)k_pme_plane_fwd_batch<PLANE_THREADS>
                                              : (const void*)k_pme_plane_fwd_batch<PLANE_BATCH_SMALL>;
   MDX_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf));
-  MDX_HIP(hipFuncSetAttribute((const void*)k_fft_axis_batch, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lx));
+  MDX_HIP(hipFuncSetAttribute((const void*)k_fft_x_batch, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lx));
   MDX_HIP(hipFuncSetAttribute((const void*)k_pme_plane_inv_gather_batch<PLANE_THREADS>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lg));
   int rc;
@@ -1406,7 +1533,7 @@ int mdx_batch_prepare_pme(mdx_ctx* const* cs, int n, BatchKind* fwd, BatchKind* 
       (rc = batch_kind_upload(gat, pc, bp, lg)))
     return rc;
   fwd->threads = fthreads;
-  fft->threads = FFT_THREADS;
+  fft->threads = FFTX_THREADS;
   gat->threads = PLANE_THREADS;
   return 0;
 }
@@ -1423,7 +1550,7 @@ int mdx_batch_launch_pme(const BatchKind& fwd, const BatchKind& fft, const Batch
     MDX_LAUNCH_CHECK();
   }
   if (parts & 2u) {
-    k_fft_axis_batch<<<fft.blocks, FFT_THREADS, fft.lds, s>>>(fft.map, (const FftCall*)fft.calls);
+    k_fft_x_batch<<<fft.blocks, FFTX_THREADS, fft.lds, s>>>(fft.map, (const FftCall*)fft.calls);
     MDX_LAUNCH_CHECK();
   }
   if (parts & 4u) {

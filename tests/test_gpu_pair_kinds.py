@@ -67,3 +67,39 @@ def test_mixed_lj_kinds_against_float64(n, bare):
         assert np.all(np.abs(got[1][k] - got[0][k]) <= 2.0 ** -39 + 8 * 2.0 ** -24 * size)
     assert abs(got[0][2]["lj"] - en[0]) <= 1e-5 * abs(en[0]) + 1e-9
     assert abs(got[0][2]["coulomb_direct"] - en[1]) <= 1e-5 * np.abs(size).max() + 1e-9
+
+
+@pytest.mark.parametrize("grid", [(4, 5, 6), (25, 24, 27), (20, 64, 45), (16, 128, 125), (100, 9, 128), (32, 135, 12),
+                                  (30, 40, 150)])
+def test_pme_grids_against_float64(grid):
+    """Reciprocal forces and energy of odd, even, uneven and large grids (the plane kernels hold up
+    to 128 x 128 points; larger planes take the global-grid path) against the float64 oracle."""
+    from mdpy_amd import _lib as L
+    from mdpy_amd.engine import Engine
+    from mdpy_amd.unit import ONE_OVER_4PI_EPS0
+    from oracle import ewald as EW
+    print("case: PME grid", grid, flush=True)
+    rng = np.random.default_rng(sum(grid))
+    n, box = 150, np.array([24.0, 26.5, 21.25])
+    x = rng.uniform(-0.5, 0.5, (n, 3)) * box
+    q = rng.uniform(-1, 1, n)
+    q[::7] = 0.0
+    e = Engine.bare(n, box, positions=x)
+    e.set_masses(np.ones(n))
+    e.set_charges(q)
+    e.set_lj(np.tile([0.0, 1.0, 0.0, 1.0], (n, 1)))
+    e.set_exclusions(np.zeros(n + 1, int), [])
+    e.set_scaling(np.zeros(n + 1, int), [])
+    e.configure_nonbonded(9.0, skin=1.0)
+    e.configure_pme(grid, 0.36)
+    F, en = e.compute(L.TERM_COUL_RECIP)
+    F = F.cpu().numpy()
+    assert e.status() == 0
+    e.close()
+    ref = EW.spme_reciprocal(x, q, box, grid, 4, 0.36, ONE_OVER_4PI_EPS0)
+    Fr, Er = ref[0], ref[1]
+    # float32 grid arithmetic: a few roundings per transform pass and 64 gathered points an atom
+    assert np.linalg.norm(F - Fr) <= 5e-6 * np.linalg.norm(Fr)
+    self_e = -ONE_OVER_4PI_EPS0 * 0.36 / math.sqrt(math.pi) * (q * q).sum()
+    back = -ONE_OVER_4PI_EPS0 * math.pi * q.sum() ** 2 / (2 * 0.36 ** 2 * box.prod())
+    assert abs(en["coulomb_reciprocal"] - (Er + self_e + back)) <= 1e-5 * (abs(Er) + abs(self_e))
