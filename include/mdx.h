@@ -295,9 +295,9 @@ int mdx_time_kernel(mdx_ctx* ctx, int which, unsigned terms, int reps, double* h
  * keep the fastest. The choice goes to *h_lanes (may be NULL). Synchronises. */
 int mdx_nonbonded_tune(mdx_ctx* ctx, unsigned terms, int lanes, int reps, int* h_lanes);
 /* Resident nonbonded workgroups (no reference counterpart): per_cu > 0 launches per_cu
- * workgroups per compute unit that loop over the nonbonded work (default 3, the measured best
- * beside the concurrent PME kernels); 0 launches one workgroup per unit of work. Same forces
- * either way. */
+ * workgroups per compute unit that loop over the nonbonded work; 0 launches one workgroup per
+ * unit of work. Default: 3 where that gives each at most two units, else 0 (the measured best
+ * beside the concurrent PME kernels). Same forces either way. */
 int mdx_nonbonded_persist(mdx_ctx* ctx, int per_cu);
 /* Scheduled list rebuilds (no reference counterpart): every > 0 also rebuilds the neighbour
  * list in the integrator step whose step counter is a multiple of `every`, besides the rebuilds

@@ -277,9 +277,10 @@ struct mdx_ctx {
   int nbr_cap = 0;               // capacity per atom
   int nb_lanes = 32;             // lanes per atom in the nonbonded kernel (16, 32 or 64) chosen by the
   bool nb_lanes_set = false;     // caller or the tuner; else mdx_nb_lanes chooses by system size
-  // nonbonded workgroups per compute unit looping over the work (0: one per unit of work); 3 (12
-  // waves of 123 VGPRs) leaves a quarter of every SIMD's registers to the PME kernels beside it
-  int nb_persist = 3;
+  // nonbonded workgroups per compute unit looping over the work (0: one per unit of work, -1: by the
+  // amount of work); 3 (12 waves of 123 VGPRs) leaves a quarter of every SIMD's registers to the PME
+  // kernels beside it
+  int nb_persist = -1;
   int rebuild_every = 0;  // scheduled list rebuilds (step counter multiple), 0 = displacement test only
   int cells_per_rl = 2;   // list-grid cells per list radius r_c + skin along each axis (1..3)
   int ncu = 0;                   // compute units of the device

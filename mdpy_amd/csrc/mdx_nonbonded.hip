@@ -79,6 +79,11 @@ __global__ __launch_bounds__(NB_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
       nb_block<LJ, COUL, ENERGY, G, NB_BLOCK, S14>(a, P, vb);
     return;
   }
+  if (nres == nb_blocks) {  // one unit each, in the same contiguous ranges per XCD
+    const int x = blockIdx.x & 7, q = nb_blocks >> 3, rem = nb_blocks & 7;
+    nb_block<LJ, COUL, ENERGY, G, NB_BLOCK, S14>(a, P, x * q + min(x, rem) + (blockIdx.x >> 3));
+    return;
+  }
   for (int vb = blockIdx.x; vb < nb_blocks; vb += nres) nb_block<LJ, COUL, ENERGY, G, NB_BLOCK, S14>(a, P, vb);
 }
 
@@ -144,8 +149,12 @@ int mdx_enqueue_nonbonded(mdx_ctx* c, bool lj, bool coul, bool energy, unsigned 
   const int nbb = (int)div_up((long long)c->n * lanes, NB_BLOCK);
   const int nbo = bonded_terms ? mdx_bonded_args(c, bonded_terms, &ba) : 0;
   // resident workgroups: all of them, or nb_persist per compute unit looping over the rest (so
-  // that the concurrent PME kernels find room on every compute unit)
-  const int nres = c->nb_persist > 0 ? std::min(nbb, c->nb_persist * c->ncu) : nbb;
+  // that the concurrent PME kernels find room on every compute unit). Unless set, 3 per compute unit
+  // when that gives each at most two units of work, else one workgroup per unit: with more units
+  // the dispatcher's balancing is worth more. A whole step with 3 per unit / one each (us): 23,328
+  // atoms (1,458 units) 88.1 / 89.4, 31,200 (1,950) 106.6 / 102.3, 98,304 (6,144) 375 / 324.
+  const int per = c->nb_persist >= 0 ? c->nb_persist : (nbb > 6 * c->ncu ? 0 : 3);
+  const int nres = per > 0 ? std::min(nbb, per * c->ncu) : nbb;
   dim3 grid(nres + nbo);
 #define NB_LAUNCH4(L_, C_, E_, S_)                                                                     \
   do {                                                                                                 \

@@ -103,3 +103,29 @@ def test_pme_grids_against_float64(grid):
     self_e = -ONE_OVER_4PI_EPS0 * 0.36 / math.sqrt(math.pi) * (q * q).sum()
     back = -ONE_OVER_4PI_EPS0 * math.pi * q.sum() ** 2 / (2 * 0.36 ** 2 * box.prod())
     assert abs(en["coulomb_reciprocal"] - (Er + self_e + back)) <= 1e-5 * (abs(Er) + abs(self_e))
+
+
+@pytest.mark.parametrize("n", [24576, 24577, 24700])
+def test_resident_workgroups_by_size(n):
+    """Both sides of the default's limit (at 16 lanes 1,536 units of work on 256 compute units) give
+    the bits of every explicit choice: forces are exact integer sums, in any order."""
+    from mdpy_amd import _lib as L
+    from mdpy_amd.engine import Engine
+    print("case: %d atoms" % n, flush=True)
+    rng = np.random.default_rng(n)
+    box, m = np.array([93.0, 96.0, 99.0]), 30
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    e = Engine.bare(n, box, positions=(g + 0.5) * box / m + rng.uniform(-0.4, 0.4, (n, 3)) - 0.5 * box)
+    e.set_masses(np.ones(n))
+    e.set_charges(rng.uniform(-1, 1, n))
+    e.set_lj(np.tile([0.1, 2.0, 0.1, 2.0], (n, 1)))
+    e.set_exclusions(np.zeros(n + 1, int), [])
+    e.set_scaling(np.zeros(n + 1, int), [])
+    e.configure_nonbonded(9.0, skin=1.0)
+    e.configure_pme((24, 24, 24), 0.36)
+    F = e.compute_forces_only(L.TERM_LJ | L.TERM_COUL_DIRECT).cpu().numpy().copy()
+    assert e.status() == 0 and np.abs(F).max() > 0
+    for per_cu in (0, 2, 3):
+        e.set_nonbonded_persist(per_cu)
+        assert np.array_equal(F, e.compute_forces_only(L.TERM_LJ | L.TERM_COUL_DIRECT).cpu().numpy()), per_cu
+    e.close()
