@@ -128,6 +128,7 @@ __device__ __forceinline__ int nbr_slot(unsigned e) { return (int)(e >> 4); }
 // neighbour-list entries allocated past the last row (at least the longest read-ahead: one
 // chunk of 64 lanes x 4 entries)
 #define MDX_LIST_SLACK 512
+#define MDX_LIST_PAD 64  // places of a list row past its capacity (the fast build stores 64 at a time)
 
 // ------------------------------------------------------------------ batched launches
 // One launch of a kernel covers the workgroups of many contexts (replicas): workgroup b belongs

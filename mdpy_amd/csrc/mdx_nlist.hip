@@ -413,6 +413,7 @@ __device__ __forceinline__ int cyc_dist(int a, int b, int n) {
 struct ListCall {
   ListArgs a;
   const float4* xq;
+  const int4* xf;
   const int* sorted_orig;
   const int* cell_start;
   const int* cell_count;
@@ -430,6 +431,7 @@ struct ListCall {
   unsigned* nbr_list;
   DevState* st;
   double thr2;
+  int split;  // fast build: workgroups per home cell
 };
 
 // the build of home cell `cell`
@@ -718,188 +720,318 @@ __global__ __launch_bounds__(BL_THREADS) void k_build_list_cell(ListCall L) {
   build_list_cell_body<EXACT64, FAST>(L, blockIdx.x);
 }
 
-// The common case of the build above as its own kernel: shifted candidates, exact pair mode,
-// float32 list radius, window masks present. One wave per home atom, so every ballot, count and
-// branch is wave-uniform; exclusions, the atom itself (bit 32) and 1-4 partners are mask bits, the
-// window offset is clamped to bit 63 (always clear) instead of range-checked, and the staged
-// chunk is padded with far-away candidates up to a multiple of the pass width, so a candidate
-// test is distance, two mask bits and the ballot. Home atoms with a partner outside the window
-// scan their CSR lists. A group of 64 candidates with none inside the list radius skips the mask
-// and store work. Produces the same lists, in the same order, as k_build_list_cell.
-#define BLF_PASS (64 * BL_U)
-__device__ __forceinline__ void build_list_fast_body(const ListCall& L, const int cell) {
+// The common case of the build above as its own kernel: exact pair mode, float32 list radius, and
+// either no exclusions or window masks present.
+//
+// Vector-instruction bound (the distance tests), so a test is made as short as it can be:
+// - positions are 32-bit box fractions, staged relative to the home cell's centre with their squared
+//   length, so "inside the list radius" is three fma and a compare, |b|^2 - 2 a.b < r^2 - |a|^2.
+//   Rounding moves r^2 by less than 3.2e-6 r_l^2 (cells of r_l/3 to r_l, at most 2.1 r_l from the
+//   centre to a listed atom); rl2 carries 1e-5 on top of r_l^2, so no pair inside r_l is missed.
+//   WRAP (a stencil that wraps onto itself, where one image per cell isn't enough) takes each
+//   pair's wrapped integer difference instead;
+// - a wave holds BLF_H home atoms in scalar registers and tests each staged candidate it reads from
+//   LDS against all of them, without a branch: lanes with nothing to store get an offset past the
+//   rows, and a row has room for one whole group after its capacity;
+// - exclusions, the atom itself and 1-4 partners are bits of window masks; 64 candidates of which none
+//   is near any of the home atoms both in space and in index (all but a few) skip them.
+// - candidates farther than the list radius from the home cell's box (3 of 10) are dropped as they
+//   are staged.
+// Home atoms with a partner outside the window scan their CSR lists. A grid of few cells gives each
+// cell to `split` workgroups (a share of its home atoms each). The lists are in the order of
+// k_build_list_cell.
+// Before (one home atom per wave pass, 40 vector and scalar instructions with 6 branches per test,
+// small boxes by k_build_list_cell) / now (us): 648 atoms 23 / 11, 2,592 r_c 12 92 / 24, 3,000 r_c 9
+// 75 / 23, 23,328 r_c 12 86 / 69, 98,304 r_c 12 285 / 226. The vector unit is busy 80 % of the time.
+#define BLF_H 4
+#define BLF_WAVES (BL_THREADS / 64)
+struct BlfShared {
+  float4 x[BL_CH];  // (x, y, z, |.|^2) from the home cell's centre; WRAP: box fractions and 0
+  int2 e[BL_CH];    // (list entry, original atom id)
+  int2 sc[BL_MAXST + 1];  // stencil cells: (first candidate, sorted slot of candidate 0 if it were in this cell)
+  int kept[BL_CH / 64];   // candidates kept of each 64
+  int acnt[SORT_MAX];
+  int exl[BLF_WAVES][BL_MAXEX], s4l[BLF_WAVES][BL_MAXEX];
+  int4 hx[BL_HMAX];
+  int ho[BL_HMAX];
+  unsigned long long hexm[BL_HMAX], hs4m[BL_HMAX];
+  unsigned char hbad[BL_HMAX];
+};
+
+// One chunk of nch staged candidates against H home atoms; lane k of the *l arguments holds home
+// atom k's position terms (WRAP: fractions), limit, atom id, count and masks. Returns the counts.
+template <int H, bool WRAP>
+__device__ __forceinline__ int blf_scan(const float4* __restrict__ x, const int2* __restrict__ e, int nch, float al,
+                                        float bl, float cl, float rl, int ol, int cntl, unsigned long long exl,
+                                        unsigned long long s4l, unsigned* rows_p, int cap, float sx, float sy, float sz) {
+  const int lane = threadIdx.x & 63, lim = cap - MDX_LIST_PAD;
+  int ia[H], ib[H], ic[H], cnt[H];
+  unsigned o32[H];
+  float rhs[H];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    ia[k] = __builtin_amdgcn_readlane(__float_as_int(al), k);
+    ib[k] = __builtin_amdgcn_readlane(__float_as_int(bl), k);
+    ic[k] = __builtin_amdgcn_readlane(__float_as_int(cl), k);
+    rhs[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rl), k));
+    o32[k] = (unsigned)__builtin_amdgcn_readlane(ol, k) - 32u;
+    cnt[k] = __builtin_amdgcn_readlane(cntl, k);
+  }
+  // the rows of these home atoms; a store past their end is dropped
+  __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(rows_p, 0, H * cap * 4, 0x00020000);
+  float4 xn = x[lane];
+  int2 en = e[lane];
+  for (int cb = 0; cb < nch; cb += 64) {
+    const float4 xj = xn;
+    const int2 ej = en;
+    const int nb = cb + 64 < nch ? cb + 64 : 0;  // the next 64, in flight
+    xn = x[nb + lane];
+    en = e[nb + lane];
+    unsigned long long m[H], any = 0;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      bool near;
+      if (WRAP) {
+        const float dx = (float)(int)(__float_as_uint(xj.x) - (unsigned)ia[k]) * sx;
+        const float dy = (float)(int)(__float_as_uint(xj.y) - (unsigned)ib[k]) * sy;
+        const float dz = (float)(int)(__float_as_uint(xj.z) - (unsigned)ic[k]) * sz;
+        near = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, xj.w))) < rhs[k];
+      } else {
+        near = fmaf(xj.x, __int_as_float(ia[k]),
+                    fmaf(xj.y, __int_as_float(ib[k]), fmaf(xj.z, __int_as_float(ic[k]), xj.w))) < rhs[k];
+      }
+      m[k] = __ballot(near);
+      any |= m[k] & __ballot((unsigned)ej.y - o32[k] < 64u);
+    }
+    int entry[H];
+#pragma unroll
+    for (int k = 0; k < H; ++k) entry[k] = ej.x;
+    if (any != 0) {  // scalar: some candidate is near a home atom in space and in index
+#pragma unroll
+      for (int k = 0; k < H; ++k) {
+        const unsigned dw = min((unsigned)ej.y - o32[k], 63u);  // bit 63 is always clear
+        const unsigned long long exm = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(exl >> 32), k) << 32 |
+                                       (unsigned)__builtin_amdgcn_readlane((int)exl, k);
+        const unsigned long long s4m = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(s4l >> 32), k) << 32 |
+                                       (unsigned)__builtin_amdgcn_readlane((int)s4l, k);
+        m[k] &= __ballot(!((exm >> dw) & 1ull));
+        entry[k] |= (int)((s4m >> dw) & 1ull);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      int slot4 = 4 * (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m[k] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m[k], 0u));
+      asm volatile("" : "+v"(slot4));  // computed for every lane: a select follows, not a branch
+      const int off = __builtin_amdgcn_inverse_ballot_w64(m[k]) ? slot4 : (int)0x80000000;
+      __builtin_amdgcn_raw_buffer_store_b32((unsigned)entry[k], rows, off, (k * cap + min(cnt[k], lim)) * 4, 0);
+      cnt[k] += __popcll(m[k]);
+    }
+  }
+  int out = 0;
+#pragma unroll
+  for (int k = 0; k < H; ++k) out = lane == k ? cnt[k] : out;
+  return out;
+}
+
+template <bool WRAP>
+__device__ __forceinline__ void build_list_fast_body(const ListCall& L, const int block, BlfShared& sh) {
+  static_assert(BL_CH % BL_THREADS == 0 && BL_CH / 64 <= 64, "a lane per 64 of a chunk");
   const ListArgs& a = L.a;
-  const float4* __restrict__ xq = L.xq;
+  const int4* __restrict__ xf = L.xf;
   const int* __restrict__ sorted_orig = L.sorted_orig;
-  const int* __restrict__ cell_start = L.cell_start;
-  const int* __restrict__ cell_count = L.cell_count;
-  const int* __restrict__ stencil = L.stencil;
   const int* __restrict__ excl_ptr = L.excl_ptr;
   const int* __restrict__ excl_idx = L.excl_idx;
   const int* __restrict__ s14_ptr = L.s14_ptr;
   const int* __restrict__ s14_idx = L.s14_idx;
-  const unsigned long long* __restrict__ ex_win = L.ex_win;
-  const unsigned long long* __restrict__ s4_win = L.s4_win;
-  const unsigned char* __restrict__ win_bad = L.win_bad;
   int* __restrict__ nbr_count = L.nbr_count;
   unsigned* __restrict__ nbr_list = L.nbr_list;
   DevState* st = L.st;
-  const double thr2 = L.thr2;
-  static_assert(BL_CH % BLF_PASS == 0, "chunks must hold whole passes");
-  if (!need_rebuild(st, thr2)) return;
-  __shared__ float4 cxq[BL_CH];
-  __shared__ int2 cto[BL_CH];  // (sorted slot, original atom id)
-  __shared__ int sb[BL_MAXST], sp[BL_MAXST + 1];
-  __shared__ unsigned char shc[BL_MAXST];
-  __shared__ int acnt[SORT_MAX];
-  __shared__ int exl[BL_THREADS / 64][BL_MAXEX], s4l[BL_THREADS / 64][BL_MAXEX];
-  __shared__ float4 hxi[BL_HMAX];
-  __shared__ int ho[BL_HMAX];
-  __shared__ unsigned long long hexm[BL_HMAX], hs4m[BL_HMAX];
-  __shared__ unsigned char hbad[BL_HMAX];
+  if (!need_rebuild(st, L.thr2)) return;
+  const int cell = block / L.split, part = block - cell * L.split;
   const GridArgs& gr = a.g;
-  const int hb = cell_start[cell], hn = cell_count[cell];
-  if (hn > SORT_MAX) {  // oversize cells are flagged where the cells are counted: empty lists
-    for (int t = threadIdx.x; t < hn; t += blockDim.x) nbr_count[hb + t] = 0;
+  const int hb = L.cell_start[cell], hn_all = L.cell_count[cell];
+  // this workgroup's share of the home atoms
+  const int p0 = (int)((long long)hn_all * part / L.split), p1 = (int)((long long)hn_all * (part + 1) / L.split);
+  const int tid = threadIdx.x;
+  if (hn_all > SORT_MAX) {  // oversize cells are flagged where the cells are counted: empty lists
+    for (int t = p0 + tid; t < p1; t += BL_THREADS) nbr_count[hb + t] = 0;
     return;
   }
-  if (hn == 0) return;
-  const int tid = threadIdx.x;
+  if (p0 == p1) return;
+  const int s0 = hb + p0, hn = p1 - p0;
   const int hz = cell % gr.nz, hy = (cell / gr.nz) % gr.ny, hx = cell / (gr.nz * gr.ny);
-  for (int k = tid; k < a.nstencil; k += blockDim.x) {
-    int p = stencil[k];
+  for (int k = tid; k < a.nstencil; k += BL_THREADS) {
+    const int p = L.stencil[k];
     int nx = hx + ((p >> 16) & 0xff) - 128, ny = hy + ((p >> 8) & 0xff) - 128, nz = hz + (p & 0xff) - 128;
-    const int cx = nx < 0 ? 0 : (nx >= gr.nx ? 2 : 1);
-    const int cy = ny < 0 ? 0 : (ny >= gr.ny ? 2 : 1);
-    const int cz = nz < 0 ? 0 : (nz >= gr.nz ? 2 : 1);
-    shc[k] = (unsigned char)(cx | (cy << 2) | (cz << 4));
     nx += nx < 0 ? gr.nx : (nx >= gr.nx ? -gr.nx : 0);
     ny += ny < 0 ? gr.ny : (ny >= gr.ny ? -gr.ny : 0);
     nz += nz < 0 ? gr.nz : (nz >= gr.nz ? -gr.nz : 0);
     const int nc = (nx * gr.ny + ny) * gr.nz + nz;
-    sb[k] = cell_start[nc];
-    sp[k + 1] = cell_count[nc];
+    sh.sc[k] = make_int2(L.cell_count[nc], L.cell_start[nc]);
   }
-  for (int j = tid; j < hn; j += blockDim.x) acnt[j] = 0;
+  for (int j = tid; j < hn; j += BL_THREADS) sh.acnt[j] = 0;
   const bool fit = hn <= BL_HMAX;
   if (fit) {
-    for (int h = tid; h < hn; h += blockDim.x) {
-      const int o = sorted_orig[hb + h];
-      ho[h] = o;
-      hxi[h] = xq[hb + h];
-      hexm[h] = ex_win[o];
-      hs4m[h] = s4_win[o];
-      hbad[h] = win_bad[o];
+    for (int h = tid; h < hn; h += BL_THREADS) {
+      const int o = sorted_orig[s0 + h];
+      sh.ho[h] = o;
+      sh.hx[h] = xf[s0 + h];
+      sh.hexm[h] = L.ex_win ? L.ex_win[o] : 1ull << 32;
+      sh.hs4m[h] = L.s4_win ? L.s4_win[o] : 0ull;
+      sh.hbad[h] = L.win_bad ? L.win_bad[o] : (unsigned char)0;
     }
   }
-  __syncthreads();
-  if (tid == 0) {
-    sp[0] = 0;
-    for (int k = 0; k < a.nstencil; ++k) sp[k + 1] += sp[k];
-  }
-  __syncthreads();
-  const int total = sp[a.nstencil];
-  const float Lx = (float)gr.Lx, Ly = (float)gr.Ly, Lz = (float)gr.Lz;
-  float4 pv[BL_SLOTS];
-  int2 pt[BL_SLOTS];
-  auto fetch = [&](int base) {
-    const int nch = min(BL_CH, total - base);
-#pragma unroll
-    for (int r = 0; r < BL_SLOTS; ++r) {
-      const int c = tid + r * BL_THREADS;
-      if (c < nch) {
-        const int idx = base + c;
-        int lo = 0, hi = a.nstencil - 1;  // last stencil cell whose prefix <= idx
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if (sp[mid] <= idx) lo = mid;
-          else hi = mid - 1;
-        }
-        const int t = sb[lo] + (idx - sp[lo]);
-        float4 v = xq[t];
-        const int code = shc[lo];
-        v.x += (float)((code & 3) - 1) * Lx;
-        v.y += (float)(((code >> 2) & 3) - 1) * Ly;
-        v.z += (float)(((code >> 4) & 3) - 1) * Lz;
-        pv[r] = v;
-        pt[r] = make_int2(t, sorted_orig[t]);
-      }
-    }
-  };
-  auto store = [&](int base) {
-    const int nch = min(BL_CH, total - base);
-    const int npad = min(BL_CH, (nch + BLF_PASS - 1) / BLF_PASS * BLF_PASS);
-#pragma unroll
-    for (int r = 0; r < BL_SLOTS; ++r) {
-      const int c = tid + r * BL_THREADS;
-      if (c < nch) {
-        cxq[c] = pv[r];
-        cto[c] = pt[r];
-      } else if (c < npad) {  // far away: fails the distance test
-        cxq[c] = make_float4(1e30f, 1e30f, 1e30f, 0.f);
-        cto[c] = make_int2(0, 0);
-      }
-    }
-  };
-  if (total > 0) fetch(0);
-  store(0);
   __syncthreads();
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar registers
-  constexpr int nw = BL_THREADS / 64;
-  int* my_ex = exl[w];
-  int* my_s4 = s4l[w];
+  if (w == 0) {  // prefix sums of the stencil cells' sizes, a run of them per lane
+    const int per = (a.nstencil + 63) >> 6, k0 = lane * per, k1 = min(a.nstencil, k0 + per);
+    int sum = 0;
+    for (int k = k0; k < k1; ++k) sum += sh.sc[k].x;
+    int incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += v;
+    }
+    int run = incl - sum;
+    for (int k = k0; k < k1; ++k) {
+      const int2 v = sh.sc[k];
+      sh.sc[k] = make_int2(run, v.y - run);
+      run += v.x;
+    }
+    if (lane == 63) sh.sc[a.nstencil] = make_int2(incl, 0);
+  }
+  __syncthreads();
+  const int total = sh.sc[a.nstencil].x;
+  const float sx = (float)(gr.Lx * 0x1p-32), sy = (float)(gr.Ly * 0x1p-32), sz = (float)(gr.Lz * 0x1p-32);
+  // centre of the home cell as box fractions, and its half widths
+  const int ccx = (int)(unsigned)((hx + 0.5) / gr.nx * 4294967296.0), ccy = (int)(unsigned)((hy + 0.5) / gr.ny * 4294967296.0),
+            ccz = (int)(unsigned)((hz + 0.5) / gr.nz * 4294967296.0);
+  const float hwx = 0.5f * (float)gr.wx, hwy = 0.5f * (float)gr.wy, hwz = 0.5f * (float)gr.wz;
+  const float reach2 = a.rl2 * 1.0001f;
+  auto relative = [&](const int4& f) {
+    float4 v;
+    v.x = (float)(int)((unsigned)f.x - (unsigned)ccx) * sx;
+    v.y = (float)(int)((unsigned)f.y - (unsigned)ccy) * sy;
+    v.z = (float)(int)((unsigned)f.z - (unsigned)ccz) * sz;
+    v.w = fmaf(v.x, v.x, fmaf(v.y, v.y, v.z * v.z));
+    return v;
+  };
+  int4 pv[BL_SLOTS];
+  int2 pt[BL_SLOTS];
+  auto fetch = [&](int base) {
+#pragma unroll
+    for (int r = 0; r < BL_SLOTS; ++r) {
+      const int first = base + w * 64 + r * BL_THREADS, idx = first + lane;  // the wave's candidates: first ..
+      if (first >= total) break;
+      // the cell of the first one, by counting the cells that begin at or before it; then on from cell
+      // to cell while they begin inside the wave's 64
+      int k = -1;
+      for (int b = 0; b < a.nstencil; b += 64)
+        k += __popcll(__ballot(b + lane < a.nstencil && sh.sc[min(b + lane, a.nstencil)].x <= first));
+      int off = sh.sc[k].y;
+      for (++k; k < a.nstencil; ++k) {
+        const int2 v = sh.sc[k];
+        if (__builtin_amdgcn_readfirstlane(v.x) > first + 63) break;
+        if (idx >= v.x) off = v.y;
+      }
+      if (idx < total) {
+        const int t = off + idx;
+        pv[r] = xf[t];
+        pt[r] = make_int2((int)nbr_entry(t, false), sorted_orig[t]);
+      }
+    }
+  };
+  // the fetched candidates within the list radius of the home cell's box
+  float4 sv[BL_SLOTS];
+  unsigned long long keep[BL_SLOTS];
+  auto select = [&](int base) {
+#pragma unroll
+    for (int r = 0; r < BL_SLOTS; ++r) {
+      const float4 v = relative(pv[r]);
+      const float dx = fmaxf(fabsf(v.x) - hwx, 0.f), dy = fmaxf(fabsf(v.y) - hwy, 0.f), dz = fmaxf(fabsf(v.z) - hwz, 0.f);
+      keep[r] = __ballot(base + tid + r * BL_THREADS < total && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < reach2);
+      sv[r] = WRAP ? make_float4(__int_as_float(pv[r].x), __int_as_float(pv[r].y), __int_as_float(pv[r].z), 0.f) : v;
+      if (lane == 0) sh.kept[r * BLF_WAVES + w] = __popcll(keep[r]);
+    }
+  };
+  // staged in order, behind the candidates kept of the 64s before; padded to whole passes with
+  // candidates far away from everything. Returns their number.
+  auto store = [&]() {
+    int incl = lane < BL_CH / 64 ? sh.kept[lane] : 0;
+    for (int d = 1; d < BL_CH / 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += v;
+    }
+    const int n = __builtin_amdgcn_readlane(incl, BL_CH / 64 - 1);
+#pragma unroll
+    for (int r = 0; r < BL_SLOTS; ++r) {
+      const int c0 = __builtin_amdgcn_readlane(incl, r * BLF_WAVES + w) - __popcll(keep[r]);
+      const int c = c0 + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(keep[r] >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((unsigned)keep[r], 0u));
+      if (__builtin_amdgcn_inverse_ballot_w64(keep[r])) {
+        sh.x[c] = sv[r];
+        sh.e[c] = pt[r];
+      }
+    }
+    if (n + tid < ((n + 63) & ~63)) {
+      sh.x[n + tid] = make_float4(0.f, 0.f, 0.f, 1e30f);
+      sh.e[n + tid] = make_int2(0, 0);
+    }
+    return n;
+  };
+  fetch(0);
+  select(0);
+  __syncthreads();
+  int nch = store();
+  __syncthreads();
+  int* my_ex = sh.exl[w];
+  int* my_s4 = sh.s4l[w];
+  const int lim = a.cap - MDX_LIST_PAD;  // capacity of a row: a group's 64 entries fit after it
+  const int hw0 = hn * w / BLF_WAVES, hw1 = hn * (w + 1) / BLF_WAVES;  // this wave's home atoms
   for (int base = 0; base < total; base += BL_CH) {
-    const int nch = min(BL_CH, total - base);
     const bool more = base + BL_CH < total;
     if (more) fetch(base + BL_CH);  // in flight during this chunk's scan
-    for (int h = w; h < hn; h += nw) {  // wave-uniform
-      const int s = hb + h;
-      int o;
-      float4 xi;
+    for (int h0 = hw0, nh; h0 < hw1; h0 += nh) {
+      const int rounds = (hw1 - h0 + BLF_H - 1) / BLF_H;
+      nh = (hw1 - h0 + rounds - 1) / rounds;
+      // one lane per home atom reads its data
+      const int hl = h0 + min(lane, nh - 1), sl = s0 + hl;
+      int4 fl;
+      int ol;
       unsigned long long exm, s4m;
-      bool masked;
+      bool bad;
       if (fit) {
-        o = ho[h];
-        xi = hxi[h];
-        exm = hexm[h];
-        s4m = hs4m[h];
-        masked = hbad[h] == 0;
+        fl = sh.hx[hl];
+        ol = sh.ho[hl];
+        exm = sh.hexm[hl];
+        s4m = sh.hs4m[hl];
+        bad = sh.hbad[hl] != 0;
       } else {
-        o = sorted_orig[s];
-        xi = xq[s];
-        exm = ex_win[o];
-        s4m = s4_win[o];
-        masked = win_bad[o] == 0;
+        fl = xf[sl];
+        ol = sorted_orig[sl];
+        exm = L.ex_win ? L.ex_win[ol] : 1ull << 32;
+        s4m = L.s4_win ? L.s4_win[ol] : 0ull;
+        bad = L.win_bad && L.win_bad[ol] != 0;
       }
-      unsigned* row = nbr_list + (long long)s * a.cap;
-      int cnt = acnt[h];
-      if (masked) {
-        const unsigned o32 = __builtin_amdgcn_readfirstlane((unsigned)(o - 32));
-        for (int cb = 0; cb < nch; cb += BLF_PASS) {
-          float4 xj[BL_U];
-          int2 tj[BL_U];
-#pragma unroll
-          for (int u = 0; u < BL_U; ++u) {
-            xj[u] = cxq[cb + u * 64 + lane];
-            tj[u] = cto[cb + u * 64 + lane];
-          }
-#pragma unroll
-          for (int u = 0; u < BL_U; ++u) {
-            const float dx = xj[u].x - xi.x, dy = xj[u].y - xi.y, dz = xj[u].z - xi.z;
-            const bool near = dx * dx + dy * dy + dz * dz < a.rl2;
-            const unsigned long long mn = __ballot(near);
-            if (mn == 0) continue;  // wave-uniform: no candidate of these 64 inside the list radius
-            const unsigned dw = min((unsigned)tj[u].y - o32, 63u);
-            const bool kept = !((exm >> dw) & 1ull);
-            const bool acc = near && kept;
-            const unsigned long long m = mn & __ballot(kept);  // two compares, no re-materialised mask
-            const int slot = cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-            if (acc && slot < a.cap) row[slot] = nbr_entry(tj[u].x, (s4m >> dw) & 1ull);
-            cnt += __popcll(m);
-          }
-        }
-      } else {  // a partner outside the index window: the CSR lists
+      const float4 rel = relative(fl);
+      const float ha = WRAP ? __int_as_float(fl.x) : -2.f * rel.x, hbb = WRAP ? __int_as_float(fl.y) : -2.f * rel.y,
+                  hc = WRAP ? __int_as_float(fl.z) : -2.f * rel.z, hr = WRAP ? a.rl2 : a.rl2 - rel.w;
+      const float rhs = bad ? -3e38f : hr;  // no candidate is inside: done below
+      const int before = sh.acnt[hl];
+      unsigned* rows = nbr_list + (long long)(s0 + h0) * a.cap;
+      int after;
+#define BLF_SCAN(H_) after = blf_scan<H_, WRAP>(sh.x, sh.e, nch, ha, hbb, hc, rhs, ol, before, exm, s4m, rows, a.cap, sx, sy, sz)
+      if (nh == 4) BLF_SCAN(4);
+      else if (nh == 3) BLF_SCAN(3);
+      else if (nh == 2) BLF_SCAN(2);
+      else BLF_SCAN(1);
+#undef BLF_SCAN
+      if (lane < nh) sh.acnt[hl] = after;
+      for (unsigned left = (unsigned)__ballot(bad && lane < nh); left; left &= left - 1u) {
+        // a partner outside the index window: the CSR lists
+        const int k = __builtin_amdgcn_readfirstlane(__ffs(left) - 1);
+        const int o = __builtin_amdgcn_readlane(ol, k), s = s0 + h0 + k;
+        int count = __builtin_amdgcn_readlane(before, k);
         const int e0 = excl_ptr ? excl_ptr[o] : 0, t0s = s14_ptr ? s14_ptr[o] : 0;
         const int nex_all = excl_ptr ? excl_ptr[o + 1] - e0 : 0, ns4_all = s14_ptr ? s14_ptr[o + 1] - t0s : 0;
         const int nex = min(nex_all, BL_MAXEX), ns4 = min(ns4_all, BL_MAXEX);
@@ -907,45 +1039,65 @@ __device__ __forceinline__ void build_list_fast_body(const ListCall& L, const in
         if (lane < ns4) my_s4[lane] = s14_idx[t0s + lane];
         if (lane == 0 && (nex_all > BL_MAXEX || ns4_all > BL_MAXEX)) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
         wave_lds_sync();
+        unsigned* row = nbr_list + (long long)s * a.cap;
+        const float kx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ha), k)),
+                    ky = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hbb), k)),
+                    kz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hc), k)),
+                    kr = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hr), k));
         for (int cb = 0; cb < nch; cb += 64) {
-          const float4 xj = cxq[cb + lane];
-          const int2 tj = cto[cb + lane];
-          const float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-          bool acc = dx * dx + dy * dy + dz * dz < a.rl2 && tj.x != s;
+          const float4 xj = sh.x[cb + lane];
+          const int2 ej = sh.e[cb + lane];
+          float r2;
+          if (WRAP) {
+            const float dx = (float)(int)(__float_as_uint(xj.x) - __float_as_uint(kx)) * sx;
+            const float dy = (float)(int)(__float_as_uint(xj.y) - __float_as_uint(ky)) * sy;
+            const float dz = (float)(int)(__float_as_uint(xj.z) - __float_as_uint(kz)) * sz;
+            r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, xj.w)));
+          } else {
+            r2 = fmaf(xj.x, kx, fmaf(xj.y, ky, fmaf(xj.z, kz, xj.w)));
+          }
+          bool acc = r2 < kr && ej.y != o;
           bool s14 = false;
-          for (int r = 0; r < nex; ++r) acc &= (my_ex[r] != tj.y);
-          for (int r = 0; r < ns4; ++r) s14 |= (my_s4[r] == tj.y);
+          for (int r = 0; r < nex; ++r) acc &= (my_ex[r] != ej.y);
+          for (int r = 0; r < ns4; ++r) s14 |= (my_s4[r] == ej.y);
           const unsigned long long m = __ballot(acc);
-          const int slot = cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-          if (acc && slot < a.cap) row[slot] = nbr_entry(tj.x, s14);
-          cnt += __popcll(m);
+          const int slot = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+          if (acc && slot < lim) row[slot] = (unsigned)(ej.x | (int)s14);
+          count += __popcll(m);
         }
+        if (lane == 0) sh.acnt[h0 + k] = count;
         wave_lds_sync();  // the wave's next home atom overwrites my_ex / my_s4
       }
-      if (lane == 0) acnt[h] = cnt;
     }
+    if (more) select(base + BL_CH);
     __syncthreads();
     if (more) {
-      store(base + BL_CH);
+      nch = store();
       __syncthreads();
     }
   }
-  for (int h = tid; h < hn; h += blockDim.x) {
-    const int cnt = acnt[h];
-    nbr_count[hb + h] = min(cnt, a.cap);
-    if (cnt > a.cap) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
+  for (int h = tid; h < hn; h += BL_THREADS) {
+    const int cnt = sh.acnt[h];
+    nbr_count[s0 + h] = min(cnt, lim);
+    if (cnt > lim) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
   }
 }
 
-__global__ __launch_bounds__(BL_THREADS) void k_build_list_fast(ListCall L) { build_list_fast_body(L, blockIdx.x); }
+template <bool WRAP>
+__global__ __launch_bounds__(BL_THREADS) void k_build_list_fast(ListCall L) {
+  __shared__ BlfShared sh;
+  build_list_fast_body<WRAP>(L, blockIdx.x, sh);
+}
 
-// every replica's list build in one launch (the fast build, or the cell build of a grid whose
-// stencil wraps onto itself)
+// every replica's list build in one launch (the fast build, or the cell build of a replica whose
+// exclusions have no window masks)
 __global__ __launch_bounds__(BL_THREADS) void k_build_list_fast_batch(BatchMap map, const ListCall* __restrict__ calls) {
-  int cell;
-  const int r = batch_replica(map, &cell);
-  build_list_fast_body(calls[r], cell);
+  __shared__ BlfShared sh;
+  int block;
+  const int r = batch_replica(map, &block);
+  if (calls[r].a.shifted) build_list_fast_body<false>(calls[r], block, sh);
+  else build_list_fast_body<true>(calls[r], block, sh);
 }
 __global__ __launch_bounds__(BL_THREADS) void k_build_list_cell_batch(BatchMap map, const ListCall* __restrict__ calls) {
   int cell;
@@ -1039,6 +1191,7 @@ int mdx_nlist_prepare(mdx_ctx* c) {
   double expect = 4.0 / 3.0 * M_PI * rl * rl * rl * dens;
   int cap = (int)(expect * 1.5 + 64);
   if (cap > c->n) cap = c->n;
+  cap += MDX_LIST_PAD;
   if (cap < c->nbr_cap) cap = c->nbr_cap;
   c->nbr_cap = cap;
   c->list_stride = cap;
@@ -1114,8 +1267,18 @@ int mdx_nlist_update_order(mdx_ctx* c, bool force_rebuild) {
   return pro ? 0 : mdx_nlist_enqueue_pack(c);
 }
 
-// The list-build launch of a context: its arguments and kernel (0: the fast build; 1-4: the cell
-// build <EXACT64, FAST> = <false,false>, <false,true>, <true,false>, <true,true>).
+// Fast build: workgroups per home cell. Grids of few cells leave the chip idle: up to 8 workgroups
+// share a cell's atoms until there's about one per compute unit (each stages the cell's candidates,
+// so more cost more than they give). One / by this rule (us): 648 atoms r_c 9 (27 cells) 14.6 / 11.4,
+// 2,592 r_c 12 (64 cells) 41 / 24, 3,000 r_c 9 (125 cells) 29 / 23.
+static int blf_split(const mdx_ctx* c) {
+  int s = 1;
+  while (s < 8 && 2 * s * c->ncell <= c->ncu) s *= 2;
+  return s;
+}
+
+// The list-build launch of a context: its arguments and kernel (0: the fast build; 1-3: the cell
+// build <EXACT64, FAST> = <false,false>, <true,false>, <true,true>).
 static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   const bool ref = c->pair_mode == MDX_PAIRS_REFERENCE;
   ListArgs& a = L->a;
@@ -1138,8 +1301,10 @@ static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   for (int d = 0; d < 3; ++d)
     if (2 * c->reach[d] + 1 >= c->gn[d]) a.shifted = 0;
   const bool win = c->win_ready && c->h_win_bad.size() == (size_t)c->n;
-  const bool fastk = a.shifted && !a.ref_mode && win;
+  const bool masks = win || !(c->has_excl || c->has_s14);  // without either only the atom itself is masked
+  const bool fast = masks && !a.ref_mode && !a.exact64;
   L->xq = c->xq.p;
+  L->xf = c->xf.p;
   L->sorted_orig = c->sorted_orig.p;
   L->cell_start = c->cell_start.p;
   L->cell_count = c->cell_count.p;
@@ -1157,7 +1322,8 @@ static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   L->nbr_list = c->nbr_list.p;
   L->st = c->dstate.p;
   L->thr2 = rebuild_thr2(c);
-  *kind = fastk && !a.exact64 ? 0 : 1 + (a.exact64 ? 2 : 0) + (fastk ? 1 : 0);
+  L->split = blf_split(c);
+  *kind = fast ? 0 : (!a.exact64 ? 1 : (win && a.shifted && !a.ref_mode ? 3 : 2));
   return 0;
 }
 
@@ -1168,10 +1334,14 @@ int mdx_nlist_update_list(mdx_ctx* c) {
   if (rc) return rc;
   dim3 grid(c->ncell), block(BL_THREADS);
   switch (kind) {
-    case 0: k_build_list_fast<<<grid, block, 0, c->stream>>>(L); break;
+    case 0: {
+      grid.x *= L.split;
+      if (L.a.shifted) k_build_list_fast<false><<<grid, block, 0, c->stream>>>(L);
+      else k_build_list_fast<true><<<grid, block, 0, c->stream>>>(L);
+      break;
+    }
     case 1: k_build_list_cell<false, false><<<grid, block, 0, c->stream>>>(L); break;
-    case 2: k_build_list_cell<false, true><<<grid, block, 0, c->stream>>>(L); break;
-    case 3: k_build_list_cell<true, false><<<grid, block, 0, c->stream>>>(L); break;
+    case 2: k_build_list_cell<true, false><<<grid, block, 0, c->stream>>>(L); break;
     default: k_build_list_cell<true, true><<<grid, block, 0, c->stream>>>(L); break;
   }
   MDX_LAUNCH_CHECK();
@@ -1202,7 +1372,7 @@ int mdx_batch_prepare_list(mdx_ctx* const* cs, int n, BatchKind* fill, BatchKind
     // every replica holds a place in both builds (zero workgroups in the one it does not use)
     lf.push_back(L);
     lc.push_back(L);
-    bf.push_back(kind == 0 ? c->ncell : 0);
+    bf.push_back(kind == 0 ? c->ncell * L.split : 0);
     bc.push_back(kind == 1 ? c->ncell : 0);
   }
   int rc;
