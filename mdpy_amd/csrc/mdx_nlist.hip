@@ -734,7 +734,7 @@ __global__ __launch_bounds__(BL_THREADS) void k_build_list_cell(ListCall L) {
 //   LDS against all of them, without a branch: lanes with nothing to store get an offset past the
 //   rows, and a row has room for one whole group after its capacity;
 // - exclusions, the atom itself and 1-4 partners are bits of window masks; 64 candidates of which none
-//   is near any of the home atoms both in space and in index (all but a few) skip them.
+//   is near any of the home atoms both in space and in index (all but a few) skip them;
 // - candidates farther than the list radius from the home cell's box (3 of 10) are dropped as they
 //   are staged.
 // Home atoms with a partner outside the window scan their CSR lists. A grid of few cells gives each
