@@ -713,24 +713,47 @@ __global__ void k_ml_top(int rows, int row_split, const float* __restrict__ a3, 
   dz16[i] = f2bf(v);
   dz32[i] = v;
 }
-// column sums over rows [r0, r1) of in[row][c] in a fixed order: block b sums its chunk of rows
-// (one lane per column, coalesced), then one lane per column adds the chunk sums in order
+// Column sums over rows [r0, r1) of the four ML_H-wide arrays, in a fixed order: workgroup (b, q) sums
+// chunk b of array q's rows (wave w the rows w, w + 4, ..; a float4 of columns per lane, so a row is
+// one coalesced load of a wave), its waves' sums are added in order, then one lane per column adds
+// the chunks' sums in order. Bandwidth bound: one launch for the four arrays and enough chunks to
+// have the whole chip reading, where one lane per column ran a chain of dependent loads. 23,328
+// rows, both elements (us): 277 + 40 -> 27 + 9.
 #define COLSUM_CHUNKS 128
-__global__ void k_ml_colsum_part(const float* __restrict__ in, int r0, int r1, int ncol, float* __restrict__ part) {
-  const int c = threadIdx.x;
+#define COLSUM_ARRAYS 4
+struct ColsumArgs {
+  const float* in[COLSUM_ARRAYS];
+  float* out[COLSUM_ARRAYS];
+};
+__global__ __launch_bounds__(256) void k_ml_colsum_part(ColsumArgs a, int r0, int r1, float* __restrict__ part) {
+  __shared__ float4 sm[4][ML_H / 4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int len = (r1 - r0 + COLSUM_CHUNKS - 1) / COLSUM_CHUNKS;
-  const int a = r0 + blockIdx.x * len, b = min(r1, a + len);
-  if (c >= ncol) return;
-  float s = 0.f;
-  for (int r = a; r < b; ++r) s += in[(long long)r * ncol + c];
-  part[blockIdx.x * ncol + c] = s;
-}
-__global__ void k_ml_colsum_fin(const float* __restrict__ part, int ncol, float* __restrict__ out) {
+  const int b0 = r0 + blockIdx.x * len, b1 = min(r1, b0 + len);
+  const float4* __restrict__ in = (const float4*)a.in[blockIdx.y];
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 8
+  for (int r = b0 + w; r < b1; r += 4) {
+    const float4 v = in[(long long)r * (ML_H / 4) + lane];
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  sm[w][lane] = s;
+  __syncthreads();
+  const float* f = (const float*)sm;
   const int c = threadIdx.x;
-  if (c >= ncol) return;
+  part[((long long)blockIdx.y * COLSUM_CHUNKS + blockIdx.x) * ML_H + c] =
+      ((f[c] + f[ML_H + c]) + f[2 * ML_H + c]) + f[3 * ML_H + c];
+}
+__global__ __launch_bounds__(ML_H) void k_ml_colsum_fin(ColsumArgs a, const float* __restrict__ part) {
+  const int c = threadIdx.x;
+  part += (long long)blockIdx.x * COLSUM_CHUNKS * ML_H;
   float s = 0.f;
-  for (int k = 0; k < COLSUM_CHUNKS; ++k) s += part[k * ncol + c];
-  out[c] = s;
+#pragma unroll 16
+  for (int k = 0; k < COLSUM_CHUNKS; ++k) s += part[k * ML_H + c];
+  a.out[blockIdx.x][c] = s;
 }
 // sum of split-K partials [z][rows][cols] into out (fixed order)
 __global__ void k_ml_reduce_splits(const float* __restrict__ part, int nz, long long count, float* __restrict__ out) {
@@ -875,7 +898,9 @@ static int ml_alloc(mdx_mlp* m, bool training) {
       return rc;
     MDX_HIP(hipMemset(m->U.p, 0, R * ML_F * sizeof(bf16_t)));
     const int maxsplit = std::max(1, m->rows / 512 + 1);
-    if ((rc = m->part.ensure((size_t)maxsplit * ML_H * ML_H))) return rc;
+    // split-K partials, or the column sums' chunks
+    const size_t part = std::max((size_t)maxsplit * ML_H * ML_H, (size_t)COLSUM_ARRAYS * COLSUM_CHUNKS * ML_H);
+    if ((rc = m->part.ensure(part))) return rc;
     for (int e = 0; e < 2; ++e)
       if ((rc = m->net[e].grad.ensure(P_N)) || (rc = m->net[e].m.ensure(P_N)) || (rc = m->net[e].v.ensure(P_N)))
         return rc;
@@ -1241,12 +1266,10 @@ static int ml_weight_grads(mdx_mlp* m, int e, int r0, int r1) {
       (rc = wgrad(ML_H, ML_H, m->B2.p, m->G3.p, m->H2.p, m->DZ16_3.p, N.grad.p + P_W3)))
     return rc;
   // bias and head gradients: column sums (the split-K partial buffer is free again here)
-  const float* cols_in[4] = {m->DZ1.p, m->DZ2.p, m->DZ3.p, m->T4.p};
-  const int cols_out[4] = {P_B1, P_B2, P_B3, P_W4};
-  for (int q = 0; q < 4; ++q) {
-    k_ml_colsum_part<<<COLSUM_CHUNKS, ML_H, 0, st>>>(cols_in[q], r0, r1, ML_H, m->part.p);
-    k_ml_colsum_fin<<<1, ML_H, 0, st>>>(m->part.p, ML_H, N.grad.p + cols_out[q]);
-  }
+  const ColsumArgs cs = {{m->DZ1.p, m->DZ2.p, m->DZ3.p, m->T4.p},
+                         {N.grad.p + P_B1, N.grad.p + P_B2, N.grad.p + P_B3, N.grad.p + P_W4}};
+  k_ml_colsum_part<<<dim3(COLSUM_CHUNKS, COLSUM_ARRAYS), 256, 0, st>>>(cs, r0, r1, m->part.p);
+  k_ml_colsum_fin<<<COLSUM_ARRAYS, ML_H, 0, st>>>(cs, m->part.p);
   k_ml_fill_f32<<<1, 64, 0, st>>>(1, N.grad.p + P_B4, 0.f);
   MDX_LAUNCH_CHECK();
   return 0;
