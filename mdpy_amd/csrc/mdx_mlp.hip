@@ -113,44 +113,6 @@ struct MlAtoms {
   float Lx, Ly, Lz, ix, iy, iz;
 };
 
-// stage up to 64 neighbours of sorted slot s (lane k = base + lane): unit vector, r, element
-struct NbStage {
-  float ux[64], uy[64], uz[64], r[64];
-  int e[64], t[64];
-};
-
-__device__ __forceinline__ void stage_neighbours(const MlAtoms& a, const MlConst& k, const float4& xi,
-                                                 const float4* __restrict__ xq, const unsigned* __restrict__ row,
-                                                 int cnt, int base, NbStage& S) {
-  const int lane = threadIdx.x;
-  const int kk = base + lane;
-  float ux = 0.f, uy = 0.f, uz = 0.f, r = 1e30f;
-  int e = 0, t = 0;
-  if (kk < cnt) {
-    t = nbr_slot(row[kk]);
-    const float4 xj = xq[t];
-    float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-    dx -= a.Lx * rintf(dx * a.ix);
-    dy -= a.Ly * rintf(dy * a.iy);
-    dz -= a.Lz * rintf(dz * a.iz);
-    const float rr = sqrtf(dx * dx + dy * dy + dz * dz);
-    if (rr < k.rd && rr > 0.f) {
-      r = rr;
-      const float ir = __builtin_amdgcn_rcpf(rr);
-      ux = dx * ir;
-      uy = dy * ir;
-      uz = dz * ir;
-    }
-    e = (int)xj.w;
-  }
-  S.ux[lane] = ux;
-  S.uy[lane] = uy;
-  S.uz[lane] = uz;
-  S.r[lane] = r;
-  S.e[lane] = e;
-  S.t[lane] = t;
-}
-
 // ---------------------------------------------------------------- descriptors
 // One wave per atom. Each chunk of 64 list neighbours is first evaluated with one lane per
 // neighbour: the in-range ones (r < r_d) are compacted per element, in list order, into LDS rows
@@ -300,8 +262,8 @@ __global__ __launch_bounds__(64) void k_ml_desc(MlAtoms a, MlConst k, const floa
   }
 }
 
-// dG_i/dr_ij . w for all 96 features of atom i is assembled by the JVP kernel; the force kernel
-// needs the transposed product gG . dG_i/dr_ij for one pair, computed here (gG = dE_i/dG_i,
+// The JVP kernel has dG_i/dr_ij . w for all 96 features of atom i; the force kernel needs the
+// transposed product gG . dG_i/dr_ij for one pair, computed here (gG = dE_i/dG_i,
 // tt = the atom's moment tensors, both in LDS).
 // Radial terms: only the 2 ML_RWIN + 1 Gaussians centred nearest r. The centres are dmu apart and
 // eta dmu^2 = 1/2, so a Gaussian k centres away weighs exp(-k^2/2): the terms left out
@@ -438,71 +400,147 @@ __global__ __launch_bounds__(64) void k_ml_force(MlAtoms a, MlConst k, const flo
 }
 
 // ---------------------------------------------------------------- descriptor JVP (training)
-// U[row][f] = rstd_f * sum_j (w_j - w_i) . dG_if/dr_ij, one wave per atom, lane per feature
-// (f = lane and lane + 64 < 96), neighbours staged 64 at a time.
+// U[row][f] = rstd_f * dG_if along the displacement rates w: r_ij changes at w_j - w_i.
+// The descriptors' own walk, differentiated: with the rate of r, q = u . (w_j - w_i), and of the unit
+// vector, u' = (w_j - w_i - q u) / r, a radial Gaussian changes at ex (dfc - 2 eta (r - mu) fc) q and
+// a moment component at g' q mono + g mono'(u, u'); the angular features are squares of moments, so
+// their rate is 2 sum_c weight_c T_c T'_c from the stored T. As in the descriptor kernel, one lane
+// per neighbour prepares a row (compacted per element, in list order), then lanes are features and
+// walk the rows: per row one exponential per lane pair and four products, where every lane walked every
+// neighbour with its own exponentials and tensor contractions before. 23,328 atoms: 435 -> 143 us.
 __global__ __launch_bounds__(64) void k_ml_jvp(MlAtoms a, MlConst k, const float4* __restrict__ xq,
                                               const int* __restrict__ sorted_orig, const int* __restrict__ nbr_count,
                                               const unsigned* __restrict__ nbr_list, const int* __restrict__ row_of,
                                               const float* __restrict__ T, const double* __restrict__ w,
                                               const float* __restrict__ rstd, bf16_t* __restrict__ U) {
-  __shared__ NbStage S;
-  __shared__ float tt[ML_T];
-  __shared__ float dw[64][3];
+  __shared__ float4 rq[64];                           // r, fc q, dfc q
+  __shared__ float2 ga[64][ML_CH];                    // channel weight g and its rate
+  __shared__ float2 mo[64][ML_MOM + 1];               // monomials and their rates
+  __shared__ float sm[ML_T];
   const int s = blockIdx.x;
   const int lane = threadIdx.x;
   const float4 xi = xq[s];
   const int o = sorted_orig[s];
   const int row = row_of[o];
-  for (int c = lane; c < ML_T; c += 64) tt[c] = T[(long long)row * ML_T + c];
-  const float wi[3] = {(float)w[3 * o], (float)w[3 * o + 1], (float)w[3 * o + 2]};
   const int cnt = nbr_count[s];
   const unsigned* lrow = nbr_list + (long long)s * a.cap;
-  float acc[2] = {0.f, 0.f};
+  const float wi[3] = {(float)w[3 * o], (float)w[3 * o + 1], (float)w[3 * o + 2]};
+  const int half = lane >> 5;
+  const float mu = k.rad_mu0 + (float)(lane & 31) * k.rad_dmu;  // this lane's Gaussian centre
+  const int ch0 = lane / ML_MOM, cp0 = lane % ML_MOM;
+  const int c1 = 64 + (lane & 15);
+  const int ch1 = c1 / ML_MOM, cp1 = c1 % ML_MOM;
+  const bool has1 = lane < 16;
+  float rad[2] = {0.f, 0.f};  // per element: Gaussian lane & 31 over this lane's half of the rows
+  float m0[2] = {0.f, 0.f}, m1[2] = {0.f, 0.f};
   for (int base = 0; base < cnt; base += 64) {
-    stage_neighbours(a, k, xi, xq, lrow, cnt, base, S);
-    if (base + lane < cnt) {
-      const int oj = sorted_orig[S.t[lane]];
-      for (int d = 0; d < 3; ++d) dw[lane][d] = (float)w[3 * oj + d] - wi[d];
+    const int kk = base + lane;
+    float ux = 0.f, uy = 0.f, uz = 0.f, r = 1e30f, ir = 0.f;
+    int e = 0, t = 0;
+    if (kk < cnt) {
+      t = nbr_slot(lrow[kk]);
+      const float4 xj = xq[t];
+      float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+      dx -= a.Lx * rintf(dx * a.ix);
+      dy -= a.Ly * rintf(dy * a.iy);
+      dz -= a.Lz * rintf(dz * a.iz);
+      const float rr2 = sqrtf(dx * dx + dy * dy + dz * dz);
+      if (rr2 < k.rd && rr2 > 0.f) {
+        r = rr2;
+        ir = __builtin_amdgcn_rcpf(rr2);
+        ux = dx * ir;
+        uy = dy * ir;
+        uz = dz * ir;
+      }
+      e = (int)xj.w;
     }
-    __syncthreads();
-    const int m = min(64, cnt - base);
-    for (int jj = 0; jj < m; ++jj) {
-      const float r = S.r[jj];
-      if (r >= k.rd) continue;
-      const int e = S.e[jj];
-      const float ux = S.ux[jj], uy = S.uy[jj], uz = S.uz[jj];
-      const float wx = dw[jj][0], wy = dw[jj][1], wz = dw[jj][2];
-      const float uw = ux * wx + uy * wy + uz * wz;
+    const bool keep = r < k.rd;
+    const unsigned long long b0 = __ballot(keep && e == 0), b1 = __ballot(keep && e != 0);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int n0 = __popcll(b0), n1 = __popcll(b1);
+    if (keep) {
+      const int slot = e == 0 ? __popcll(b0 & below) : 63 - __popcll(b1 & below);
+      const int oj = sorted_orig[t];
+      const float wx = (float)w[3 * oj] - wi[0], wy = (float)w[3 * oj + 1] - wi[1], wz = (float)w[3 * oj + 2] - wi[2];
+      const float q = ux * wx + uy * wy + uz * wz;
+      const float px = (wx - q * ux) * ir, py = (wy - q * uy) * ir, pz = (wz - q * uz) * ir;
       float fc, dfc;
       cutoff_fc(k, r, &fc, &dfc);
+      rq[slot] = make_float4(r, fc * q, dfc * q, 0.f);
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int f = lane + 64 * q;
-        if (f >= ML_F || f / ML_PER != e) continue;
-        const int loc = f % ML_PER;
-        if (loc < ML_RAD) {
-          const float dr = r - (k.rad_mu0 + loc * k.rad_dmu);
-          const float ex = __expf(-k.rad_eta * dr * dr);
-          acc[q] += ex * (dfc - 2.f * k.rad_eta * dr * fc) * uw;
-        } else {
-          const int ch = (loc - ML_RAD) >> 2, l = (loc - ML_RAD) & 3;
-          const float dn = r - k.ang_nu[ch];
-          const float ex = __expf(-k.ang_eta * dn * dn);
-          const float g = ex * fc, dg = ex * (dfc - 2.f * k.ang_eta * dn * fc);
-          float sl[4], vl[4][3];
-          contract(tt + e * 80 + ch * 20, ux, uy, uz, sl, vl);
-          const float vw = vl[l][0] * wx + vl[l][1] * wy + vl[l][2] * wz;
-          const float vu = vl[l][0] * ux + vl[l][1] * uy + vl[l][2] * uz;
-          acc[q] += 2.f * (dg * sl[l] * uw + g * (vw - vu * uw) / r);
-        }
+      for (int ch = 0; ch < ML_CH; ++ch) {
+        const float dn = r - k.ang_nu[ch];
+        const float ex = __expf(-k.ang_eta * dn * dn);
+        ga[slot][ch] = make_float2(ex * fc, ex * (dfc - 2.f * k.ang_eta * dn * fc) * q);
       }
+      const float xx = ux * ux, yy = uy * uy, zz = uz * uz, xy = ux * uy, xz = ux * uz, yz = uy * uz;
+      const float dxx = 2.f * ux * px, dyy = 2.f * uy * py, dzz = 2.f * uz * pz;
+      const float dxy = px * uy + ux * py, dxz = px * uz + ux * pz, dyz = py * uz + uy * pz;
+      float2* mm = mo[slot];
+      mm[0] = make_float2(1.f, 0.f);
+      mm[1] = make_float2(ux, px);
+      mm[2] = make_float2(uy, py);
+      mm[3] = make_float2(uz, pz);
+      mm[4] = make_float2(xx, dxx);
+      mm[5] = make_float2(xy, dxy);
+      mm[6] = make_float2(xz, dxz);
+      mm[7] = make_float2(yy, dyy);
+      mm[8] = make_float2(yz, dyz);
+      mm[9] = make_float2(zz, dzz);
+      mm[10] = make_float2(xx * ux, dxx * ux + xx * px);
+      mm[11] = make_float2(xx * uy, dxx * uy + xx * py);
+      mm[12] = make_float2(xx * uz, dxx * uz + xx * pz);
+      mm[13] = make_float2(ux * yy, px * yy + ux * dyy);
+      mm[14] = make_float2(xy * uz, dxy * uz + xy * pz);
+      mm[15] = make_float2(ux * zz, px * zz + ux * dzz);
+      mm[16] = make_float2(yy * uy, dyy * uy + yy * py);
+      mm[17] = make_float2(yy * uz, dyy * uz + yy * pz);
+      mm[18] = make_float2(uy * zz, py * zz + uy * dzz);
+      mm[19] = make_float2(zz * uz, dzz * uz + zz * pz);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int el = 0; el < 2; ++el) {
+      const int n = el == 0 ? n0 : n1;
+      float acc = 0.f;
+      for (int jj = half; jj < n; jj += 2) {  // radial: two rows per step
+        const float4 v = rq[el == 0 ? jj : 63 - jj];
+        const float d = v.x - mu;
+        acc += __expf(-k.rad_eta * d * d) * (v.z - 2.f * k.rad_eta * d * v.y);
+      }
+      rad[el] += acc;
+      float a0 = 0.f, a1 = 0.f;
+#pragma unroll 4
+      for (int jj = 0; jj < n; ++jj) {  // moments: one row per step
+        const int q = el == 0 ? jj : 63 - jj;
+        const float2 g0 = ga[q][ch0], x0 = mo[q][cp0], g1 = ga[q][ch1], x1 = mo[q][cp1];
+        a0 += g0.y * x0.x + g0.x * x0.y;
+        a1 += g1.y * x1.x + g1.x * x1.y;
+      }
+      m0[el] += a0;
+      m1[el] += a1;
     }
     __syncthreads();
   }
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int f = lane + 64 * q;
-    if (f < ML_F) U[(long long)row * ML_F + f] = f2bf(acc[q] * rstd[f]);
+  for (int el = 0; el < 2; ++el) {
+    sm[el * 80 + lane] = m0[el] * T[(long long)row * ML_T + el * 80 + lane];
+    if (has1) sm[el * 80 + c1] = m1[el] * T[(long long)row * ML_T + el * 80 + c1];
+  }
+  __syncthreads();
+  {
+    const float g0 = rad[0] + __shfl_xor(rad[0], 32, 64), g1 = rad[1] + __shfl_xor(rad[1], 32, 64);
+    const int f = half * ML_PER + (lane & 31);
+    U[(long long)row * ML_F + f] = f2bf((half == 0 ? g0 : g1) * rstd[f]);
+  }
+  if (lane < 32) {
+    const int e = lane >> 4, ch = (lane >> 2) & 3, l = lane & 3;
+    const float* t = sm + e * 80 + ch * 20;
+    float p = 0.f;
+    for (int c = 0; c < ML_MOM; ++c)
+      if (mom_l(c) == l) p += mom_weight(c) * t[c];
+    const int f = e * ML_PER + ML_RAD + ch * ML_L + l;
+    U[(long long)row * ML_F + f] = f2bf(2.f * p * rstd[f]);
   }
 }
 
