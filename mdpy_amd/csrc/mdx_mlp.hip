@@ -550,17 +550,16 @@ __global__ __launch_bounds__(64) void k_ml_jvp(MlAtoms a, MlConst k, const float
 // each wave a 32x32 sub-tile on gfx950's v_mfma_f32_32x32x16_bf16 (lane l: A row l%32, k
 // 8(l/32)..+7; B col l%32, same k; D row 8(i/4) + 4(l/32) + i%4, col l%32 for accumulator i).
 // Rows >= row_split use the second operand B1 / bias1 (the second element's weights).
-enum { EPI_F32 = 0, EPI_F32_ACC = 1, EPI_BIAS_SILU = 2, EPI_MUL_S = 3 };
+enum { EPI_F32 = 0, EPI_BIAS_SILU = 1, EPI_MUL_S = 2 };
 struct GemmArgs {
   int M, N, K;
   const bf16_t* A;
-  long long a_m, a_k;
+  long long a_m;              // A's row stride (its k index is contiguous)
   const bf16_t* B0;
   const bf16_t* B1;
   long long b_k, b_n;
   int row_split;
-  int kchunk;                 // K per blockIdx.z (split-K)
-  float* C;                   // EPI_F32*: partials [z][M][ldc]; EPI_BIAS_SILU: Z (+bias); EPI_MUL_S: raw product
+  float* C;                   // EPI_F32: the product; EPI_BIAS_SILU: Z (+bias); EPI_MUL_S: raw product
   long long ldc;
   const float* bias0;
   const float* bias1;
@@ -590,33 +589,27 @@ __device__ __forceinline__ void load8(const bf16_t* __restrict__ base, long long
   }
 }
 
-// A_KC: A's k index is contiguous in memory (a_k == 1), else its row index is (a_m == 1);
-// B_KC: B's k index is contiguous (b_k == 1), else its column index is (b_n == 1). Each k-step
+// A's k index is contiguous in memory; B_KC: so is B's (b_k == 1), else its column index is (b_n == 1). Each k-step
 // every lane moves one 8-element vector of A and one of B into LDS, where both tiles are
 // stored k-contiguous per row / column so each MFMA operand is one 8-byte LDS read.
-template <bool A_KC, bool B_KC>
+template <bool B_KC>
 __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g, int epi) {
   __shared__ __attribute__((aligned(16))) bf16_t As[ML_TILE][GK + 8];
   __shared__ __attribute__((aligned(16))) bf16_t Bs[ML_TILE][GK + 8];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
   const int row0 = blockIdx.y * ML_TILE, col0 = blockIdx.x * ML_TILE;
-  const int kb = blockIdx.z * g.kchunk, ke = min(g.K, kb + g.kchunk);
+  const int ke = g.K;
   const bool second = row0 >= g.row_split;
   const bf16_t* B = second ? g.B1 : g.B0;
   f32x16 acc;
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-  // this lane's tile vectors: A (row ra / k offset ka, or k ka / rows ra..+7), B likewise
-  const int ra = A_KC ? (tid >> 2) : (tid & 7) * 8, ka = A_KC ? (tid & 3) * 8 : (tid >> 3);
+  // this lane's tile vectors: A (row ra, k offset ka), B likewise or k kbv / columns rb..+7
+  const int ra = tid >> 2, ka = (tid & 3) * 8;
   const int rb = B_KC ? (tid >> 2) : (tid & 7) * 8, kbv = B_KC ? (tid & 3) * 8 : (tid >> 3);
   auto fetch = [&](int k0, bf16_t* va, bf16_t* vb) {
-    if (A_KC) {
-      const int m = row0 + ra, kx = k0 + ka;
-      load8(g.A, (long long)m * g.a_m + kx, 1, m < g.M ? max(0, min(8, ke - kx)) : 0, va);
-    } else {
-      const int m = row0 + ra, kx = k0 + ka;
-      load8(g.A, (long long)kx * g.a_k + m, 1, kx < ke ? max(0, min(8, g.M - m)) : 0, va);
-    }
+    const int m = row0 + ra, ax = k0 + ka;
+    load8(g.A, (long long)m * g.a_m + ax, 1, m < g.M ? max(0, min(8, ke - ax)) : 0, va);
     if (B_KC) {
       const int n = col0 + rb, kx = k0 + kbv;
       load8(B, (long long)n * g.b_n + kx, 1, n < g.N ? max(0, min(8, ke - kx)) : 0, vb);
@@ -626,12 +619,11 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g, int epi) {
     }
   };
   bf16_t va[8], vb[8];
-  if (kb < ke) fetch(kb, va, vb);
-  for (int k0 = kb; k0 < ke; k0 += GK) {
+  fetch(0, va, vb);
+  for (int k0 = 0; k0 < ke; k0 += GK) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if (A_KC) As[ra][ka + i] = va[i];
-      else As[ra + i][ka] = va[i];
+      As[ra][ka + i] = va[i];
       if (B_KC) Bs[rb][kbv + i] = vb[i];
       else Bs[rb + i][kbv] = vb[i];
     }
@@ -657,9 +649,7 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g, int epi) {
     if (m >= g.M || n >= g.N) continue;
     const float v = acc[i];
     if (epi == EPI_F32) {
-      g.C[((long long)blockIdx.z * g.M + m) * g.ldc + n] = v;
-    } else if (epi == EPI_F32_ACC) {
-      g.C[((long long)blockIdx.z * g.M + m) * g.ldc + n] += v;
+      g.C[(long long)m * g.ldc + n] = v;
     } else if (epi == EPI_BIAS_SILU) {
       const float z = v + (second ? g.bias1 : g.bias0)[n];
       const float sg = 1.f / (1.f + __expf(-z));
@@ -793,14 +783,113 @@ __global__ __launch_bounds__(ML_H) void k_ml_colsum_fin(ColsumArgs a, const floa
   for (int k = 0; k < COLSUM_CHUNKS; ++k) s += part[k * ML_H + c];
   a.out[blockIdx.x][c] = s;
 }
-// sum of split-K partials [z][rows][cols] into out (fixed order)
-__global__ void k_ml_reduce_splits(const float* __restrict__ part, int nz, long long count, float* __restrict__ out) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  float s = 0.f;
-  for (int z = 0; z < nz; ++z) s += part[(long long)z * count + i];
-  out[i] = s;
+// Weight gradients: W_l' = P_l^T Q_l + R_l^T S_l over an element's rows, for the three layers of both
+// element networks in one launch. blockIdx.x is one of the 64x64 tiles of the three matrices,
+// blockIdx.y a share of an element's rows; the shares' float32 partial tiles are added in order by
+// k_ml_wgrad_reduce. Both operands are row-major with the rows summed over, so a lane loads 8 columns
+// of two rows (16 B each) and writes them to LDS as pairs of rows, k-contiguous per column: one
+// 16-byte LDS read per MFMA operand. Load latency bound (16 steps of 64 rows a share): the twelve
+// products ran one after the other before, 240 or 480 workgroups each, and re-read the partial
+// sums of the first product to add the second. 23,328 rows (us): 304 + 44 (12 products, 6 sums) -> 75 + 12.
+#define WG_K 64
+#define WG_ROWS 512  // rows of a share, at least
+#define WG_SHARES 48 // of an element, at most
+#define WG_TILES1 ((ML_F + 63) / 64 * (ML_H / 64))
+#define WG_TILES (WG_TILES1 + 2 * (ML_H / 64) * (ML_H / 64))
+#define WG_N (ML_F * ML_H + 2 * ML_H * ML_H)  // weights of a network without biases and head
+struct WgradArgs {
+  const bf16_t* A[3][2];  // P_l, R_l [row][M_l]
+  const bf16_t* B[3][2];  // Q_l, S_l [row][ML_H]
+  int r0[2], r1[2];       // rows of each element
+  int rows;               // of a share
+  int shares0;            // shares of element 0 (blockIdx.y below it)
+  float* part;            // [share][WG_N]
+  float* out[2];
+};
+static int wgrad_rows(int n) { return std::max(WG_ROWS, div_up(n, WG_SHARES * WG_K) * WG_K); }
+__device__ __forceinline__ void wgrad_tile(int tile, int* l, int* M, int* row0, int* col0, int* base) {
+  const int k = tile - WG_TILES1;
+  *l = k < 0 ? 0 : 1 + k / ((ML_H / 64) * (ML_H / 64));
+  const int q = k < 0 ? tile : k % ((ML_H / 64) * (ML_H / 64));
+  *M = k < 0 ? ML_F : ML_H;
+  *row0 = q / (ML_H / 64) * 64;
+  *col0 = q % (ML_H / 64) * 64;
+  *base = *l == 0 ? 0 : ML_F * ML_H + (*l - 1) * ML_H * ML_H;
 }
+__global__ __launch_bounds__(256) void k_ml_wgrad(WgradArgs g) {
+  __shared__ __attribute__((aligned(16))) bf16_t As[64][WG_K + 8];
+  __shared__ __attribute__((aligned(16))) bf16_t Bs[64][WG_K + 8];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wm = w >> 1, wn = w & 1;
+  int l, M, row0, col0, base;
+  wgrad_tile(blockIdx.x, &l, &M, &row0, &col0, &base);
+  const int el = (int)blockIdx.y < g.shares0 ? 0 : 1;
+  const int kb = g.r0[el] + ((int)blockIdx.y - (el ? g.shares0 : 0)) * g.rows, ke = min(g.r1[el], kb + g.rows);
+  const int c8 = (tid & 7) * 8, kp = tid >> 3;  // this lane's 8 columns and pair of rows
+  const bool am = row0 + c8 < M;                // M is a multiple of 8
+  f32x16 acc;
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 va[2], vb[2];
+  // step s: rows kb + 64 (s / 2).. of product s % 2
+  auto fetch = [&](int s) {
+    const bf16_t* __restrict__ A = g.A[l][s & 1];
+    const bf16_t* __restrict__ B = g.B[l][s & 1];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int k = kb + (s >> 1) * WG_K + 2 * kp + u;
+      va[u] = am && k < ke ? *(const u32x4*)(A + (long long)k * M + row0 + c8) : zero;
+      vb[u] = k < ke ? *(const u32x4*)(B + (long long)k * ML_H + col0 + c8) : zero;
+    }
+  };
+  const int steps = 2 * ((ke - kb + WG_K - 1) / WG_K);
+  fetch(0);
+  for (int s = 0; s < steps; ++s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *(unsigned*)&As[c8 + 2 * i][2 * kp] = (va[0][i] & 0xffffu) | (va[1][i] << 16);
+      *(unsigned*)&As[c8 + 2 * i + 1][2 * kp] = (va[0][i] >> 16) | (va[1][i] & 0xffff0000u);
+      *(unsigned*)&Bs[c8 + 2 * i][2 * kp] = (vb[0][i] & 0xffffu) | (vb[1][i] << 16);
+      *(unsigned*)&Bs[c8 + 2 * i + 1][2 * kp] = (vb[0][i] >> 16) | (vb[1][i] & 0xffff0000u);
+    }
+    __syncthreads();
+    if (s + 1 < steps) fetch(s + 1);  // in flight during the MFMAs
+#pragma unroll
+    for (int ks = 0; ks < WG_K; ks += 16) {  // operand layout as in k_gemm_bf16
+      const int kq = ks + (lane >> 5) * 8;
+      const bf16x8 av = *(const bf16x8*)&As[wm * 32 + (lane & 31)][kq];
+      const bf16x8 bv = *(const bf16x8*)&Bs[wn * 32 + (lane & 31)][kq];
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
+    }
+    __syncthreads();
+  }
+  float* __restrict__ out = g.part + (long long)blockIdx.y * WG_N + base;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int m = row0 + wm * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3), n = col0 + wn * 32 + (lane & 31);
+    if (m < M) out[(long long)m * ML_H + n] = acc[i];
+  }
+}
+// element blockIdx.y: the shares' partial gradients added in order (a float4 per lane)
+__global__ __launch_bounds__(256) void k_ml_wgrad_reduce(WgradArgs g, int shares1) {
+  const int i = 4 * (blockIdx.x * 256 + threadIdx.x), el = blockIdx.y;
+  if (i >= WG_N) return;
+  const int s0 = el ? g.shares0 : 0, n = el ? shares1 : g.shares0;
+  if (n == 0) return;
+  const float* __restrict__ in = g.part + (long long)s0 * WG_N + i;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 8
+  for (int z = 0; z < n; ++z) {
+    const float4 v = *(const float4*)(in + (long long)z * WG_N);
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  const int b2 = ML_F * ML_H, b3 = b2 + ML_H * ML_H;
+  *(float4*)(g.out[el] + (i < b2 ? P_W1 + i : (i < b3 ? P_W2 + i - b2 : P_W3 + i - b3))) = s;
+}
+static_assert(WG_N % 4 == 0 && ML_F % 8 == 0 && P_W1 % 4 == 0 && P_W2 % 4 == 0 && P_W3 % 4 == 0, "16-byte accesses");
 // force error and its loss weight: err = F_hat - F_ref, w = -(2/3N) err, loss += sum err^2/(3N)
 __global__ void k_ml_loss(int n, const long long* __restrict__ ffix, const double* __restrict__ fref,
                           double* __restrict__ w, long long* __restrict__ lslot) {
@@ -935,9 +1024,10 @@ static int ml_alloc(mdx_mlp* m, bool training) {
         (rc = m->DZ16_3.ensure(R * ML_H)) || (rc = m->w.ensure(3 * (size_t)m->n)))
       return rc;
     MDX_HIP(hipMemset(m->U.p, 0, R * ML_F * sizeof(bf16_t)));
-    const int maxsplit = std::max(1, m->rows / 512 + 1);
-    // split-K partials, or the column sums' chunks
-    const size_t part = std::max((size_t)maxsplit * ML_H * ML_H, (size_t)COLSUM_ARRAYS * COLSUM_CHUNKS * ML_H);
+    // weight gradients' partials, or the column sums' chunks
+    const int rows = wgrad_rows(std::max(m->nO, m->nH));
+    const size_t shares = div_up(m->nO, rows) + div_up(m->nH, rows);
+    const size_t part = std::max(shares * WG_N, (size_t)COLSUM_ARRAYS * COLSUM_CHUNKS * ML_H);
     if ((rc = m->part.ensure(part))) return rc;
     for (int e = 0; e < 2; ++e)
       if ((rc = m->net[e].grad.ensure(P_N)) || (rc = m->net[e].m.ensure(P_N)) || (rc = m->net[e].v.ensure(P_N)))
@@ -1119,23 +1209,21 @@ extern "C" int mdx_mlp_set_norm(mdx_mlp* m, const float* h_mean, const float* h_
 }
 
 // ---- GEMM launcher
-static int gemm(mdx_mlp* m, int epi, int M, int N, int K, const bf16_t* A, long long a_m, long long a_k,
-                const bf16_t* B0, const bf16_t* B1, long long b_k, long long b_n, int row_split, float* C,
-                long long ldc, int splits = 1, const float* bias0 = nullptr, const float* bias1 = nullptr,
-                bf16_t* H = nullptr, float* S = nullptr, float* DD = nullptr) {
+static int gemm(mdx_mlp* m, int epi, int M, int N, int K, const bf16_t* A, long long a_m, const bf16_t* B0,
+                const bf16_t* B1, long long b_k, long long b_n, int row_split, float* C, long long ldc,
+                const float* bias0 = nullptr, const float* bias1 = nullptr, bf16_t* H = nullptr, float* S = nullptr,
+                float* DD = nullptr) {
   GemmArgs g;
   g.M = M;
   g.N = N;
   g.K = K;
   g.A = A;
   g.a_m = a_m;
-  g.a_k = a_k;
   g.B0 = B0;
   g.B1 = B1 ? B1 : B0;
   g.b_k = b_k;
   g.b_n = b_n;
   g.row_split = row_split;
-  g.kchunk = div_up(div_up(K, splits), GK) * GK;
   g.C = C;
   g.ldc = ldc;
   g.bias0 = bias0;
@@ -1143,14 +1231,11 @@ static int gemm(mdx_mlp* m, int epi, int M, int N, int K, const bf16_t* A, long 
   g.H = H;
   g.S = S;
   g.DD = DD;
-  dim3 grid(div_up(N, ML_TILE), div_up(M, ML_TILE), splits);
-  MDX_CHECK((a_k == 1 || a_m == 1) && (b_k == 1 || b_n == 1), MDX_ERR_INVALID,
-            "gemm: one stride of each operand must be 1");
+  dim3 grid(div_up(N, ML_TILE), div_up(M, ML_TILE));
+  MDX_CHECK(b_k == 1 || b_n == 1, MDX_ERR_INVALID, "gemm: one stride of B must be 1");
   hipStream_t st = m->host->stream;
-  if (a_k == 1 && b_k == 1) k_gemm_bf16<true, true><<<grid, 256, 0, st>>>(g, epi);
-  else if (a_k == 1) k_gemm_bf16<true, false><<<grid, 256, 0, st>>>(g, epi);
-  else if (b_k == 1) k_gemm_bf16<false, true><<<grid, 256, 0, st>>>(g, epi);
-  else k_gemm_bf16<false, false><<<grid, 256, 0, st>>>(g, epi);
+  if (b_k == 1) k_gemm_bf16<true><<<grid, 256, 0, st>>>(g, epi);
+  else k_gemm_bf16<false><<<grid, 256, 0, st>>>(g, epi);
   MDX_LAUNCH_CHECK();
   return 0;
 }
@@ -1169,22 +1254,22 @@ static int ml_forward_backward(mdx_mlp* m, long long* eslot, bool keep_training_
   float* DD1 = keep_training_state ? m->D1.p : nullptr;
   float* DD2 = keep_training_state ? m->D2.p : nullptr;
   float* DD3 = keep_training_state ? m->D3.p : nullptr;
-  if ((rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_F, m->X.p, ML_F, 1, N0.w1.p, N1.w1.p, ML_H, 1, rs, nullptr, ML_H, 1,
+  if ((rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_F, m->X.p, ML_F, N0.w1.p, N1.w1.p, ML_H, 1, rs, nullptr, ML_H,
                  N0.p.p + P_B1, N1.p.p + P_B1, m->H1.p, m->S1.p, DD1)) ||
-      (rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_H, m->H1.p, ML_H, 1, N0.w2.p, N1.w2.p, ML_H, 1, rs, nullptr, ML_H, 1,
+      (rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_H, m->H1.p, ML_H, N0.w2.p, N1.w2.p, ML_H, 1, rs, nullptr, ML_H,
                  N0.p.p + P_B2, N1.p.p + P_B2, m->H2.p, m->S2.p, DD2)) ||
-      (rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_H, m->H2.p, ML_H, 1, N0.w3.p, N1.w3.p, ML_H, 1, rs, nullptr, ML_H, 1,
+      (rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_H, m->H2.p, ML_H, N0.w3.p, N1.w3.p, ML_H, 1, rs, nullptr, ML_H,
                  N0.p.p + P_B3, N1.p.p + P_B3, m->H3.p, m->S3.p, DD3)))
     return rc;
   k_ml_head<<<div_up(R, HEAD_ROWS), 256, 0, st>>>(R, rs, m->H3.p, m->S3.p, N0.p.p, N1.p.p, m->atom_of_row.p,
                                                    m->G3.p, nullptr, eslot);
   MDX_LAUNCH_CHECK();
   // input gradient: G2 = (G3 W3^T) * S2, G1 = (G2 W2^T) * S1, GX = G1 W1^T
-  if ((rc = gemm(m, EPI_MUL_S, R, ML_H, ML_H, m->G3.p, ML_H, 1, N0.w3.p, N1.w3.p, 1, ML_H, rs,
-                 keep_training_state ? m->HB2.p : nullptr, ML_H, 1, nullptr, nullptr, m->G2.p, m->S2.p)) ||
-      (rc = gemm(m, EPI_MUL_S, R, ML_H, ML_H, m->G2.p, ML_H, 1, N0.w2.p, N1.w2.p, 1, ML_H, rs,
-                 keep_training_state ? m->HB1.p : nullptr, ML_H, 1, nullptr, nullptr, m->G1.p, m->S1.p)) ||
-      (rc = gemm(m, EPI_F32, R, ML_F, ML_H, m->G1.p, ML_H, 1, N0.w1.p, N1.w1.p, 1, ML_H, rs, m->GX.p, ML_F)))
+  if ((rc = gemm(m, EPI_MUL_S, R, ML_H, ML_H, m->G3.p, ML_H, N0.w3.p, N1.w3.p, 1, ML_H, rs,
+                 keep_training_state ? m->HB2.p : nullptr, ML_H, nullptr, nullptr, m->G2.p, m->S2.p)) ||
+      (rc = gemm(m, EPI_MUL_S, R, ML_H, ML_H, m->G2.p, ML_H, N0.w2.p, N1.w2.p, 1, ML_H, rs,
+                 keep_training_state ? m->HB1.p : nullptr, ML_H, nullptr, nullptr, m->G1.p, m->S1.p)) ||
+      (rc = gemm(m, EPI_F32, R, ML_F, ML_H, m->G1.p, ML_H, N0.w1.p, N1.w1.p, 1, ML_H, rs, m->GX.p, ML_F)))
     return rc;
   return 0;
 }
@@ -1272,43 +1357,41 @@ extern "C" int mdx_mlp_adam_config(mdx_mlp* m, double beta1, double beta2, doubl
   return 0;
 }
 
-// weight gradients of one element network from the rows [r0, r1)
-static int ml_weight_grads(mdx_mlp* m, int e, int r0, int r1) {
+// Gradients of both element networks (rows [0, nO) and [rowsO, rowsO + nH)): dW1 = U^T G1 + X^T dz1,
+// dW2 = B1^T G2 + H1^T dz2, dW3 = B2^T G3 + H2^T dz3, biases and head from column sums.
+static int ml_weight_grads(mdx_mlp* m) {
   hipStream_t st = m->host->stream;
-  MlNet& N = m->net[e];
-  const int K = r1 - r0;
-  if (K <= 0) {
-    MDX_HIP(hipMemsetAsync(N.grad.p, 0, P_N * sizeof(float), st));
-    return 0;
+  WgradArgs g{};
+  const bf16_t *A[3][2] = {{m->U.p, m->X.p}, {m->B1.p, m->H1.p}, {m->B2.p, m->H2.p}};
+  const bf16_t *B[3][2] = {{m->G1.p, m->DZ16_1.p}, {m->G2.p, m->DZ16_2.p}, {m->G3.p, m->DZ16_3.p}};
+  for (int l = 0; l < 3; ++l)
+    for (int q = 0; q < 2; ++q) {
+      g.A[l][q] = A[l][q];
+      g.B[l][q] = B[l][q];
+    }
+  int shares[2];
+  g.rows = wgrad_rows(std::max(m->nO, m->nH));
+  for (int e = 0; e < 2; ++e) {
+    g.r0[e] = e ? m->rowsO : 0;
+    g.r1[e] = g.r0[e] + (e ? m->nH : m->nO);
+    shares[e] = div_up(g.r1[e] - g.r0[e], g.rows);
+    g.out[e] = m->net[e].grad.p;
+    if (shares[e] == 0) MDX_HIP(hipMemsetAsync(m->net[e].grad.p, 0, P_N * sizeof(float), st));
   }
-  const int splits = std::max(1, std::min(K / 512, (int)(m->part.n / (ML_H * ML_H))));
-  int rc;
-  auto wgrad = [&](int M, int Nn, const bf16_t* At, const bf16_t* Bm, const bf16_t* At2, const bf16_t* Bm2,
-                   float* out) -> int {
-    // out (M x Nn) = At^T Bm + At2^T Bm2, At rows = atoms (row-major [row][M]), Bm [row][Nn]
-    int r;
-    if ((r = gemm(m, EPI_F32, M, Nn, K, At + (long long)r0 * M, 1, M, Bm + (long long)r0 * Nn, nullptr, Nn, 1,
-                  1 << 30, m->part.p, Nn, splits)))
-      return r;
-    if ((r = gemm(m, EPI_F32_ACC, M, Nn, K, At2 + (long long)r0 * M, 1, M, Bm2 + (long long)r0 * Nn, nullptr, Nn, 1,
-                  1 << 30, m->part.p, Nn, splits)))
-      return r;
-    const long long cnt = (long long)M * Nn;
-    k_ml_reduce_splits<<<div_up(cnt, 256), 256, 0, st>>>(m->part.p, splits, cnt, out);
-    MDX_LAUNCH_CHECK();
-    return 0;
-  };
-  // dW1 = U^T G1 + X^T dz1 ; dW2 = B1^T G2 + H1^T dz2 ; dW3 = B2^T G3 + H2^T dz3
-  if ((rc = wgrad(ML_F, ML_H, m->U.p, m->G1.p, m->X.p, m->DZ16_1.p, N.grad.p + P_W1)) ||
-      (rc = wgrad(ML_H, ML_H, m->B1.p, m->G2.p, m->H1.p, m->DZ16_2.p, N.grad.p + P_W2)) ||
-      (rc = wgrad(ML_H, ML_H, m->B2.p, m->G3.p, m->H2.p, m->DZ16_3.p, N.grad.p + P_W3)))
-    return rc;
-  // bias and head gradients: column sums (the split-K partial buffer is free again here)
-  const ColsumArgs cs = {{m->DZ1.p, m->DZ2.p, m->DZ3.p, m->T4.p},
-                         {N.grad.p + P_B1, N.grad.p + P_B2, N.grad.p + P_B3, N.grad.p + P_W4}};
-  k_ml_colsum_part<<<dim3(COLSUM_CHUNKS, COLSUM_ARRAYS), 256, 0, st>>>(cs, r0, r1, m->part.p);
-  k_ml_colsum_fin<<<COLSUM_ARRAYS, ML_H, 0, st>>>(cs, m->part.p);
-  k_ml_fill_f32<<<1, 64, 0, st>>>(1, N.grad.p + P_B4, 0.f);
+  g.shares0 = shares[0];
+  g.part = m->part.p;
+  k_ml_wgrad<<<dim3(WG_TILES, shares[0] + shares[1]), 256, 0, st>>>(g);
+  k_ml_wgrad_reduce<<<dim3(div_up(WG_N / 4, 256), 2), 256, 0, st>>>(g, shares[1]);
+  MDX_LAUNCH_CHECK();
+  for (int e = 0; e < 2; ++e) {
+    if (shares[e] == 0) continue;
+    float* gr = m->net[e].grad.p;
+    const ColsumArgs cs = {{m->DZ1.p, m->DZ2.p, m->DZ3.p, m->T4.p}, {gr + P_B1, gr + P_B2, gr + P_B3, gr + P_W4}};
+    // the partial buffer is free again here
+    k_ml_colsum_part<<<dim3(COLSUM_CHUNKS, COLSUM_ARRAYS), 256, 0, st>>>(cs, g.r0[e], g.r1[e], m->part.p);
+    k_ml_colsum_fin<<<COLSUM_ARRAYS, ML_H, 0, st>>>(cs, m->part.p);
+    k_ml_fill_f32<<<1, 64, 0, st>>>(1, gr + P_B4, 0.f);
+  }
   MDX_LAUNCH_CHECK();
   return 0;
 }
@@ -1340,25 +1423,25 @@ extern "C" int mdx_mlp_train_step(mdx_mlp* m, const double* d_pos, const double*
                                m->row_of.p, m->T.p, m->w.p, m->rstd.p, m->U.p);
   MDX_LAUNCH_CHECK();
   // tangent pass: a1 = U W1 ; b1 = a1 S1, c1 = a1 hb1 DD1 ; a2 = b1 W2 ; ... a3 = b2 W3
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_F, m->U.p, ML_F, 1, N0.w1.p, N1.w1.p, ML_H, 1, rs, m->A1.p, ML_H)))
+  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_F, m->U.p, ML_F, N0.w1.p, N1.w1.p, ML_H, 1, rs, m->A1.p, ML_H)))
     MDX_LEAVE_RET(rc);
   k_ml_tangent<<<div_up(RH, 256), 256, 0, st>>>(RH, m->A1.p, m->S1.p, m->HB1.p, m->D1.p, m->B1.p, m->C1.p);
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->B1.p, ML_H, 1, N0.w2.p, N1.w2.p, ML_H, 1, rs, m->A2.p, ML_H)))
+  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->B1.p, ML_H, N0.w2.p, N1.w2.p, ML_H, 1, rs, m->A2.p, ML_H)))
     MDX_LEAVE_RET(rc);
   k_ml_tangent<<<div_up(RH, 256), 256, 0, st>>>(RH, m->A2.p, m->S2.p, m->HB2.p, m->D2.p, m->B2.p, m->C2.p);
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->B2.p, ML_H, 1, N0.w3.p, N1.w3.p, ML_H, 1, rs, m->A3.p, ML_H)))
+  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->B2.p, ML_H, N0.w3.p, N1.w3.p, ML_H, 1, rs, m->A3.p, ML_H)))
     MDX_LEAVE_RET(rc);
   k_ml_top<<<div_up(RH, 256), 256, 0, st>>>(R, rs, m->A3.p, m->S3.p, m->D3.p, N0.p.p, N1.p.p, m->T4.p, m->DZ16_3.p,
                                             m->DZ3.p);
   // reverse through the forward pass: dH2 = dz3 W3^T ; dz2 = c2 + dH2 S2 ; dH1 = dz2 W2^T ; dz1 = c1 + dH1 S1
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->DZ16_3.p, ML_H, 1, N0.w3.p, N1.w3.p, 1, ML_H, rs, m->DH2.p, ML_H)))
+  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->DZ16_3.p, ML_H, N0.w3.p, N1.w3.p, 1, ML_H, rs, m->DH2.p, ML_H)))
     MDX_LEAVE_RET(rc);
   k_ml_dz<<<div_up(RH, 256), 256, 0, st>>>(RH, m->C2.p, m->DH2.p, m->S2.p, m->DZ16_2.p, m->DZ2.p);
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->DZ16_2.p, ML_H, 1, N0.w2.p, N1.w2.p, 1, ML_H, rs, m->DH1.p, ML_H)))
+  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->DZ16_2.p, ML_H, N0.w2.p, N1.w2.p, 1, ML_H, rs, m->DH1.p, ML_H)))
     MDX_LEAVE_RET(rc);
   k_ml_dz<<<div_up(RH, 256), 256, 0, st>>>(RH, m->C1.p, m->DH1.p, m->S1.p, m->DZ16_1.p, m->DZ1.p);
   MDX_LAUNCH_CHECK();
-  if ((rc = ml_weight_grads(m, 0, 0, m->nO)) || (rc = ml_weight_grads(m, 1, rs, rs + m->nH))) MDX_LEAVE_RET(rc);
+  if ((rc = ml_weight_grads(m))) MDX_LEAVE_RET(rc);
   if (lr > 0) {
     m->adam_t++;
     const float c1 = 1.f / (1.f - std::pow(m->beta1, (float)m->adam_t));
@@ -1398,6 +1481,6 @@ extern "C" int mdx_mlp_gemm_check(mdx_mlp* m, int M, int N, int K, const void* d
   MDX_CHECK(m && d_A && d_B && d_C && M > 0 && N > 0 && K > 0, MDX_ERR_INVALID, "mdx_mlp_gemm_check: bad arguments");
   mdx_ctx* c = m->host;
   MDX_ENTER();
-  int rc = gemm(m, EPI_F32, M, N, K, (const bf16_t*)d_A, K, 1, (const bf16_t*)d_B, nullptr, N, 1, 1 << 30, d_C, N);
+  int rc = gemm(m, EPI_F32, M, N, K, (const bf16_t*)d_A, K, (const bf16_t*)d_B, nullptr, N, 1, 1 << 30, d_C, N);
   MDX_LEAVE_RET(rc);
 }
