@@ -545,123 +545,150 @@ __global__ __launch_bounds__(64) void k_ml_jvp(MlAtoms a, MlConst k, const float
 }
 
 // ---------------------------------------------------------------- BF16 MFMA GEMM
-// C[m][n] = sum_k A[m][k] B[k][n] over k in this block's K range, A and B read through
-// arbitrary (row, col) strides (transposes are strides). 64x64 tile per 256-lane workgroup,
-// each wave a 32x32 sub-tile on gfx950's v_mfma_f32_32x32x16_bf16 (lane l: A row l%32, k
-// 8(l/32)..+7; B col l%32, same k; D row 8(i/4) + 4(l/32) + i%4, col l%32 for accumulator i).
-// Rows >= row_split use the second operand B1 / bias1 (the second element's weights).
-enum { EPI_F32 = 0, EPI_BIAS_SILU = 1, EPI_MUL_S = 2 };
+// C[m][n] = sum_k A[m][k] B[k][n], A row-major, B with either index contiguous (transposes are
+// strides). 64x64 tile per 256-lane workgroup, each wave a 32x32 sub-tile on gfx950's
+// v_mfma_f32_32x32x16_bf16 (lane l: A row l%32, k 8(l/32)..+7; B col l%32, same k; D row
+// 8(i/4) + 4(l/32) + i%4, col l%32 for accumulator i). Rows >= row_split use the second operand
+// B1 / bias1 (the second element's weights).
+//
+// Load latency and epilogue traffic bound it (K is at most 256): 64 k a step, both operands in
+// 16-byte loads, a row-contiguous B written to LDS as pairs of rows; the workgroups of one row tile on
+// one XCD, so A comes from memory once; and the elementwise step that follows the product is its
+// epilogue, which saves writing the product and reading it again. 23,328 rows x 256 x 256 (us):
+// forward 21.9 -> 16.7, input gradient 15.9 -> 15.3 (its last layer 16 -> 8); training's tangent and
+// adjoint products with their elementwise kernels 214 -> 150.
+enum {
+  EPI_F32 = 0,    // C = v
+  EPI_BIAS_SILU,  // z = v + bias: H = SiLU(z), S = SiLU'(z), DD = SiLU''(z) unless null
+  EPI_MUL_S,      // H = v S; C = v unless null
+  EPI_TANGENT,    // H = v S; C = v X DD
+  EPI_TOP,        // C = v S; Y = v bias DD, H = Y
+  EPI_DZ          // Y = X + v S, H = Y
+};
 struct GemmArgs {
   int M, N, K;
   const bf16_t* A;
-  long long a_m;              // A's row stride (its k index is contiguous)
+  long long a_m;  // A's row stride (its k index is contiguous)
   const bf16_t* B0;
   const bf16_t* B1;
   long long b_k, b_n;
   int row_split;
-  float* C;                   // EPI_F32: the product; EPI_BIAS_SILU: Z (+bias); EPI_MUL_S: raw product
+  float* C;
   long long ldc;
   const float* bias0;
   const float* bias1;
-  bf16_t* H;                  // bf16 output (SiLU(z) or product * S)
-  float* S;                   // EPI_BIAS_SILU: writes SiLU'(z); EPI_MUL_S: reads the multiplier
-  float* DD;                  // EPI_BIAS_SILU: writes SiLU''(z) when not null
+  bf16_t* H;
+  float* S;
+  float* DD;
+  const float* X;
+  float* Y;
 };
-#define GK 32
+#define GK 64
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// 8 consecutive bf16 of a tile row from global memory (16 B when all 8 are in range and the
-// address is 16-byte aligned, element by element with zero fill otherwise)
-__device__ __forceinline__ void load8(const bf16_t* __restrict__ base, long long off, long long step, int nvalid,
-                                      bf16_t* out) {
-  const bf16_t* p = base + off;
-  if (nvalid >= 8 && step == 1 && (((unsigned long long)p) & 15ull) == 0) {
-    const u32x4 v = *(const u32x4*)p;
-    const unsigned w[4] = {v.x, v.y, v.z, v.w};
+// 8 consecutive bf16 from global memory (16 B when all 8 are in range and the address is 16-byte
+// aligned, element by element with zero fill otherwise)
+__device__ __forceinline__ u32x4 load8(const bf16_t* __restrict__ p, int nvalid) {
+  if (nvalid >= 8 && (((unsigned long long)p) & 15ull) == 0) return *(const u32x4*)p;
+  u32x4 v;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      out[2 * i] = (bf16_t)(w[i] & 0xffffu);
-      out[2 * i + 1] = (bf16_t)(w[i] >> 16);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = i < nvalid ? p[(long long)i * step] : (bf16_t)0;
-  }
+  for (int i = 0; i < 4; ++i)
+    v[i] = (2 * i < nvalid ? (unsigned)p[2 * i] : 0u) | (2 * i + 1 < nvalid ? (unsigned)p[2 * i + 1] << 16 : 0u);
+  return v;
 }
 
-// A's k index is contiguous in memory; B_KC: so is B's (b_k == 1), else its column index is (b_n == 1). Each k-step
-// every lane moves one 8-element vector of A and one of B into LDS, where both tiles are
-// stored k-contiguous per row / column so each MFMA operand is one 8-byte LDS read.
-template <bool B_KC>
-__global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g, int epi) {
+// B_KC: B's k index is contiguous (b_k == 1), else its column index is (b_n == 1). Both tiles are
+// stored k-contiguous per row / column, so each MFMA operand is one 16-byte LDS read.
+template <bool B_KC, int EPI>
+__global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) bf16_t As[ML_TILE][GK + 8];
   __shared__ __attribute__((aligned(16))) bf16_t Bs[ML_TILE][GK + 8];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
-  const int row0 = blockIdx.y * ML_TILE, col0 = blockIdx.x * ML_TILE;
-  const int ke = g.K;
+  // workgroups go to the 8 XCDs in turn: 8 row tiles at a time, all column tiles of one on one XCD
+  const int nx = (g.N + ML_TILE - 1) / ML_TILE;
+  const int grp = blockIdx.x / (8 * nx), in = blockIdx.x - grp * (8 * nx);
+  const int row0 = (grp * 8 + (in & 7)) * ML_TILE, col0 = (in >> 3) * ML_TILE;
+  if (row0 >= g.M) return;
   const bool second = row0 >= g.row_split;
   const bf16_t* B = second ? g.B1 : g.B0;
   f32x16 acc;
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-  // this lane's tile vectors: A (row ra, k offset ka), B likewise or k kbv / columns rb..+7
-  const int ra = tid >> 2, ka = (tid & 3) * 8;
-  const int rb = B_KC ? (tid >> 2) : (tid & 7) * 8, kbv = B_KC ? (tid & 3) * 8 : (tid >> 3);
-  auto fetch = [&](int k0, bf16_t* va, bf16_t* vb) {
-    const int m = row0 + ra, ax = k0 + ka;
-    load8(g.A, (long long)m * g.a_m + ax, 1, m < g.M ? max(0, min(8, ke - ax)) : 0, va);
-    if (B_KC) {
-      const int n = col0 + rb, kx = k0 + kbv;
-      load8(B, (long long)n * g.b_n + kx, 1, n < g.N ? max(0, min(8, ke - kx)) : 0, vb);
-    } else {
-      const int n = col0 + rb, kx = k0 + kbv;
-      load8(B, (long long)kx * g.b_k + n, 1, kx < ke ? max(0, min(8, g.N - n)) : 0, vb);
+  // this lane's part of a step: 16 k of row / column r, or 8 columns of a pair of rows of B
+  const int r = tid >> 2, k16 = (tid & 3) * 16;
+  const int c8 = (tid & 7) * 8, kp = tid >> 3;
+  u32x4 va[2], vb[2];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int k = k0 + k16 + 8 * u;
+      va[u] = load8(g.A + (long long)(row0 + r) * g.a_m + k, row0 + r < g.M ? g.K - k : 0);
+      if (B_KC) {
+        vb[u] = load8(B + (long long)(col0 + r) * g.b_n + k, col0 + r < g.N ? g.K - k : 0);
+      } else {
+        const int kb = k0 + 2 * kp + u;
+        vb[u] = load8(B + (long long)kb * g.b_k + col0 + c8, kb < g.K ? g.N - col0 - c8 : 0);
+      }
     }
   };
-  bf16_t va[8], vb[8];
-  fetch(0, va, vb);
-  for (int k0 = 0; k0 < ke; k0 += GK) {
+  fetch(0);
+  for (int k0 = 0; k0 < g.K; k0 += GK) {
+    *(u32x4*)&As[r][k16] = va[0];
+    *(u32x4*)&As[r][k16 + 8] = va[1];
+    if (B_KC) {
+      *(u32x4*)&Bs[r][k16] = vb[0];
+      *(u32x4*)&Bs[r][k16 + 8] = vb[1];
+    } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      As[ra][ka + i] = va[i];
-      if (B_KC) Bs[rb][kbv + i] = vb[i];
-      else Bs[rb + i][kbv] = vb[i];
+      for (int i = 0; i < 4; ++i) {
+        *(unsigned*)&Bs[c8 + 2 * i][2 * kp] = (vb[0][i] & 0xffffu) | (vb[1][i] << 16);
+        *(unsigned*)&Bs[c8 + 2 * i + 1][2 * kp] = (vb[0][i] >> 16) | (vb[1][i] & 0xffff0000u);
+      }
     }
     __syncthreads();
-    if (k0 + GK < ke) fetch(k0 + GK, va, vb);  // next step's loads in flight during the MFMAs
+    if (k0 + GK < g.K) fetch(k0 + GK);  // next step's loads in flight during the MFMAs
 #pragma unroll
     for (int ks = 0; ks < GK; ks += 16) {
-      // v_mfma_f32_32x32x16_bf16: lane l supplies row (or column) l%32 and k 8(l/32)..+7, one
-      // 16-byte LDS read per operand (rows are 80 B, k offsets multiples of 8: 16-byte aligned)
-      const int ar = wm * 32 + (lane & 31), kq = ks + (lane >> 5) * 8;
-      const int bc = wn * 32 + (lane & 31);
-      const bf16x8 av = *(const bf16x8*)&As[ar][kq];
-      const bf16x8 bv = *(const bf16x8*)&Bs[bc][kq];
+      // rows are 144 B, k offsets multiples of 8: 16-byte aligned
+      const int kq = ks + (lane >> 5) * 8;
+      const bf16x8 av = *(const bf16x8*)&As[wm * 32 + (lane & 31)][kq];
+      const bf16x8 bv = *(const bf16x8*)&Bs[wn * 32 + (lane & 31)][kq];
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
     }
     __syncthreads();
   }
+  const int n = col0 + wn * 32 + (lane & 31);
+  if (n >= g.N) return;
+  const float bias = EPI == EPI_BIAS_SILU || EPI == EPI_TOP ? (second ? g.bias1 : g.bias0)[n] : 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int r = wm * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-    const int c = wn * 32 + (lane & 31);
-    const int m = row0 + r, n = col0 + c;
-    if (m >= g.M || n >= g.N) continue;
+    const int m = row0 + wm * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
+    if (m >= g.M) continue;
     const float v = acc[i];
-    if (epi == EPI_F32) {
-      g.C[(long long)m * g.ldc + n] = v;
-    } else if (epi == EPI_BIAS_SILU) {
-      const float z = v + (second ? g.bias1 : g.bias0)[n];
+    const long long idx = (long long)m * g.ldc + n;
+    if (EPI == EPI_F32) {
+      g.C[idx] = v;
+    } else if (EPI == EPI_BIAS_SILU) {
+      const float z = v + bias;
       const float sg = 1.f / (1.f + __expf(-z));
-      const long long idx = (long long)m * g.ldc + n;
-      if (g.C) g.C[idx] = z;
       g.H[idx] = f2bf(z * sg);
       g.S[idx] = sg * (1.f + z * (1.f - sg));
       if (g.DD) g.DD[idx] = sg * (1.f - sg) * (2.f + z * (1.f - 2.f * sg));
-    } else {  // EPI_MUL_S
-      const long long idx = (long long)m * g.ldc + n;
+    } else if (EPI == EPI_MUL_S) {
       if (g.C) g.C[idx] = v;
       g.H[idx] = f2bf(v * g.S[idx]);
+    } else if (EPI == EPI_TANGENT) {
+      g.H[idx] = f2bf(v * g.S[idx]);
+      g.C[idx] = v * g.X[idx] * g.DD[idx];
+    } else if (EPI == EPI_TOP) {
+      g.C[idx] = v * g.S[idx];
+      const float y = v * bias * g.DD[idx];
+      g.H[idx] = f2bf(y);
+      g.Y[idx] = y;
+    } else {
+      const float y = g.X[idx] + v * g.S[idx];
+      g.H[idx] = f2bf(y);
+      g.Y[idx] = y;
     }
   }
 }
@@ -710,37 +737,6 @@ __global__ __launch_bounds__(256) void k_ml_head(int rows, int row_split, const 
     atomicAdd((unsigned long long*)eslot, (unsigned long long)to_fix(wsum[0] + wsum[1] + wsum[2] + wsum[3]));
 }
 
-// tangent step of one layer: b = a * S (bf16), c = a * hb * DD (fp32)
-__global__ void k_ml_tangent(long long count, const float* __restrict__ a, const float* __restrict__ S,
-                             const float* __restrict__ hb, const float* __restrict__ DD, bf16_t* __restrict__ b,
-                             float* __restrict__ c) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  b[i] = f2bf(a[i] * S[i]);
-  c[i] = a[i] * hb[i] * DD[i];
-}
-// dz = c + dh * S (bf16; also fp32 for the bias sums)
-__global__ void k_ml_dz(long long count, const float* __restrict__ c, const float* __restrict__ dh,
-                        const float* __restrict__ S, bf16_t* __restrict__ dz16, float* __restrict__ dz32) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const float v = c[i] + (dh ? dh[i] * S[i] : 0.f);
-  dz16[i] = f2bf(v);
-  dz32[i] = v;
-}
-// last layer: dw4 terms a3 * S3 (fp32) and dz3 = a3 * w4 * DD3
-__global__ void k_ml_top(int rows, int row_split, const float* __restrict__ a3, const float* __restrict__ S3,
-                         const float* __restrict__ DD3, const float* __restrict__ p0, const float* __restrict__ p1,
-                         float* __restrict__ t4, bf16_t* __restrict__ dz16, float* __restrict__ dz32) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)rows * ML_H) return;
-  const int row = (int)(i / ML_H), c = (int)(i % ML_H);
-  const float* p = row >= row_split ? p1 : p0;
-  t4[i] = a3[i] * S3[i];
-  const float v = a3[i] * p[P_W4 + c] * DD3[i];
-  dz16[i] = f2bf(v);
-  dz32[i] = v;
-}
 // Column sums over rows [r0, r1) of the four ML_H-wide arrays, in a fixed order: workgroup (b, q) sums
 // chunk b of array q's rows (wave w the rows w, w + 4, ..; a float4 of columns per lane, so a row is
 // one coalesced load of a wave), its waves' sums are added in order, then one lane per column adds
@@ -967,7 +963,7 @@ struct mdx_mlp {
   MlNet net[2];
   MlConst k;
   // activations (rows x width)
-  DevBuf<float> G, T, GX, S1, S2, S3, D1, D2, D3, HB1, HB2, A1, A2, A3, C1, C2, T4, DZ1, DZ2, DZ3, DH1, DH2;
+  DevBuf<float> G, T, GX, S1, S2, S3, D1, D2, D3, HB1, HB2, C1, C2, T4, DZ1, DZ2, DZ3;
   DevBuf<bf16_t> X, H1, H2, H3, G1, G2, G3, U, B1, B2, DZ16_1, DZ16_2, DZ16_3;
   DevBuf<float> part;           // split-K partials
   DevBuf<double> w;             // loss weights (3N)
@@ -1015,11 +1011,10 @@ static int ml_alloc(mdx_mlp* m, bool training) {
   }
   if (training && !m->trained_buffers) {
     if ((rc = m->D1.ensure(R * ML_H)) || (rc = m->D2.ensure(R * ML_H)) || (rc = m->D3.ensure(R * ML_H)) ||
-        (rc = m->HB1.ensure(R * ML_H)) || (rc = m->HB2.ensure(R * ML_H)) || (rc = m->A1.ensure(R * ML_H)) ||
-        (rc = m->A2.ensure(R * ML_H)) || (rc = m->A3.ensure(R * ML_H)) || (rc = m->C1.ensure(R * ML_H)) ||
+        (rc = m->HB1.ensure(R * ML_H)) || (rc = m->HB2.ensure(R * ML_H)) || (rc = m->C1.ensure(R * ML_H)) ||
         (rc = m->C2.ensure(R * ML_H)) || (rc = m->T4.ensure(R * ML_H)) || (rc = m->DZ1.ensure(R * ML_H)) ||
-        (rc = m->DZ2.ensure(R * ML_H)) || (rc = m->DZ3.ensure(R * ML_H)) || (rc = m->DH1.ensure(R * ML_H)) ||
-        (rc = m->DH2.ensure(R * ML_H)) || (rc = m->U.ensure(R * ML_F)) || (rc = m->B1.ensure(R * ML_H)) ||
+        (rc = m->DZ2.ensure(R * ML_H)) || (rc = m->DZ3.ensure(R * ML_H)) ||
+        (rc = m->U.ensure(R * ML_F)) || (rc = m->B1.ensure(R * ML_H)) ||
         (rc = m->B2.ensure(R * ML_H)) || (rc = m->DZ16_1.ensure(R * ML_H)) || (rc = m->DZ16_2.ensure(R * ML_H)) ||
         (rc = m->DZ16_3.ensure(R * ML_H)) || (rc = m->w.ensure(3 * (size_t)m->n)))
       return rc;
@@ -1136,8 +1131,8 @@ extern "C" int mdx_mlp_destroy(mdx_mlp* m) {
   if (m->host->mlp == m) m->host->mlp = nullptr;
   mdx_ctx_destroy(m->nl);
   for (DevBuf<float>* b : {&m->mean, &m->rstd, &m->G, &m->T, &m->GX, &m->S1, &m->S2, &m->S3,
-                           &m->D1, &m->D2, &m->D3, &m->HB1, &m->HB2, &m->A1, &m->A2, &m->A3, &m->C1, &m->C2, &m->T4,
-                           &m->DZ1, &m->DZ2, &m->DZ3, &m->DH1, &m->DH2, &m->part})
+                           &m->D1, &m->D2, &m->D3, &m->HB1, &m->HB2, &m->C1, &m->C2, &m->T4,
+                           &m->DZ1, &m->DZ2, &m->DZ3, &m->part})
     b->release();
   for (DevBuf<bf16_t>* b : {&m->X, &m->H1, &m->H2, &m->H3, &m->G1, &m->G2, &m->G3, &m->U, &m->B1, &m->B2, &m->DZ16_1,
                             &m->DZ16_2, &m->DZ16_3})
@@ -1209,35 +1204,117 @@ extern "C" int mdx_mlp_set_norm(mdx_mlp* m, const float* h_mean, const float* h_
 }
 
 // ---- GEMM launcher
-static int gemm(mdx_mlp* m, int epi, int M, int N, int K, const bf16_t* A, long long a_m, const bf16_t* B0,
-                const bf16_t* B1, long long b_k, long long b_n, int row_split, float* C, long long ldc,
-                const float* bias0 = nullptr, const float* bias1 = nullptr, bf16_t* H = nullptr, float* S = nullptr,
-                float* DD = nullptr) {
+struct Epilogue {
+  int kind = EPI_F32;
+  float* C = nullptr;
+  bf16_t* H = nullptr;
+  float* S = nullptr;
+  float* DD = nullptr;
+  const float* bias0 = nullptr;
+  const float* bias1 = nullptr;
+  const float* X = nullptr;
+  float* Y = nullptr;
+};
+static int gemm(mdx_mlp* m, int M, int N, int K, const bf16_t* A, const bf16_t* B0, const bf16_t* B1, long long b_k,
+                long long b_n, int row_split, const Epilogue& e) {
   GemmArgs g;
   g.M = M;
   g.N = N;
   g.K = K;
   g.A = A;
-  g.a_m = a_m;
+  g.a_m = K;
   g.B0 = B0;
   g.B1 = B1 ? B1 : B0;
   g.b_k = b_k;
   g.b_n = b_n;
   g.row_split = row_split;
-  g.C = C;
-  g.ldc = ldc;
-  g.bias0 = bias0;
-  g.bias1 = bias1 ? bias1 : bias0;
-  g.H = H;
-  g.S = S;
-  g.DD = DD;
-  dim3 grid(div_up(N, ML_TILE), div_up(M, ML_TILE));
+  g.C = e.C;
+  g.ldc = N;
+  g.bias0 = e.bias0;
+  g.bias1 = e.bias1;
+  g.H = e.H;
+  g.S = e.S;
+  g.DD = e.DD;
+  g.X = e.X;
+  g.Y = e.Y;
+  const int grid = div_up(N, ML_TILE) * div_up(div_up(M, ML_TILE), 8) * 8;
   MDX_CHECK(b_k == 1 || b_n == 1, MDX_ERR_INVALID, "gemm: one stride of B must be 1");
   hipStream_t st = m->host->stream;
-  if (b_k == 1) k_gemm_bf16<true><<<grid, 256, 0, st>>>(g, epi);
-  else k_gemm_bf16<false><<<grid, 256, 0, st>>>(g, epi);
+  const bool kc = b_k == 1 && b_n != 1;
+#define ML_GEMM(KC_, E_) else if (kc == KC_ && e.kind == E_) k_gemm_bf16<KC_, E_><<<grid, 256, 0, st>>>(g)
+  if (false) {}
+  ML_GEMM(false, EPI_F32);
+  ML_GEMM(true, EPI_F32);
+  ML_GEMM(false, EPI_BIAS_SILU);
+  ML_GEMM(true, EPI_MUL_S);
+  ML_GEMM(false, EPI_TANGENT);
+  ML_GEMM(false, EPI_TOP);
+  ML_GEMM(true, EPI_DZ);
+  else MDX_CHECK(false, MDX_ERR_INVALID, "gemm: no kernel for this epilogue");
+#undef ML_GEMM
   MDX_LAUNCH_CHECK();
   return 0;
+}
+// the layers' products: A (rows x in) W (in x out), or A (rows x out) W^T
+static int layer(mdx_mlp* m, int in, int out, const bf16_t* A, const bf16_t* W0, const bf16_t* W1, const Epilogue& e) {
+  return gemm(m, m->rows, out, in, A, W0, W1, out, 1, m->rowsO, e);
+}
+static int layer_t(mdx_mlp* m, int in, int out, const bf16_t* A, const bf16_t* W0, const bf16_t* W1, const Epilogue& e) {
+  return gemm(m, m->rows, in, out, A, W0, W1, 1, out, m->rowsO, e);
+}
+static Epilogue epi_silu(bf16_t* H, float* S, float* DD, const float* b0, const float* b1) {
+  Epilogue e;
+  e.kind = EPI_BIAS_SILU;
+  e.H = H;
+  e.S = S;
+  e.DD = DD;
+  e.bias0 = b0;
+  e.bias1 = b1;
+  return e;
+}
+static Epilogue epi_mul(float* C, bf16_t* H, float* S) {
+  Epilogue e;
+  e.kind = EPI_MUL_S;
+  e.C = C;
+  e.H = H;
+  e.S = S;
+  return e;
+}
+static Epilogue epi_f32(float* C) {
+  Epilogue e;
+  e.C = C;
+  return e;
+}
+static Epilogue epi_tangent(bf16_t* b, float* c, float* S, const float* hb, float* DD) {
+  Epilogue e;
+  e.kind = EPI_TANGENT;
+  e.H = b;
+  e.C = c;
+  e.S = S;
+  e.X = hb;
+  e.DD = DD;
+  return e;
+}
+static Epilogue epi_top(float* t4, bf16_t* dz16, float* dz, float* S, float* DD, const float* w0, const float* w1) {
+  Epilogue e;
+  e.kind = EPI_TOP;
+  e.C = t4;
+  e.H = dz16;
+  e.Y = dz;
+  e.S = S;
+  e.DD = DD;
+  e.bias0 = w0;
+  e.bias1 = w1;
+  return e;
+}
+static Epilogue epi_dz(bf16_t* dz16, float* dz, const float* c, float* S) {
+  Epilogue e;
+  e.kind = EPI_DZ;
+  e.H = dz16;
+  e.Y = dz;
+  e.X = c;
+  e.S = S;
+  return e;
 }
 
 // descriptors + forward + input gradient (GX); energy into eslot when given
@@ -1254,22 +1331,19 @@ static int ml_forward_backward(mdx_mlp* m, long long* eslot, bool keep_training_
   float* DD1 = keep_training_state ? m->D1.p : nullptr;
   float* DD2 = keep_training_state ? m->D2.p : nullptr;
   float* DD3 = keep_training_state ? m->D3.p : nullptr;
-  if ((rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_F, m->X.p, ML_F, N0.w1.p, N1.w1.p, ML_H, 1, rs, nullptr, ML_H,
-                 N0.p.p + P_B1, N1.p.p + P_B1, m->H1.p, m->S1.p, DD1)) ||
-      (rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_H, m->H1.p, ML_H, N0.w2.p, N1.w2.p, ML_H, 1, rs, nullptr, ML_H,
-                 N0.p.p + P_B2, N1.p.p + P_B2, m->H2.p, m->S2.p, DD2)) ||
-      (rc = gemm(m, EPI_BIAS_SILU, R, ML_H, ML_H, m->H2.p, ML_H, N0.w3.p, N1.w3.p, ML_H, 1, rs, nullptr, ML_H,
-                 N0.p.p + P_B3, N1.p.p + P_B3, m->H3.p, m->S3.p, DD3)))
+  if ((rc = layer(m, ML_F, ML_H, m->X.p, N0.w1.p, N1.w1.p, epi_silu(m->H1.p, m->S1.p, DD1, N0.p.p + P_B1, N1.p.p + P_B1))) ||
+      (rc = layer(m, ML_H, ML_H, m->H1.p, N0.w2.p, N1.w2.p, epi_silu(m->H2.p, m->S2.p, DD2, N0.p.p + P_B2, N1.p.p + P_B2))) ||
+      (rc = layer(m, ML_H, ML_H, m->H2.p, N0.w3.p, N1.w3.p, epi_silu(m->H3.p, m->S3.p, DD3, N0.p.p + P_B3, N1.p.p + P_B3))))
     return rc;
   k_ml_head<<<div_up(R, HEAD_ROWS), 256, 0, st>>>(R, rs, m->H3.p, m->S3.p, N0.p.p, N1.p.p, m->atom_of_row.p,
                                                    m->G3.p, nullptr, eslot);
   MDX_LAUNCH_CHECK();
   // input gradient: G2 = (G3 W3^T) * S2, G1 = (G2 W2^T) * S1, GX = G1 W1^T
-  if ((rc = gemm(m, EPI_MUL_S, R, ML_H, ML_H, m->G3.p, ML_H, N0.w3.p, N1.w3.p, 1, ML_H, rs,
-                 keep_training_state ? m->HB2.p : nullptr, ML_H, nullptr, nullptr, m->G2.p, m->S2.p)) ||
-      (rc = gemm(m, EPI_MUL_S, R, ML_H, ML_H, m->G2.p, ML_H, N0.w2.p, N1.w2.p, 1, ML_H, rs,
-                 keep_training_state ? m->HB1.p : nullptr, ML_H, nullptr, nullptr, m->G1.p, m->S1.p)) ||
-      (rc = gemm(m, EPI_F32, R, ML_F, ML_H, m->G1.p, ML_H, N0.w1.p, N1.w1.p, 1, ML_H, rs, m->GX.p, ML_F)))
+  float* HB2 = keep_training_state ? m->HB2.p : nullptr;
+  float* HB1 = keep_training_state ? m->HB1.p : nullptr;
+  if ((rc = layer_t(m, ML_H, ML_H, m->G3.p, N0.w3.p, N1.w3.p, epi_mul(HB2, m->G2.p, m->S2.p))) ||
+      (rc = layer_t(m, ML_H, ML_H, m->G2.p, N0.w2.p, N1.w2.p, epi_mul(HB1, m->G1.p, m->S1.p))) ||
+      (rc = layer_t(m, ML_F, ML_H, m->G1.p, N0.w1.p, N1.w1.p, epi_f32(m->GX.p))))
     return rc;
   return 0;
 }
@@ -1409,8 +1483,6 @@ extern "C" int mdx_mlp_train_step(mdx_mlp* m, const double* d_pos, const double*
   if (rc) MDX_LEAVE_RET(rc);
   m->nl->pos = const_cast<double*>(d_pos);
   const long long n3 = 3LL * m->n;
-  const int R = m->rows, rs = m->rowsO;
-  const long long RH = (long long)R * ML_H;
   MlNet &N0 = m->net[0], &N1 = m->net[1];
   if ((rc = mdx_nlist_update(m->nl, true)) || (rc = mdx_nlist_enqueue_clear(m->nl))) MDX_LEAVE_RET(rc);
   k_ml_zero_i64<<<div_up(n3, 256), 256, 0, st>>>(n3, m->nl->ffix.p);
@@ -1422,25 +1494,15 @@ extern "C" int mdx_mlp_train_step(mdx_mlp* m, const double* d_pos, const double*
   k_ml_jvp<<<m->n, 64, 0, st>>>(a, m->k, m->nl->xq.p, m->nl->sorted_orig.p, m->nl->nbr_count.p, m->nl->nbr_list.p,
                                m->row_of.p, m->T.p, m->w.p, m->rstd.p, m->U.p);
   MDX_LAUNCH_CHECK();
-  // tangent pass: a1 = U W1 ; b1 = a1 S1, c1 = a1 hb1 DD1 ; a2 = b1 W2 ; ... a3 = b2 W3
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_F, m->U.p, ML_F, N0.w1.p, N1.w1.p, ML_H, 1, rs, m->A1.p, ML_H)))
+  // tangent pass: a1 = U W1, b1 = a1 S1, c1 = a1 hb1 DD1; a2 = b1 W2, ..; a3 = b2 W3, t4 = a3 S3,
+  // dz3 = a3 w4 DD3. Reverse through the forward pass: dz2 = c2 + (dz3 W3^T) S2, dz1 = c1 + (dz2 W2^T) S1
+  if ((rc = layer(m, ML_F, ML_H, m->U.p, N0.w1.p, N1.w1.p, epi_tangent(m->B1.p, m->C1.p, m->S1.p, m->HB1.p, m->D1.p))) ||
+      (rc = layer(m, ML_H, ML_H, m->B1.p, N0.w2.p, N1.w2.p, epi_tangent(m->B2.p, m->C2.p, m->S2.p, m->HB2.p, m->D2.p))) ||
+      (rc = layer(m, ML_H, ML_H, m->B2.p, N0.w3.p, N1.w3.p,
+                  epi_top(m->T4.p, m->DZ16_3.p, m->DZ3.p, m->S3.p, m->D3.p, N0.p.p + P_W4, N1.p.p + P_W4))) ||
+      (rc = layer_t(m, ML_H, ML_H, m->DZ16_3.p, N0.w3.p, N1.w3.p, epi_dz(m->DZ16_2.p, m->DZ2.p, m->C2.p, m->S2.p))) ||
+      (rc = layer_t(m, ML_H, ML_H, m->DZ16_2.p, N0.w2.p, N1.w2.p, epi_dz(m->DZ16_1.p, m->DZ1.p, m->C1.p, m->S1.p))))
     MDX_LEAVE_RET(rc);
-  k_ml_tangent<<<div_up(RH, 256), 256, 0, st>>>(RH, m->A1.p, m->S1.p, m->HB1.p, m->D1.p, m->B1.p, m->C1.p);
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->B1.p, ML_H, N0.w2.p, N1.w2.p, ML_H, 1, rs, m->A2.p, ML_H)))
-    MDX_LEAVE_RET(rc);
-  k_ml_tangent<<<div_up(RH, 256), 256, 0, st>>>(RH, m->A2.p, m->S2.p, m->HB2.p, m->D2.p, m->B2.p, m->C2.p);
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->B2.p, ML_H, N0.w3.p, N1.w3.p, ML_H, 1, rs, m->A3.p, ML_H)))
-    MDX_LEAVE_RET(rc);
-  k_ml_top<<<div_up(RH, 256), 256, 0, st>>>(R, rs, m->A3.p, m->S3.p, m->D3.p, N0.p.p, N1.p.p, m->T4.p, m->DZ16_3.p,
-                                            m->DZ3.p);
-  // reverse through the forward pass: dH2 = dz3 W3^T ; dz2 = c2 + dH2 S2 ; dH1 = dz2 W2^T ; dz1 = c1 + dH1 S1
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->DZ16_3.p, ML_H, N0.w3.p, N1.w3.p, 1, ML_H, rs, m->DH2.p, ML_H)))
-    MDX_LEAVE_RET(rc);
-  k_ml_dz<<<div_up(RH, 256), 256, 0, st>>>(RH, m->C2.p, m->DH2.p, m->S2.p, m->DZ16_2.p, m->DZ2.p);
-  if ((rc = gemm(m, EPI_F32, R, ML_H, ML_H, m->DZ16_2.p, ML_H, N0.w2.p, N1.w2.p, 1, ML_H, rs, m->DH1.p, ML_H)))
-    MDX_LEAVE_RET(rc);
-  k_ml_dz<<<div_up(RH, 256), 256, 0, st>>>(RH, m->C1.p, m->DH1.p, m->S1.p, m->DZ16_1.p, m->DZ1.p);
-  MDX_LAUNCH_CHECK();
   if ((rc = ml_weight_grads(m))) MDX_LEAVE_RET(rc);
   if (lr > 0) {
     m->adam_t++;
@@ -1481,6 +1543,6 @@ extern "C" int mdx_mlp_gemm_check(mdx_mlp* m, int M, int N, int K, const void* d
   MDX_CHECK(m && d_A && d_B && d_C && M > 0 && N > 0 && K > 0, MDX_ERR_INVALID, "mdx_mlp_gemm_check: bad arguments");
   mdx_ctx* c = m->host;
   MDX_ENTER();
-  int rc = gemm(m, EPI_F32, M, N, K, (const bf16_t*)d_A, K, (const bf16_t*)d_B, nullptr, N, 1, 1 << 30, d_C, N);
+  int rc = gemm(m, M, N, K, (const bf16_t*)d_A, (const bf16_t*)d_B, nullptr, N, 1, 1 << 30, epi_f32(d_C));
   MDX_LEAVE_RET(rc);
 }
