@@ -816,7 +816,7 @@ extern "C" int mdx_ctx_destroy(mdx_ctx* c) {
   c->bond_par.release(); c->angle_par.release(); c->dih_par.release(); c->imp_par.release();
   c->ffix.release(); c->efix.release(); c->dstate.release();
   c->ref_cell_lin.release(); c->ref_counts.release(); c->ref_cursor.release();
-  c->cell_count.release(); c->cell_start.release(); c->cell_cursor.release(); c->atom_cell.release();
+  c->cell_count.release(); c->cell_start.release(); c->atom_place.release(); c->atom_cell.release();
   c->sorted_orig.release(); c->orig_sorted.release(); c->xq.release(); c->xf.release(); c->ljs.release(); c->ljs14.release();
   c->ref_cell_sorted.release(); c->pos_at_build.release(); c->nbr_count.release(); c->nbr_list.release();
   c->d_stencil.release(); c->qfix.release(); c->cgrid.release(); c->conv.release(); c->bc.release(); c->bch.release();

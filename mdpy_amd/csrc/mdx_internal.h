@@ -261,7 +261,7 @@ struct mdx_ctx {
   int gn[3] = {0, 0, 0};
   int reach[3] = {0, 0, 0};
   int ncell = 0;
-  DevBuf<int> cell_count, cell_start, cell_cursor, atom_cell;
+  DevBuf<int> cell_count, cell_start, atom_place, atom_cell;
   DevBuf<int> sorted_orig;       // sorted slot -> original atom
   DevBuf<int> orig_sorted;       // original atom -> sorted slot
   DevBuf<float4> xq;             // sorted: x, y, z (centred, float), q*sqrt(ke)
