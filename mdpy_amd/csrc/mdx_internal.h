@@ -16,17 +16,20 @@ static constexpr double kFixScale = 1099511627776.0;          // 2^40
 static constexpr double kFixInv = 1.0 / 1099511627776.0;
 
 __device__ __forceinline__ long long to_fix(double v) { return __double2ll_rn(v * kFixScale); }
-// v * 2^40 rounded to nearest even, in float32: the scaling and both words' split are exact. The
+// v * 2^40 rounded to nearest even, in float32. The magnitude is converted and the sign applied to the
+// 64-bit result: for |f| the scaling and the split into two words are exact (the low word of a
+// negative f would be 2^32 - |f|, which does not fit 24 bits), so both signs give the same bits. The
 // conversions are the instructions themselves, which saturate (and give 0 for NaN).
 __device__ __forceinline__ long long to_fix_f(float v) {
-  const float f = rintf(v * 1099511627776.f);
-  const float h = floorf(f * 0x1p-32f);
-  const float l = fmaf(-h, 4294967296.f, f);  // 0 <= l < 2^32
+  const float f = rintf(v * 1099511627776.f), m = fabsf(f);
+  const float h = floorf(m * 0x1p-32f);
+  const float l = fmaf(-h, 4294967296.f, m);  // 0 <= l < 2^32
   int hi;
   unsigned lo;
   asm("v_cvt_i32_f32 %0, %1" : "=v"(hi) : "v"(h));
   asm("v_cvt_u32_f32 %0, %1" : "=v"(lo) : "v"(l));
-  return (long long)(((unsigned long long)(unsigned)hi << 32) | lo);
+  const long long r = (long long)((unsigned long long)(unsigned)hi << 32 | lo);
+  return f < 0.f ? -r : r;
 }
 
 // Orders one wave's LDS writes before its later LDS reads (and the reads before later writes):
