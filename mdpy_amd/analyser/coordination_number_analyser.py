@@ -3,7 +3,7 @@
 frames; mean and std over the first selection. Histograms from the GPU (pair_histograms)."""
 import numpy as np
 
-from ..utils import check_topological_selection_condition, parse_selection_condition, select_first_frame
+from ..utils import check_topological_selection_condition, parse_selection_condition, select_pair_first_frame
 from ..unit import check_quantity_value
 from .analyser_result import AnalyserResult
 from .pair_histogram import pair_histograms
@@ -21,9 +21,7 @@ class CoordinationNumberAnalyser:
         self._num_bins = num_bins
 
     def analysis(self, trajectory, is_dimensionless=True) -> AnalyserResult:
-        ids1 = select_first_frame(trajectory, self._selection_condition_1)
-        ids2 = ids1 if self._selection_condition_2 == self._selection_condition_1 else \
-            select_first_frame(trajectory, self._selection_condition_2)
+        ids1, ids2 = select_pair_first_frame(trajectory, self._selection_condition_1, self._selection_condition_2)
         counts, bin_edge = pair_histograms(trajectory, ids1, ids2, self._cutoff_radius, self._num_bins)
         # the frame mean of the per-frame cumulative sums is the cumulative sum of the summed counts
         # over the frame count

@@ -5,7 +5,7 @@ over frames, the shell-volume normalisation, the mean / std over the first selec
 overall scaling are the reference's (rdf_analyser.py:44-65)."""
 import numpy as np
 
-from ..utils import check_topological_selection_condition, parse_selection_condition, select_first_frame
+from ..utils import check_topological_selection_condition, parse_selection_condition, select_pair_first_frame
 from ..unit import check_quantity_value
 from .analyser_result import AnalyserResult
 from .pair_histogram import pair_histograms
@@ -23,9 +23,7 @@ class RDFAnalyser:
         self._num_bins = num_bins
 
     def analysis(self, trajectory, is_dimensionless=True) -> AnalyserResult:
-        ids1 = select_first_frame(trajectory, self._selection_condition_1)
-        ids2 = ids1 if self._selection_condition_2 == self._selection_condition_1 else \
-            select_first_frame(trajectory, self._selection_condition_2)
+        ids1, ids2 = select_pair_first_frame(trajectory, self._selection_condition_1, self._selection_condition_2)
         counts, bin_edge = pair_histograms(trajectory, ids1, ids2, self._cutoff_radius, self._num_bins)
         hist = counts / trajectory.num_frames  # frame mean per atom of selection 1
         bin_width = bin_edge[1] - bin_edge[0]

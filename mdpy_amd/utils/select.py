@@ -217,6 +217,23 @@ def select_first_frame(trajectory, conditions):
     return _select_frame(trajectory, conditions, 0, {})
 
 
+def _same_condition(a, b):
+    """Whether two conditions are surely the same. Values may be arrays, whose comparison has no truth
+    value (ValueError): those are the same only as one object."""
+    if a is b:
+        return True
+    try:
+        return bool(a == b)
+    except ValueError:
+        return False
+
+
+def select_pair_first_frame(trajectory, conditions_1, conditions_2):
+    """select_first_frame of two conditions; equal ones are evaluated once."""
+    ids1 = select_first_frame(trajectory, conditions_1)
+    return ids1, ids1 if _same_condition(conditions_2, conditions_1) else select_first_frame(trajectory, conditions_2)
+
+
 def select(target, conditions):
     """Matrix ids of a Topology (one list) or of each frame of a Trajectory (list of lists)."""
     from ..core.trajectory import Trajectory
