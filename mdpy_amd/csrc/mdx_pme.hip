@@ -577,6 +577,24 @@ __device__ __forceinline__ int reserve_slot(bool keep, int* counter) {
   return base + __popcll(m & ((1ull << lane) - 1ull));
 }
 
+// the record of sorted slot s for plane x0: splines' offsets and kx (beyond 3: it does not touch the plane)
+__device__ __forceinline__ GatherRec plane_record(const PlaneArgs& a, const int* __restrict__ sorted_orig,
+                                                  const double* __restrict__ pos_sorted, const float4* __restrict__ xq,
+                                                  int s, int x0, int* by, int* bz, int* kx) {
+  const double x = pos_sorted[3 * s], y = pos_sorted[3 * s + 1], z = pos_sorted[3 * s + 2];
+  GatherRec g;
+  g.q = xq[s].w;
+  g.atom = sorted_orig[s];
+  int bx;
+  frac_coord(x, a.iLx, a.Kx, &bx, &g.wx);
+  frac_coord(y, a.iLy, a.Ky, by, &g.wy);
+  frac_coord(z, a.iLz, a.Kz, bz, &g.wz);
+  *kx = bx - x0;
+  *kx += *kx < 0 ? a.Kx : 0;
+  g.yzk = *by | (*bz << 12) | (*kx << 24);
+  return g;
+}
+
 // candidates examined per lane per round of phase 1 (independent loads in flight), and gather
 // records held ahead per lane
 #define PLANE_U 4
@@ -646,19 +664,9 @@ __device__ __forceinline__ void plane_fwd_body(const PlaneArgs& a, const FftPlan
     __syncthreads();
     const int nt = ntouch;
     for (int e = threadIdx.x; e < nt; e += blockDim.x) {
-      const int s = list[e];
-      const double x = pos_sorted[3 * s], y = pos_sorted[3 * s + 1], z = pos_sorted[3 * s + 2];
-      const float q = xq[s].w;
-      GatherRec g;
-      g.atom = sorted_orig[s];
-      int bx, by, bz;
-      frac_coord(x, a.iLx, a.Kx, &bx, &g.wx);
-      frac_coord(y, a.iLy, a.Ky, &by, &g.wy);
-      frac_coord(z, a.iLz, a.Kz, &bz, &g.wz);
-      int kx = bx - x0;
-      kx += kx < 0 ? a.Kx : 0;
-      g.yzk = by | (bz << 12) | (kx << 24);
-      g.q = q;
+      int by, bz, kx;
+      const GatherRec g = plane_record(a, sorted_orig, pos_sorted, xq, list[e], x0, &by, &bz, &kx);
+      const float q = g.q;
       // the gather's record (zero charges included: the gather writes their slot, so every atom
       // owns exactly four)
       if (done + e < a.rec_cap) gout[done + e] = g;
@@ -683,10 +691,7 @@ __device__ __forceinline__ void plane_fwd_body(const PlaneArgs& a, const FftPlan
     __syncthreads();
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    grec_n[x0] = min(done, a.rec_cap);
-    if (done > a.rec_cap) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
-  }
+  if (threadIdx.x == 0) grec_n[x0] = done;  // beyond rec_cap: the gather walks the candidates itself
   // Rows 2m and 2m + 1 become the real and imaginary part of packed line m (stride Kz | 1). The
   // packed lines overlay the fixed-point plane: every value is in registers before the first
   // store (pairs * Kz <= PLANE_REG * lanes, plane_lanes_ok).
@@ -770,7 +775,8 @@ __device__ __forceinline__ void plane_gather_body(const PlaneArgs& a, const FftP
   load_twiddles(twy, twy_g, a.Ky);
   // the records of the atoms touching this plane, written by the forward kernel; each lane's first
   // ones are loaded with the grid, the others GATHER_U at a time ahead of their use
-  const int nr = grec_n[x0];
+  const int touching = grec_n[x0];
+  const int nr = touching <= a.rec_cap ? touching : 0;
   const GatherRec* gin = grec + (long long)x0 * a.rec_cap;
   GatherRec rec[GATHER_U];
   auto fetch = [&](int e0) {
@@ -848,11 +854,23 @@ __device__ __forceinline__ void plane_gather_body(const PlaneArgs& a, const FftP
     for (int u = 0; u < GATHER_U; ++u)
       if (e0 + u * (int)blockDim.x < nr) share(now[u]);
   }
+  if (touching > a.rec_cap) {
+    // more atoms than records (a dense slab along x): every candidate again, as the forward kernel does
+    int b0, e0, b1, e1;
+    plane_ranges(a, cell_start, x0, &b0, &e0, &b1, &e1);
+    const int len0 = e0 - b0, total = len0 + (e1 - b1);
+    for (int c = threadIdx.x; c < total; c += blockDim.x) {
+      int by, bz, kx;
+      const GatherRec g = plane_record(a, sorted_orig, pos_sorted, xq, c < len0 ? b0 + c : b1 + (c - len0), x0, &by,
+                                       &bz, &kx);
+      if (kx <= 3) share(g);
+    }
+  }
   // every atom owns exactly one slot per kx: the grid-wide count must be 4 n. One 64-bit add per
   // workgroup carries its slots (40 bits) and its arrival (above); the last of the Kx plane
   // workgroups (launches may hold others) checks the total and re-arms the counter.
   if (threadIdx.x == 0) {
-    const unsigned long long mine = (1ull << 40) + (unsigned)nr;
+    const unsigned long long mine = (1ull << 40) + (unsigned)touching;
     const unsigned long long all = atomicAdd(&st->pme_count, mine) + mine;
     if (all >> 40 == (unsigned)a.Kx) {
       if ((all & ((1ull << 40) - 1ull)) != 4ull * (unsigned)a.n) atomicOr(&st->flags, MDX_FLAG_PME_COVERAGE);
@@ -1114,7 +1132,8 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
     if (!c->pme_wf && plane_fwd_lds(c->K[1], c->K[2], W) <= budget) c->pme_wf = W;
   c->pme_planes = c->pme_wf > 0 && plane_gather_lds(c->K[1], c->K[2]) <= budget &&
                   plane_lanes_ok(c->K[1], c->K[2], PLANE_THREADS) && c->K[1] < 4096 && c->K[2] < 4096;
-  // gather records: each atom touches 4 of the Kx planes; room for twice the mean plus slack
+  // gather records: each atom touches 4 of the Kx planes; room for twice the mean plus slack (planes that
+  // more atoms touch do without)
   c->pme_rec_cap = (int)std::min<long long>(c->n, 8LL * c->n / c->K[0] + 4096);
   if ((rc = c->pme_grec.ensure((size_t)c->K[0] * c->pme_rec_cap * 6)) || (rc = c->pme_grec_n.ensure(c->K[0])))
     return rc;
