@@ -402,6 +402,7 @@ __device__ void prologue_block_end(const StepPro& P, DevState* st, double d2, bo
   __shared__ double sm[16];
   __shared__ int last;
   if (bad) atomicOr(&st->flags, MDX_FLAG_NONFINITE);
+  if (d2 != d2) d2 = INFINITY;  // a position that is not finite, now or at the build: the list is due
   for (int off = 32; off > 0; off >>= 1) d2 = fmax(d2, __shfl_xor(d2, off, 64));
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = d2;
   __syncthreads();

@@ -199,7 +199,12 @@ __device__ __forceinline__ int clamped_floor_index(double u, int n) {
 // build), xf the position as 32-bit fractions of the box with the same charge (pair kernels: the
 // wrapped difference of two fractions is the minimum image, to 2^-32 of an edge where centred
 // float32 positions carry 2^-24), and its float64 position (PME). iL: inverse edges.
-__device__ __forceinline__ void pack_atom(double x, double y, double z, float q, const double* L, const double* iL,
+//
+// A position that is not finite has no fraction: the atom stands at fraction 0, without charge in xf.
+// It is flagged where displacements are measured, which also makes the list due, and the fill of a
+// rebuild takes its LJ parameters (fill_slot), so the pair terms of the other atoms are those without
+// it. Returns whether the position is such a one.
+__device__ __forceinline__ bool pack_atom(double x, double y, double z, float q, const double* L, const double* iL,
                                           float4* __restrict__ xq_s, int4* __restrict__ xf_s,
                                           double* __restrict__ ps_s) {
   ps_s[0] = x;
@@ -208,16 +213,20 @@ __device__ __forceinline__ void pack_atom(double x, double y, double z, float q,
   const double p[3] = {x, y, z};
   double u[3];
   int f[3];
+  bool lost = false;
   for (int d = 0; d < 3; ++d) {
     // the primary image first (exact for a coordinate within one image): the same fraction for a
     // coordinate before and after it is wrapped
     u[d] = fma(-rint(p[d] * iL[d]), L[d], p[d]) * iL[d];
     u[d] -= floor(u[d]);
+    const bool some = u[d] >= 0.0;
+    lost |= !some;
     // the range is decided before the conversion (NaN, or a tiny negative coordinate rounding to 1)
-    f[d] = (int)(u[d] >= 0.0 && u[d] < 1.0 ? (unsigned)(u[d] * 4294967296.0) : 0u);
+    f[d] = (int)(some && u[d] < 1.0 ? (unsigned)(u[d] * 4294967296.0) : 0u);
   }
   *xq_s = make_float4((float)((u[0] - 0.5) * L[0]), (float)((u[1] - 0.5) * L[1]), (float)((u[2] - 0.5) * L[2]), q);
-  *xf_s = make_int4(f[0], f[1], f[2], __float_as_int(q));
+  *xf_s = make_int4(f[0], f[1], f[2], lost ? 0 : __float_as_int(q));
+  return lost;
 }
 
 struct mdx_ctx {
@@ -428,13 +437,13 @@ struct FillArgs {
 __device__ inline void fill_slot(const FillArgs& f, int s, int o) {
   f.orig_sorted[o] = s;
   for (int d = 0; d < 3; ++d) f.pos_build[3 * o + d] = f.pos[3 * o + d];
-  pack_atom(f.pos[3 * o], f.pos[3 * o + 1], f.pos[3 * o + 2], f.qs ? f.qs[o] : 0.f, f.L, f.iL, &f.xq[s], &f.xf[s],
-            &f.pos_sorted[3 * s]);
+  const bool lost = pack_atom(f.pos[3 * o], f.pos[3 * o + 1], f.pos[3 * o + 2], f.qs ? f.qs[o] : 0.f, f.L, f.iL,
+                              &f.xq[s], &f.xf[s], &f.pos_sorted[3 * s]);
   if (f.lj64) {
     double e = f.lj64[4 * o + 0], sg = f.lj64[4 * o + 1], e14 = f.lj64[4 * o + 2], s14 = f.lj64[4 * o + 3];
     // (sigma/2, sqrt(24 eps)): a pair's 24 eps_ij is one product
-    f.ljs[s] = make_float2((float)(0.5 * sg), (float)sqrt(24.0 * e));
-    f.ljs14[s] = make_float2((float)(0.5 * s14), (float)sqrt(24.0 * e14));
+    f.ljs[s] = make_float2((float)(0.5 * sg), lost ? 0.f : (float)sqrt(24.0 * e));
+    f.ljs14[s] = make_float2((float)(0.5 * s14), lost ? 0.f : (float)sqrt(24.0 * e14));
   }
   if (f.ref_lin) {
     int lin = f.ref_lin[o];

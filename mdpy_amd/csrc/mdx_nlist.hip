@@ -245,6 +245,7 @@ __global__ void k_check_disp(const double* __restrict__ pos, const double* __res
     }
   }
   if (bad) atomicOr(&st->flags, MDX_FLAG_NONFINITE);
+  if (d2 != d2) d2 = INFINITY;  // a position that is not finite, now or at the build: the list is due
   for (int off = 32; off > 0; off >>= 1) d2 = fmax(d2, __shfl_xor(d2, off, 64));
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = d2;
   __syncthreads();
