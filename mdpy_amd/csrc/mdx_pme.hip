@@ -799,12 +799,16 @@ __device__ __forceinline__ void plane_gather_body(const PlaneArgs& a, const FftP
     o = f == r ? o : r;
     r = f;
     if (axis) break;
-    // rows 2m and 2m + 1 again as one packed line, Z = X_2m + i X_2m+1 over the whole period
+    // rows 2m and 2m + 1 again as one packed line, Z = X_2m + i X_2m+1 over the whole period. The
+    // coefficients of k = 0 and k = Kz/2 are real but for rounding; packed, the imaginary part of one row's
+    // would go to the other, with opposite signs, which a force along y sees in full (reciprocal
+    // forces of 30,021 atoms, 72^3: 3.2e-6 of their size off, 0.9e-6 without it)
     for (int idx = threadIdx.x; idx < pairs * nz; idx += blockDim.x) {
       const int m = (int)(((float)idx + 0.5f) * inz), k = idx - m * nz;
       const float2 p = r[2 * m * nz + k], q = 2 * m + 1 < a.Ky ? r[(2 * m + 1) * nz + k] : make_float2(0.f, 0.f);
-      o[m * ls + k] = make_float2(p.x - q.y, p.y + q.x);
-      if (k > 0 && 2 * k != a.Kz) o[m * ls + a.Kz - k] = make_float2(p.x + q.y, q.x - p.y);
+      const bool real = k == 0 || 2 * k == a.Kz;
+      o[m * ls + k] = real ? make_float2(p.x, q.x) : make_float2(p.x - q.y, p.y + q.x);
+      if (!real) o[m * ls + a.Kz - k] = make_float2(p.x + q.y, q.x - p.y);
     }
     __syncthreads();
     float2* h = o;
