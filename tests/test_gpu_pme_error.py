@@ -32,3 +32,37 @@ def test_long_waves_against_float64(waters, cutoff, grid):
     # the potential); pairs of rows along y share a transform, which must not show in the y component:
     # with the imaginary rounding of real coefficients it was 3 to 5 times the x component's
     assert np.all(err <= 50 * 2.0 ** -24) and err[1] <= 1.5 * err[0], err
+
+
+def test_reciprocal_energy_against_float64():
+    """The spread conserves charge (an error in a spread charge's sum is a long wave, to which the energy is
+    most sensitive): root mean square error over boxes whose lattice has vacancies."""
+    from mdpy_amd import _lib as L, systems
+    from mdpy_amd.engine import Engine, beta_from_tolerance
+    from mdpy_amd.unit import ONE_OVER_4PI_EPS0
+    from oracle import ewald as EW
+    waters, grid, err, size = 2000, (40, 40, 40), [], []
+    edge = (waters / 0.0334) ** (1 / 3)
+    beta = beta_from_tolerance(12.0, 1e-5)
+    for seed in range(4):
+        s = systems.water_box(13, edge / 13, n_waters=waters, seed=seed, cutoff=12.0, pme_grid=grid)
+        n, q = s.num_atoms, np.asarray(s.charges)
+        e = Engine.bare(n, s.box, positions=s.positions)
+        e.set_masses(s.masses)
+        e.set_charges(q)
+        e.set_lj(s.lj)
+        e.set_exclusions(np.zeros(n + 1, int), [])
+        e.set_scaling(np.zeros(n + 1, int), [])
+        e.configure_nonbonded(9.0, skin=1.0)
+        e.configure_pme(grid, beta)
+        got = e.compute(L.TERM_COUL_RECIP)[1]["coulomb_reciprocal"]
+        e.close()
+        Er = EW.spme_reciprocal(s.positions, q, s.box, grid, 4, beta, ONE_OVER_4PI_EPS0)[1]
+        self_e = -ONE_OVER_4PI_EPS0 * beta / math.sqrt(math.pi) * (q * q).sum()
+        err.append(got - (Er + self_e))
+        size.append(Er)
+    rel = math.sqrt(np.mean(np.square(err)) / np.mean(np.square(size)))
+    print("case: energy of 2,000 waters, relative error %.2e" % rel, flush=True)
+    # the energy is quadratic in the spread charges, whose float32 roundings (2^-24) otherwise average out
+    # over the atoms; weights whose sum is off by their own roundings gave 2.6e-7
+    assert rel <= 2 * 2.0 ** -24
