@@ -207,11 +207,11 @@ int mdx_enqueue_nonbonded(mdx_ctx* c, bool lj, bool coul, bool energy, unsigned 
 #define PC_U 4  // partners in flight per lane
 #define PC_WAVES_PER_SIMD 4
 
-// 1/sqrt(x) in float64 from the hardware estimate (x = 0 is moved to the smallest normal, so
-// coincident charges give the huge energy and NaN force that 1/0 gives)
+// 1/sqrt(x) in float64 from the hardware estimate. The estimate is of the smallest normal where x = 0, so
+// coincident charges give the huge energy and NaN force that 1/0 gives; the step takes x itself, so
+// NaN (which fmax would replace) stays NaN.
 __device__ __forceinline__ double rsqrt64(double x) {
-  x = fmax(x, 2.2250738585072014e-308);
-  const double y = __builtin_amdgcn_rsq(x);
+  const double y = __builtin_amdgcn_rsq(fmax(x, 2.2250738585072014e-308));
   const double e = fma(-x * y, y, 1.0);
   return fma(y * e, fma(0.375, e, 0.5), y);
 }

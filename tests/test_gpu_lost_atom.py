@@ -102,3 +102,26 @@ def test_other_atoms_move_without_it():
     others = np.arange(N) != k
     moved = np.abs(got[0] - x)[others].max()
     assert np.abs(got[1] - got[0])[others].max() <= 1e-4 * moved
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("charged", [True, False])
+def test_plain_coulomb(value, charged):
+    """All pairs: a charged atom without a position leaves no sum with a value (nothing is added, where a
+    clamped distance added the largest numbers there are), one without charge changes nothing."""
+    from mdpy_amd import _lib as L
+    k = N // 2
+    print("case: plain Coulomb, %s, %s" % (value, "charged" if charged else "no charge"), flush=True)
+    x, q, lj = system(None if charged else k)
+    bad = x.copy()
+    bad[k, 1] = value
+    out = []
+    for p in (x, bad):
+        e = engine(p, q, lj, 1.0)
+        F, en = e.compute(L.TERM_COUL_PLAIN)
+        out.append((F.cpu().numpy().copy(), en["coulomb_plain"]))
+        e.close()
+    if charged:
+        assert not out[1][0].any() and out[1][1] == 0.0
+    else:
+        assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
