@@ -290,14 +290,15 @@ int mdx_stats_fetch(mdx_ctx* ctx, int64_t* h_rebuilds, int64_t* h_evals);
  * next evaluation rebuilds in full), 6 / 7 / 8 = the PME plane forward kernel / x-axis pass /
  * inverse + gather kernel alone. Synchronises. */
 int mdx_time_kernel(mdx_ctx* ctx, int which, unsigned terms, int reps, double* h_avg_ms);
-/* Lanes per atom of the nonbonded kernel: 16, 32 or 64 set directly, or 0 = time each variant
- * on the current neighbour list (`reps` forces-only launches of `terms`' LJ/direct parts) and
- * keep the fastest. The choice goes to *h_lanes (may be NULL). Synchronises. */
+/* Lanes per atom of the nonbonded kernel: 16, 32 or 64 set directly, 0 = time each variant on
+ * the current neighbour list (`reps` forces-only launches of `terms`' LJ/direct parts) and keep
+ * the fastest, or -1 = chosen by system size, as before the first call. The choice goes to
+ * *h_lanes (may be NULL). Synchronises with 0. */
 int mdx_nonbonded_tune(mdx_ctx* ctx, unsigned terms, int lanes, int reps, int* h_lanes);
 /* Resident nonbonded workgroups (no reference counterpart): per_cu > 0 launches per_cu
  * workgroups per compute unit that loop over the nonbonded work; 0 launches one workgroup per
- * unit of work. Default: 3 where that gives each at most two units, else 0 (the measured best
- * beside the concurrent PME kernels). Same forces either way. */
+ * unit of work; -1, the default: 3 where that gives each at most two units, else 0 (the measured
+ * best beside the concurrent PME kernels). Same forces either way. */
 int mdx_nonbonded_persist(mdx_ctx* ctx, int per_cu);
 /* Scheduled list rebuilds (no reference counterpart): every > 0 also rebuilds the neighbour
  * list in the integrator step whose step counter is a multiple of `every`, besides the rebuilds

@@ -2310,28 +2310,35 @@ extern "C" int mdx_pair_counts(mdx_ctx* c, int64_t* h_list_slots, int64_t* h_uni
 // 3 one integrator step of `terms`.
 extern "C" int mdx_nonbonded_tune(mdx_ctx* c, unsigned terms, int lanes, int reps, int* h_lanes) {
   MDX_CHECK(c && c->nb_configured, MDX_ERR_INVALID, "mdx_nonbonded_tune: nonbonded not configured");
-  MDX_CHECK(lanes == 0 || lanes == 16 || lanes == 32 || lanes == 64, MDX_ERR_INVALID, "lanes must be 0, 16, 32 or 64");
+  MDX_CHECK(lanes == -1 || lanes == 0 || lanes == 16 || lanes == 32 || lanes == 64, MDX_ERR_INVALID,
+            "lanes must be -1, 0, 16, 32 or 64");
   int best = lanes;
   if (lanes == 0) {
     double best_ms = 1e300;
-    const int cand[3] = {16, 32, 64};
+    const int cand[3] = {16, 32, 64}, lanes0 = c->nb_lanes;
+    const bool set0 = c->nb_lanes_set;
     c->nb_lanes_set = true;
     for (int k = 0; k < 3; ++k) {
       c->nb_lanes = cand[k];
       double ms = 0;
       int rc = mdx_time_kernel(c, 0, terms, reps, &ms);
-      if (rc) return rc;
+      if (rc) {  // nothing was chosen
+        c->nb_lanes = lanes0;
+        c->nb_lanes_set = set0;
+        return rc;
+      }
       if (ms < best_ms) {
         best_ms = ms;
         best = cand[k];
       }
     }
   }
+  c->nb_lanes_set = lanes != -1;
+  if (lanes == -1) best = mdx_nb_lanes(c);
+  else c->nb_lanes = best;
   // the timing runs ended with the last candidate: captured steps hold the launch shape
   // they were captured with, so they are dropped only when that differs from the choice
   if (best != c->graph_lanes) mdx_invalidate_graph(c);
-  c->nb_lanes = best;
-  c->nb_lanes_set = true;
   if (h_lanes) *h_lanes = best;
   return 0;
 }
@@ -2356,7 +2363,7 @@ extern "C" int mdx_nonbonded_cells(mdx_ctx* c, int per_radius) {
 }
 
 extern "C" int mdx_nonbonded_persist(mdx_ctx* c, int per_cu) {
-  MDX_CHECK(c && per_cu >= 0, MDX_ERR_INVALID, "mdx_nonbonded_persist: bad arguments");
+  MDX_CHECK(c && per_cu >= -1, MDX_ERR_INVALID, "mdx_nonbonded_persist: bad arguments");
   c->nb_persist = c->ncu > 0 ? per_cu : 0;
   mdx_invalidate_graph(c);
   return 0;

@@ -264,13 +264,15 @@ class Engine:
         return a.value, b.value
 
     def tune_nonbonded(self, terms, lanes=0, reps=20):
-        """Lanes per atom of the nonbonded kernel (0 = time 16/32/64 on the current list)."""
+        """Lanes per atom of the nonbonded kernel (0 = time 16/32/64 on the current list, -1 = by
+        system size, the default)."""
         out = ctypes.c_int()
         L.call("mdx_nonbonded_tune", self.ctx, int(terms), int(lanes), int(reps), ctypes.byref(out))
         return out.value
 
     def set_nonbonded_persist(self, per_cu):
-        """Nonbonded workgroups per compute unit looping over the work (0: one per unit of work)."""
+        """Nonbonded workgroups per compute unit looping over the work (0: one per unit of work,
+        -1, the default: by the amount of work)."""
         L.call("mdx_nonbonded_persist", self.ctx, int(per_cu))
 
     def set_rebuild_every(self, every):
