@@ -73,7 +73,9 @@ int mdx_ctx_destroy(mdx_ctx* ctx);
 int mdx_ctx_set_stream(mdx_ctx* ctx, void* hip_stream);
 
 /* ---- system (State / Topology.join, mdpy/core/state.py:19-28, topology.py:59-80) --------- */
-/* Bind caller-owned device arrays: positions (N*3 f64), velocities (N*3 f64). `h_box` = 3 edges. */
+/* Bind caller-owned device arrays: positions (N*3 f64), velocities (N*3 f64). `h_box` = 3 edges.
+ * Another number of atoms than before drops the parameters, exclusions, terms and configurations
+ * set so far. */
 int mdx_system_set(mdx_ctx* ctx, int n_atoms, double* d_pos, double* d_vel, const double* h_box);
 int mdx_set_box(mdx_ctx* ctx, const double* h_box);
 /* Per-atom data from host arrays (copied): masses (N), charges (N, e), LJ (N*4: eps, sigma,

@@ -881,6 +881,10 @@ extern "C" int mdx_system_set(mdx_ctx* c, int n, double* d_pos, double* d_vel, c
     c->nb_configured = false;
     c->pme_configured = false;
     c->int_primed = false;
+    // per-atom parameters and buffers and the terms' atom indices are the old system's
+    c->int_configured = false;
+    c->has_mass = c->has_charges = c->has_lj = c->has_excl = c->has_s14 = c->win_ready = false;
+    c->n_excl_pairs = c->nb = c->na = c->nd = c->ni = 0;
   }
   MDX_HIP(hipMemset(c->ffix.p, 0, 3 * sizeof(long long) * n));
   int one = 1;
