@@ -1714,7 +1714,7 @@ extern "C" int mdx_integrate(mdx_ctx* c, unsigned terms, int nsteps, int use_gra
 // replicas' arguments in device tables (BatchKind); steps 1 .. n-1 of a call replay graphs of
 // such launches captured on the lead stream, the PME planes forked onto the batch's side stream.
 struct BatchFused {
-  BatchKind pro, fill, lfast, lcell, pfwd, pfft, pgat, nb;
+  BatchKind pro, fill, list, pfwd, pfft, pgat, nb;
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hipGraphExec_t gf[MDX_NGRAPH_SIZES] = {};
@@ -1797,7 +1797,7 @@ extern "C" int mdx_batch_destroy(mdx_batch* b) {
   if (b->fz.ev_fork) hipEventDestroy(b->fz.ev_fork);
   if (b->fz.ev_join) hipEventDestroy(b->fz.ev_join);
   if (b->fz.side) hipStreamDestroy(b->fz.side);
-  for (BatchKind* k : {&b->fz.pro, &b->fz.fill, &b->fz.lfast, &b->fz.lcell, &b->fz.pfwd, &b->fz.pfft, &b->fz.pgat,
+  for (BatchKind* k : {&b->fz.pro, &b->fz.fill, &b->fz.list, &b->fz.pfwd, &b->fz.pfft, &b->fz.pgat,
                        &b->fz.nb})
     k->buf.release();
   for (hipEvent_t e : b->ev_out)
@@ -1861,7 +1861,7 @@ static int fused_prepare(mdx_batch* b, unsigned terms) {
   }
   int rc;
   if ((rc = batch_kind_upload(&f.pro, pro, pblocks, plds)) ||
-      (rc = mdx_batch_prepare_list(b->ctx.data(), n, &f.fill, &f.lfast, &f.lcell)) ||
+      (rc = mdx_batch_prepare_list(b->ctx.data(), n, &f.fill, &f.list)) ||
       (rc = mdx_batch_prepare_pme(b->ctx.data(), n, &f.pfwd, &f.pfft, &f.pgat)) ||
       (rc = mdx_batch_prepare_nb(b->ctx.data(), n, terms & (kFusedBonded | MDX_TERM_COUL_RECIP), &f.nb)))
     return rc;
@@ -1898,7 +1898,7 @@ static int fused_step(mdx_batch* b, bool energy, bool fuse_prev) {
   MDX_HIP(hipStreamWaitEvent(f.side, f.ev_fork, 0));
   if ((rc = mdx_batch_launch_pme(f.pfwd, f.pfft, f.pgat, f.side))) return rc;
   MDX_HIP(hipEventRecord(f.ev_join, f.side));
-  if ((rc = mdx_batch_launch_list(f.lfast, f.lcell, s)) || (rc = mdx_batch_launch_nb(f.nb, f.s14, energy, s)))
+  if ((rc = mdx_batch_launch_list(f.list, s)) || (rc = mdx_batch_launch_nb(f.nb, f.s14, energy, s)))
     return rc;
   MDX_HIP(hipStreamWaitEvent(s, f.ev_join, 0));
   return 0;
@@ -2585,7 +2585,7 @@ extern "C" int mdx_batch_time_kernel(mdx_batch* b, int which, int reps, double* 
         if ((rc = on_lead(b, c, [&]() { return mdx_enqueue_request_rebuild(c); }))) break;
       if (rc) break;
       MDX_HIP(hipEventRecord(k.e0, s));
-      if ((rc = mdx_batch_launch_list(f.lfast, f.lcell, s))) break;
+      if ((rc = mdx_batch_launch_list(f.list, s))) break;
       MDX_HIP(hipEventRecord(k.e1, s));
       MDX_HIP(hipEventSynchronize(k.e1));
       float ms = 0;

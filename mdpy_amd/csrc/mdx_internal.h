@@ -542,9 +542,9 @@ int mdx_nb_lanes(const mdx_ctx* c);  // lanes per atom of the nonbonded kernel
 // PME exclusion correction with MDX_TERM_COUL_RECIP) ride along as extra workgroups
 int mdx_enqueue_nonbonded(mdx_ctx* c, bool lj, bool coul, bool energy, unsigned bonded_terms = 0u);
 // batched replicas (MDX_BATCH_FUSED): each kind's per-replica records, and its launches
-int mdx_batch_prepare_list(mdx_ctx* const* cs, int n, BatchKind* fill, BatchKind* fast, BatchKind* cell);
+int mdx_batch_prepare_list(mdx_ctx* const* cs, int n, BatchKind* fill, BatchKind* list);
 int mdx_batch_launch_fill(const BatchKind& k, hipStream_t s);
-int mdx_batch_launch_list(const BatchKind& fast, const BatchKind& cell, hipStream_t s);
+int mdx_batch_launch_list(const BatchKind& k, hipStream_t s);
 int mdx_batch_prepare_pme(mdx_ctx* const* cs, int n, BatchKind* fwd, BatchKind* fft, BatchKind* gat);
 int mdx_batch_launch_pme(const BatchKind& fwd, const BatchKind& fft, const BatchKind& gat, hipStream_t s,
                          unsigned parts = 7u);  // bits: forward, x-axis pass, inverse + gather

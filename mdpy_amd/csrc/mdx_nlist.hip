@@ -8,7 +8,7 @@
 // The force kernels do not walk the reference's dense cell table: atoms are binned into a
 // periodic grid of cells at least (rc + skin)/2 wide, sorted by cell (ascending original id
 // inside a cell, so every order is deterministic), and each atom gets a full neighbour list
-// (column-major, one lane per atom in the force kernel). In REFERENCE mode the list also drops
+// (one row of entries per atom). In REFERENCE mode the list also drops
 // pairs whose mdpy cells are not stencil neighbours, reproducing the reference's pair set.
 #include "mdx_internal.h"
 #include <algorithm>
@@ -384,7 +384,6 @@ struct ListArgs {
   int n;
   int cap;
   float rl2;          // list radius squared (float pre-filter)
-  int exact64;        // decide r <= rc in float64 (skin == 0)
   double rc;
   int ref_mode;       // REFERENCE stencil filter
   int rnx, rny, rnz;  // reference grid
@@ -406,9 +405,9 @@ __device__ __forceinline__ int cyc_dist(int a, int b, int n) {
 // periodic cell once, on no more than one side), so the scan needs no minimum-image arithmetic.
 // Exclusions and 1-4 partners within 32 atom indices of the home atom are bits of two 64-bit
 // masks; an atom with a partner outside that window scans its CSR lists (staged in LDS) instead.
-// Each lane tests BL_U candidates per pass, all LDS reads issued first. FAST instantiations
-// (shifted candidates, exact pair mode, masks present) compile out the reference-mode filter and
-// the minimum image; the float64 decision of skin-0 lists is the EXACT64 instantiation.
+// Each lane tests BL_U candidates per pass, all LDS reads issued first; r <= rc is decided in float64
+// (lists without a skin). FAST instantiations (shifted candidates, exact pair mode, masks present)
+// compile out the reference-mode filter and the minimum image.
 #ifndef BL_CH
 #define BL_CH 1024  // candidates staged per chunk (a multiple of the fast kernel's pass)
 #endif
@@ -448,7 +447,7 @@ struct ListCall {
 };
 
 // the build of home cell `cell`
-template <bool EXACT64, bool FAST>
+template <bool FAST>
 __device__ __forceinline__ void build_list_cell_body(const ListCall& L, const int cell) {
   const ListArgs& a = L.a;
   const float4* __restrict__ xq = L.xq;
@@ -647,12 +646,7 @@ __device__ __forceinline__ void build_list_cell_body(const ListCall& L, const in
         if (g == 0 && (nex_all > BL_MAXEX || ns4_all > BL_MAXEX)) atomicOr(&st->flags, MDX_FLAG_OVERFLOW);
       }
       const int rci = (!FAST && a.ref_mode) ? ref_cell_sorted[s] : 0;
-      double pi[3] = {0.0, 0.0, 0.0};
-      if (EXACT64) {
-        pi[0] = pos[3 * o];
-        pi[1] = pos[3 * o + 1];
-        pi[2] = pos[3 * o + 2];
-      }
+      const double pi[3] = {pos[3 * o], pos[3 * o + 1], pos[3 * o + 2]};
       wave_lds_sync();  // the group's lanes are in one wave
       unsigned* row = nbr_list + (long long)s * a.cap;
       int cnt = acnt[h];
@@ -695,7 +689,7 @@ __device__ __forceinline__ void build_list_cell_body(const ListCall& L, const in
             const int az = cyc_dist(rci & 1023, rcj[u] & 1023, a.rnz);
             acc &= (ax <= 1) & (ay <= 1) & (az <= 1);
           }
-          if (EXACT64 && acc) {  // float64 decision with the reference's sequence (pbc.py:40-44)
+          if (acc) {  // float64 decision with the reference's sequence (pbc.py:40-44)
             double d[3];
             const double L[3] = {gr.Lx, gr.Ly, gr.Lz};
             for (int r = 0; r < 3; ++r) {
@@ -728,9 +722,9 @@ __device__ __forceinline__ void build_list_cell_body(const ListCall& L, const in
   }
 }
 
-template <bool EXACT64, bool FAST>
+template <bool FAST>
 __global__ __launch_bounds__(BL_THREADS) void k_build_list_cell(ListCall L) {
-  build_list_cell_body<EXACT64, FAST>(L, blockIdx.x);
+  build_list_cell_body<FAST>(L, blockIdx.x);
 }
 
 // The common case of the build above as its own kernel: exact pair mode, float32 list radius, and
@@ -1103,19 +1097,13 @@ __global__ __launch_bounds__(BL_THREADS) void k_build_list_fast(ListCall L) {
   build_list_fast_body<WRAP>(L, blockIdx.x, sh);
 }
 
-// every replica's list build in one launch (the fast build, or the cell build of a replica whose
-// exclusions have no window masks)
+// every replica's list build in one launch
 __global__ __launch_bounds__(BL_THREADS) void k_build_list_fast_batch(BatchMap map, const ListCall* __restrict__ calls) {
   __shared__ BlfShared sh;
   int block;
   const int r = batch_replica(map, &block);
   if (calls[r].a.shifted) build_list_fast_body<false>(calls[r], block, sh);
   else build_list_fast_body<true>(calls[r], block, sh);
-}
-__global__ __launch_bounds__(BL_THREADS) void k_build_list_cell_batch(BatchMap map, const ListCall* __restrict__ calls) {
-  int cell;
-  const int r = batch_replica(map, &cell);
-  build_list_cell_body<false, false>(calls[r], cell);
 }
 
 __global__ void k_request_rebuild(DevState* st) { st->rebuild = 1; }
@@ -1287,8 +1275,8 @@ static int blf_split(const mdx_ctx* c) {
   return s;
 }
 
-// The list-build launch of a context: its arguments and kernel (0: the fast build; 1-3: the cell
-// build <EXACT64, FAST> = <false,false>, <true,false>, <true,true>).
+// The list-build launch of a context: its arguments and kernel (0: the fast build, of every list with a
+// skin; 1, 2: the cell build, general and FAST).
 static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   const bool ref = c->pair_mode == MDX_PAIRS_REFERENCE;
   ListArgs& a = L->a;
@@ -1297,7 +1285,6 @@ static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   a.cap = c->nbr_cap;
   double rl = c->rc + c->skin;
   a.rl2 = (float)(rl * rl) * (1.0f + 1e-5f);
-  a.exact64 = c->skin > 0 ? 0 : 1;
   a.rc = c->rc;
   a.ref_mode = ref ? 1 : 0;
   a.rnx = c->ref_n[0];
@@ -1311,8 +1298,8 @@ static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   for (int d = 0; d < 3; ++d)
     if (2 * c->reach[d] + 1 >= c->gn[d]) a.shifted = 0;
   const bool win = c->win_ready && c->h_win_bad.size() == (size_t)c->n;
-  const bool masks = win || !(c->has_excl || c->has_s14);  // without either only the atom itself is masked
-  const bool fast = masks && !a.ref_mode && !a.exact64;
+  // set with the exclusions and 1-4 pairs; without either only the atom itself is masked
+  MDX_CHECK(win || !(c->has_excl || c->has_s14), MDX_ERR_INVALID, "exclusions without their window masks");
   L->xq = c->xq.p;
   L->xf = c->xf.p;
   L->sorted_orig = c->sorted_orig.p;
@@ -1333,7 +1320,7 @@ static int list_call(mdx_ctx* c, ListCall* L, int* kind) {
   L->st = c->dstate.p;
   L->thr2 = rebuild_thr2(c);
   L->split = blf_split(c);
-  *kind = fast ? 0 : (!a.exact64 ? 1 : (win && a.shifted && !a.ref_mode ? 3 : 2));
+  *kind = c->skin > 0 ? 0 : (win && a.shifted && !a.ref_mode ? 2 : 1);  // reference mode has no skin
   return 0;
 }
 
@@ -1350,9 +1337,8 @@ int mdx_nlist_update_list(mdx_ctx* c) {
       else k_build_list_fast<true><<<grid, block, 0, c->stream>>>(L);
       break;
     }
-    case 1: k_build_list_cell<false, false><<<grid, block, 0, c->stream>>>(L); break;
-    case 2: k_build_list_cell<true, false><<<grid, block, 0, c->stream>>>(L); break;
-    default: k_build_list_cell<true, true><<<grid, block, 0, c->stream>>>(L); break;
+    case 1: k_build_list_cell<false><<<grid, block, 0, c->stream>>>(L); break;
+    default: k_build_list_cell<true><<<grid, block, 0, c->stream>>>(L); break;
   }
   MDX_LAUNCH_CHECK();
   return 0;
@@ -1367,10 +1353,10 @@ __global__ __launch_bounds__(256) void k_grid_sort_fill_batch(BatchMap map, cons
   grid_sort_fill_block(f, cell);
 }
 
-int mdx_batch_prepare_list(mdx_ctx* const* cs, int n, BatchKind* fill, BatchKind* fast, BatchKind* cell) {
+int mdx_batch_prepare_list(mdx_ctx* const* cs, int n, BatchKind* fill, BatchKind* list) {
   std::vector<FillArgs> fa;
-  std::vector<ListCall> lf, lc;
-  std::vector<int> bfa, bf, bc;
+  std::vector<ListCall> lc;
+  std::vector<int> bfa, bl;
   for (int r = 0; r < n; ++r) {
     mdx_ctx* c = cs[r];
     fa.push_back(fill_args(c, rebuild_thr2(c)));
@@ -1378,17 +1364,12 @@ int mdx_batch_prepare_list(mdx_ctx* const* cs, int n, BatchKind* fill, BatchKind
     ListCall L;
     int kind, rc = list_call(c, &L, &kind);
     if (rc) return rc;
-    MDX_CHECK(kind <= 1, MDX_ERR_INVALID, "replica %d: batched steps need a list radius larger than the pair cutoff", r);
-    // every replica holds a place in both builds (zero workgroups in the one it does not use)
-    lf.push_back(L);
+    MDX_CHECK(kind == 0, MDX_ERR_INVALID, "replica %d: batched steps need a list radius larger than the pair cutoff", r);
     lc.push_back(L);
-    bf.push_back(kind == 0 ? c->ncell * L.split : 0);
-    bc.push_back(kind == 1 ? c->ncell : 0);
+    bl.push_back(c->ncell * L.split);
   }
   int rc;
-  if ((rc = batch_kind_upload(fill, fa, bfa, 0)) || (rc = batch_kind_upload(fast, lf, bf, 0)) ||
-      (rc = batch_kind_upload(cell, lc, bc, 0)))
-    return rc;
+  if ((rc = batch_kind_upload(fill, fa, bfa, 0)) || (rc = batch_kind_upload(list, lc, bl, 0))) return rc;
   return 0;
 }
 
@@ -1399,15 +1380,9 @@ int mdx_batch_launch_fill(const BatchKind& k, hipStream_t s) {
   return 0;
 }
 
-int mdx_batch_launch_list(const BatchKind& fast, const BatchKind& cell, hipStream_t s) {
-  if (fast.blocks) {
-    k_build_list_fast_batch<<<fast.blocks, BL_THREADS, 0, s>>>(fast.map, (const ListCall*)fast.calls);
-    MDX_LAUNCH_CHECK();
-  }
-  if (cell.blocks) {
-    k_build_list_cell_batch<<<cell.blocks, BL_THREADS, 0, s>>>(cell.map, (const ListCall*)cell.calls);
-    MDX_LAUNCH_CHECK();
-  }
+int mdx_batch_launch_list(const BatchKind& k, hipStream_t s) {
+  k_build_list_fast_batch<<<k.blocks, BL_THREADS, 0, s>>>(k.map, (const ListCall*)k.calls);
+  MDX_LAUNCH_CHECK();
   return 0;
 }
 
