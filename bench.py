@@ -272,18 +272,18 @@ def batch_rooflines(b, reps):
         sl, pr = e.pair_counts()
         slots += sl
         pairs += pr
-    k3 = fftb = 0
+    k3 = half = 0
     for s in reps:
         kx, ky, kz = (int(k) for k in s.pme_grid)
         k3 += kx * ky * kz
-        fftb += 2 * (4 * kx * ky * kz + 8 * ky * kz * (kx // 2 + 1))
+        half += kx * ky * (kz // 2 + 1)
     items = [
         ("k_nonbonded_batch", 0, 20, None),
-        ("k_step_pro_batch", 4, 20, 424 * n),
-        ("k_build_list_batch", 5, 5, 4 * slots + 24 * n),
-        ("k_pme_plane_fwd_batch", 6, 20, 16 * n + 4 * k3),
-        ("k_fft_axis_batch", 7, 20, fftb),
-        ("k_pme_plane_inv_gather_batch", 8, 20, 40 * n + 4 * k3),
+        ("k_step_pro_batch", 4, 20, 440 * n),
+        ("k_build_list_fast_batch", 5, 5, 4 * slots + 24 * n),
+        ("k_pme_plane_fwd_batch", 6, 20, 16 * n + 8 * half),
+        ("k_fft_x_batch", 7, 20, 20 * half),
+        ("k_pme_plane_inv_gather_batch", 8, 20, 40 * n + 8 * half),
     ]
     out = {"atoms": n, "list_slots": slots, "unique_pairs": pairs, "grid_points": k3}
     for name, which, nrep, nbytes in items:
@@ -307,17 +307,18 @@ def secondary_rooflines(e, s, terms, slots):
     stream (mdx_time_kernel): achieved = the kernel's algorithmic bytes / its launch time."""
     n = s.num_atoms
     kx, ky, kz = (int(k) for k in s.pme_grid)
-    k3 = kx * ky * kz
+    half = kx * ky * (kz // 2 + 1)  # complex values of the half spectrum
     items = [
-        ("k_pme_plane_fwd", 6, 50, 16 * n + 4 * k3,
-         "spreading: 16 B/atom (packed position + charge) + 4 B per grid point"),
-        ("k_fft_axis", 7, 50, 2 * (4 * k3 + 8 * ky * kz * (kx // 2 + 1)),
-         "x-axis transform pair + B.C multiply: 2 x (4 K^3 + 8 K^2 (K/2+1)) bytes"),
-        ("k_pme_plane_inv_gather", 8, 50, 40 * n + 4 * k3,
-         "gather: 40 B/atom (position, charge, force out) + 4 B per grid point"),
-        ("k_step_pro", 4, 50, 424 * n,
-         "424 B/atom: reads forces 24 + reciprocal planes 96 + x, v, a_prev, xi, build position 5x24 + "
-         "masses 16 + ids 8; writes x, v, a_prev, xi, zeroed forces 5x24 + packed copies 40"),
+        ("k_pme_plane_fwd", 6, 50, 16 * n + 8 * half,
+         "spreading: 16 B/atom (packed position + charge) + 8 B per half-spectrum value out"),
+        ("k_fft_x", 7, 50, 20 * half,
+         "x-axis transform pair + B.C multiply: each of the K^2 (K/2+1) half-spectrum values read and "
+         "written (8 B each) and its influence function read (4 B)"),
+        ("k_pme_plane_inv_gather", 8, 50, 40 * n + 8 * half,
+         "gather: 40 B/atom (position, charge, force out) + 8 B per half-spectrum value in"),
+        ("k_step_pro", 4, 50, 440 * n,
+         "440 B/atom: reads forces 24 + reciprocal planes 96 + x, v, a_prev, xi, build position 5x24 + "
+         "masses 16 + ids 8; writes x, v, a_prev, xi, zeroed forces 5x24 + packed copies 56"),
         ("k_build_list_fast", 5, 10, 4 * slots + 24 * n,
          "rebuild step: 4 B per list slot written + 24 B/atom of cell data read"),
     ]
