@@ -749,7 +749,8 @@ __global__ __launch_bounds__(BL_THREADS) void k_build_list_cell(ListCall L) {
 // k_build_list_cell.
 // Before (one home atom per wave pass, 40 vector and scalar instructions with 6 branches per test,
 // small boxes by k_build_list_cell) / now (us): 648 atoms 23 / 11, 2,592 r_c 12 92 / 24, 3,000 r_c 9
-// 75 / 23, 23,328 r_c 12 86 / 69, 98,304 r_c 12 285 / 226. The vector unit is busy 80 % of the time.
+// 75 / 23, 23,328 r_c 12 86 / 69, 98,304 r_c 12 285 / 226. The vector unit issues in 82 % of the
+// busy cycles (23,328 atoms, 24.1 M of 29.5 M).
 #define BLF_H 4
 #define BLF_WAVES (BL_THREADS / 64)
 struct BlfShared {

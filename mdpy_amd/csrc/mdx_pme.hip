@@ -1498,9 +1498,11 @@ __global__ __launch_bounds__(BS) void k_pme_plane_inv_gather_batch(BatchMap map,
   plane_gather_body(p.a, p.plz, p.ply, p.twz, p.twy, p.sorted_orig, p.cell_start, p.pos_sorted, p.xq, p.cg, p.grec,
                     p.grec_n, p.fpart, p.st, x0, lds);
 }
-// Without 64 x 64 planes the batched forward kernel runs 256-lane workgroups with a window of
-// 1,024 candidates (more planes in flight: 109 vs 133 us over the 64 water replicas); the gather
-// keeps PLANE_THREADS lanes (159 us, against 172 with 256 lanes and 180 with 512).
+// The batched forward kernel runs 256-lane workgroups with a window of 1,024 candidates where every
+// replica's planes fit their registers (plane_lanes_ok: 2,048 packed values, 64 x 64 points): more planes
+// in flight, 54 us against 113 with PLANE_THREADS lanes over 64 water replicas (321,897 atoms), 4.35
+// against 4.07e8 atom-steps/s. The gather keeps PLANE_THREADS lanes: alone 71 us, 35 with 256 lanes and
+// 40 with 512, but a whole step waits for the nonbonded kernel beside it (4.35, 4.36 and 4.32e8).
 #define PLANE_BATCH_SMALL 256
 #define PLANE_BATCH_W 1024
 
