@@ -326,6 +326,7 @@ struct mdx_ctx {
   DevBuf<double> fpart;          // plane path: reciprocal force per (kx, atom), 4 x 3N
   bool pme_planes = false;       // plane kernels usable (list grid present, plane fits LDS)
   int pme_wf = 0;                // candidate window of the forward plane kernel
+  int pme_x_lines = 0;           // lines per workgroup of the x-axis pass
   int pme_rec_cap = 0;           // gather records per plane
   DevBuf<int> pme_grec;          // gather records (6 words each), pme_rec_cap per plane
   DevBuf<int> pme_grec_n;        // records per plane

@@ -1135,6 +1135,8 @@ extern "C" int mdx_pme_config(mdx_ctx* c, const int* h_grid, int order, double b
   int lds_max = 0;
   MDX_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
   const size_t budget = lds_max > 1024 ? (size_t)lds_max - 1024 : 0;  // static LDS of the kernels
+  c->pme_x_lines = FFTX_B;  // fewer where that many long lines don't fit (grids elongated along x)
+  while (c->pme_x_lines > 1 && x_pass_lds(c->K[0], c->pme_x_lines) > budget) c->pme_x_lines /= 2;
   c->pme_wf = 0;
   for (int W = 8192; W >= PLANE_THREADS; W -= PLANE_THREADS)
     if (!c->pme_wf && plane_fwd_lds(c->K[1], c->K[2], W) <= budget) c->pme_wf = W;
@@ -1324,7 +1326,7 @@ static int pme_enqueue_planes(mdx_ctx* c, unsigned parts = 7u) {
     MDX_LAUNCH_CHECK();
   }
   if (parts & 2u) {  // x forward, * B C, energy, x inverse
-    const XPass xp = x_pass_of(c, FFTX_B);
+    const XPass xp = x_pass_of(c, c->pme_x_lines);
     k_fft_x<<<div_up(xp.nl, xp.B), FFTX_THREADS, x_pass_lds(Kx, xp.B), c->stream>>>(xp, c->twiddle.p, c->cgrid.p,
                                                                                    c->bch.p, c->efix.p + 2);
     MDX_LAUNCH_CHECK();
@@ -1542,14 +1544,14 @@ int mdx_batch_prepare_pme(mdx_ctx* const* cs, int n, BatchKind* fwd, BatchKind* 
     lf = std::max(lf, plane_fwd_lds(c->K[1], c->K[2], p.a.W));
     lg = std::max(lg, plane_gather_lds(c->K[1], c->K[2]));
     FftCall f;
-    f.xp = x_pass_of(c, FFTX_B);
+    f.xp = x_pass_of(c, c->pme_x_lines);
     f.tw = c->twiddle.p;
     f.cg = c->cgrid.p;
     f.bc = c->bch.p;
     f.eslot = c->efix.p + 2;
     fc.push_back(f);
     bf.push_back(div_up(f.xp.nl, f.xp.B));
-    lx = std::max(lx, x_pass_lds(c->K[0], FFTX_B));
+    lx = std::max(lx, x_pass_lds(c->K[0], f.xp.B));
   }
   const void* kf = fthreads == PLANE_THREADS ? (const void*)k_pme_plane_fwd_batch<PLANE_THREADS>
                                              : (const void*)k_pme_plane_fwd_batch<PLANE_BATCH_SMALL>;

@@ -66,3 +66,31 @@ def test_reciprocal_energy_against_float64():
     # the energy is quadratic in the spread charges, whose float32 roundings (2^-24) otherwise average out
     # over the atoms; weights whose sum is off by their own roundings gave 2.6e-7
     assert rel <= 2 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("grid", [(1080, 4, 5), (1152, 6, 5), (1600, 5, 4), (2187, 4, 4)])
+def test_grids_elongated_along_x(grid):
+    """Lines so long that a workgroup of the x-axis pass holds fewer of them."""
+    from mdpy_amd import _lib as L
+    from mdpy_amd.engine import Engine
+    from mdpy_amd.unit import ONE_OVER_4PI_EPS0
+    from oracle import ewald as EW
+    print("case: PME grid", grid, flush=True)
+    rng = np.random.default_rng(grid[0])
+    n, box = 60, np.array([24.0, 26.5, 21.25])
+    x = rng.uniform(-0.5, 0.5, (n, 3)) * box
+    q = rng.uniform(-1, 1, n)
+    e = Engine.bare(n, box, positions=x)
+    e.set_masses(np.ones(n))
+    e.set_charges(q)
+    e.set_lj(np.tile([0.0, 1.0, 0.0, 1.0], (n, 1)))
+    e.set_exclusions(np.zeros(n + 1, int), [])
+    e.set_scaling(np.zeros(n + 1, int), [])
+    e.configure_nonbonded(9.0, skin=1.0)
+    e.configure_pme(grid, 0.36)
+    F = e.compute(L.TERM_COUL_RECIP)[0].cpu().numpy()
+    assert e.status() == 0
+    e.close()
+    Fr = EW.spme_reciprocal(x, q, box, grid, 4, 0.36, ONE_OVER_4PI_EPS0)[0]
+    # float32 roundings of up to 7 passes each way, on a derivative along x of K_x/L_x points per A
+    assert np.linalg.norm(F - Fr) <= 2.0 ** -24 * 50 * max(1.0, 0.02 * grid[0]) * np.linalg.norm(Fr)
